@@ -1197,10 +1197,9 @@ int hmx_run_tasks(int precision, int type, const void* tasks, int count, int* fl
         need = hmx::rkrk_workspace(x.parts[0].rk.cap, x.parts[1].rk.cap);
       } else if (type == hmx::T_HODLR) {
         need = hmx::hodlr_workspace(x.lda);
-      } else if (type == hmx::T_GEMM) {
-        for (int a = 0; a < (x.m.s + 63) / 64; ++a)
-          for (int b = 0; b < (x.n.s + 63) / 64; ++b) tiles.push_back(hmx::GemmTile{i, a, b});
       }
+      x.type = type;
+      hmx::append_tiles(x, i, tiles);
       x.ws = ws;
       ws += need;
     }

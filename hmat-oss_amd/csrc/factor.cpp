@@ -1270,8 +1270,31 @@ class Exec {
       t.ldc = I.ld;
       wr(I);
       emit(t);
-      solve_lower_left(b, I, dim(b->m()));
+      identity_lower(b, I, 0);
       maybe_flush();
+    }
+  }
+  // X <- L^{-1} X for the rows of an identity block that belong to L: the
+  // inverse is lower triangular, so row block [c0, c0 + m) has entries in its
+  // first c0 + m columns only (half the work of the full block's columns)
+  void identity_lower(const Block* L, const DV& X, int c0) {
+    if (L->is_leaf()) {
+      trsm(1, L, X, dim(c0 + L->m()));
+      return;
+    }
+    int off = 0;
+    std::vector<std::pair<int, int>> subs;
+    for (int i = 0; i < L->nrow; ++i) {
+      const Block* d = L->get(i, i);
+      subs.push_back({off, d->n()});
+      for (int j = 0; j < i; ++j) {
+        const Block* lij = L->get(i, j);
+        if (lij)
+          hgemv(lij, 'N', -1.0, rows_of(X, subs[j].first, subs[j].second),
+                rows_of(X, subs[i].first, subs[i].second), dim(c0 + subs[j].first + subs[j].second));
+      }
+      identity_lower(d, rows_of(X, off, d->n()), c0 + off);
+      off += d->n();
     }
   }
   void use_inverses(bool v) { use_inv_ = v; }
@@ -2380,11 +2403,7 @@ class Exec {
         t.ws = ws;
         ws += need;
         sorted[i] = t;
-        if (ty == T_GEMM) {
-          const int tm = (t.m.s + 63) / 64, tn = (t.n.s + 63) / 64;
-          for (int a = 0; a < tm; ++a)
-            for (int b = 0; b < tn; ++b) tiles.push_back(GemmTile{(int)i - L.first, a, b});
-        }
+        append_tiles(t, (int)i - L.first, tiles);
         ++L.count;
         ++i;
       }

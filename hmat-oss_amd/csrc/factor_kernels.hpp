@@ -5,6 +5,7 @@
 #include <algorithm>
 #include <cstdint>
 #include <stdexcept>
+#include <vector>
 
 #include "dev_common.hpp"
 #include "ftask.hpp"
@@ -20,7 +21,16 @@ int64_t hodlr_workspace(int cap);
 // p[0..n) = v on stream s (a kernel, so it may be captured in a graph).
 void launch_fill_int(int* p, size_t n, int v, hipStream_t s);
 
-// One batched launch of 'count' tasks of 'type' (GEMM: 'ntiles' tiles).
+// The work items of the types that cut a task into tiles, one workgroup each:
+// 64 x 64 tiles of C (GEMM), slabs of independent rows / columns (TRSM), runs
+// of entries (ZERO, AXPY, SUMK).  append_tiles adds those of a task (by its
+// static sizes; a tile past a dynamic size returns at once), task 'index' of
+// its launch.
+bool task_has_tiles(int type);
+void append_tiles(const FTask& t, int index, std::vector<GemmTile>& tiles);
+
+// One batched launch of 'count' tasks of 'type' ('ntiles' tiles where the
+// type has tiles).
 // flags[0] |= 1 on an Rk capacity overflow, flags[1] |= 1 on a non-positive
 // pivot in POTRF.
 template <typename T>

@@ -141,6 +141,11 @@ __global__ void __launch_bounds__(256) k_gemm(const FTask* tasks, const GemmTile
 constexpr int kLdsDense = 128;
 
 constexpr int kNb = 16;  // panel width of the blocked POTRF / TRSM
+constexpr int kTrsmCols = 64;  // independent rows / columns of a TRSM tile: 16 per wavefront
+// entries of a tile of the elementwise tasks (ZERO, AXPY, SUMK): one workgroup
+// per task left a 2,048 x 2,048 identity at 590 us and the sum of 8 slices of
+// 2,048 x 65 at 535 us, with 255 CUs idle
+constexpr int kElemsPerTile = 2048;
 
 // Right-looking blocked Cholesky: each 16-column panel is factorised
 // left-looking (short dots over the panel only), then the trailing lower
@@ -499,7 +504,7 @@ __global__ void __launch_bounds__(kBlock) k_hodlr(const FTask* tasks, double* ws
 }
 
 // ---------------------------------------------------------------------------
-// TRSM with a lower-triangular leaf L (n x n), L staged in LDS:
+// TRSM with a lower-triangular leaf L (n x n):
 //   mode 0: X (m x n) <- X L^{-T}     (solveUpperTriangularRight, LLt)
 //   mode 1: X (n x k) <- L^{-1} X     (solveLowerTriangularLeft)
 //   mode 2: X (n x k) <- L^{-T} X     (solveUpperTriangularLeft, Uplo LOWER)
@@ -507,313 +512,242 @@ __global__ void __launch_bounds__(kBlock) k_hodlr(const FTask* tasks, double* ws
 // triangle U (so 0 is X U^{-1}, 1 is U^{-T} X, 2 is U^{-1} X: the LU cases of
 // scalar_array.cpp:852-874), kTrsmUnit assumes a unit diagonal, kTrsmPiv
 // applies getrf's row interchanges to X first (laswp, scalar_array.cpp:855).
-// Rows (mode 0) / columns (modes 1, 2) of X are independent: one thread runs
-// the substitution of one of them, reading L from LDS (broadcast) and its own
-// row / column from LDS when it fits, so no barrier is needed inside.
+// Rows (mode 0) / columns (modes 1, 2) of X are independent: a task is cut
+// into tiles of kTrsmCols of them, one workgroup each.
 // ---------------------------------------------------------------------------
 constexpr int kShDoubles = 19456;  // 152 KiB of LDS per workgroup
 
-// Substitution with one thread per independent row / column (L or X too
-// large for the blocked-inverse kernel below).
-template <typename T>
-__device__ void trsm_rowwise(const FTask& t, double* sh) {
-  const int n = t.n.s;  // order of L
-  const int other = eff(t.m);
-  if (other <= 0) return;
-  const T* Lg = (const T*)t.A;
-  const int ldl = t.lda;
-  T* X = (T*)t.C;
-  const int ldx = t.ldc;
-  const int mode = t.mode & kTrsmBase;
-  const bool transa = (t.mode & kTrsmTransA) != 0, unit = (t.mode & kTrsmUnit) != 0;
-  const bool lds_l = n * n <= kShDoubles;
-  double* Ls = sh;
-  if (lds_l)
-    for (int e = threadIdx.x; e < n * n; e += kBlock) {
-      const int i = e % n, j = e / n;
-      Ls[e] = transa ? (double)Lg[j + (size_t)i * ldl] : (double)Lg[i + (size_t)j * ldl];
-    }
-  // X block staged in LDS behind L when it fits: rows = n for modes 1/2
-  const int xr = mode == 0 ? other : n, xc = mode == 0 ? n : other;
-  const int xl = xr | 1;  // odd leading dimension: fewer bank conflicts for column walks
-  const bool lds_x = lds_l && n * n + xl * xc <= kShDoubles;
-  double* Xs = sh + n * n;
-  if (lds_x)
-    for (int e = threadIdx.x; e < xr * xc; e += kBlock) {
-      const int i = e % xr, j = e / xr;
-      Xs[i + j * xl] = (double)X[i + (size_t)j * ldx];
-    }
-  __syncthreads();
-  auto Lat = [&](int i, int j) -> double {
-    if (lds_l) return Ls[i + j * n];
-    return transa ? (double)Lg[j + (size_t)i * ldl] : (double)Lg[i + (size_t)j * ldl];
-  };
-  auto Ldiv = [&](double s, int j) -> double { return unit ? s : s / Lat(j, j); };
-  auto Xg = [&](int i, int j) -> double { return lds_x ? Xs[i + j * xl] : (double)X[i + (size_t)j * ldx]; };
-  auto Xp = [&](int i, int j, double v) {
-    if (lds_x)
-      Xs[i + j * xl] = v;
-    else
-      X[i + (size_t)j * ldx] = (T)v;
-  };
-  if ((t.mode & kTrsmPiv) && mode != 0) {
-    // each thread replays the interchanges on its own columns
-    const int* piv = (const int*)t.B;
-    for (int c = threadIdx.x; c < other; c += kBlock)
-      for (int i = 0; i < n; ++i) {
-        int p = piv[i];
-        p = p < 0 ? 0 : (p >= n ? n - 1 : p);
-        if (p != i) {
-          const double a = Xg(i, c), b = Xg(p, c);
-          Xp(i, c, b);
-          Xp(p, c, a);
-        }
-      }
-    __syncthreads();
-  }
-  // Blocked substitution: a 16-wide diagonal block is solved with one thread per
-  // independent row / column, then the rest gets a rank-16 update from all threads.
-  if (mode == 0) {
-    for (int jb = 0; jb < n; jb += kNb) {
-      const int je = jb + kNb < n ? jb + kNb : n;
-      for (int r = threadIdx.x; r < other; r += kBlock)
-        for (int c = jb; c < je; ++c) {
-          double s = Xg(r, c);
-          for (int l = jb; l < c; ++l) s -= Lat(c, l) * Xg(r, l);
-          Xp(r, c, Ldiv(s, c));
-        }
-      __syncthreads();
-      const int nc = n - je;
-      for (int e = threadIdx.x; e < other * nc; e += kBlock) {
-        const int r = e % other, c = je + e / other;
-        double s = Xg(r, c);
-        for (int l = jb; l < je; ++l) s -= Xg(r, l) * Lat(c, l);
-        Xp(r, c, s);
-      }
-      __syncthreads();
-    }
-  } else if (mode == 1) {
-    for (int jb = 0; jb < n; jb += kNb) {
-      const int je = jb + kNb < n ? jb + kNb : n;
-      for (int c = threadIdx.x; c < other; c += kBlock)
-        for (int j = jb; j < je; ++j) {
-          double s = Xg(j, c);
-          for (int l = jb; l < j; ++l) s -= Lat(j, l) * Xg(l, c);
-          Xp(j, c, Ldiv(s, j));
-        }
-      __syncthreads();
-      const int nr = n - je;
-      for (int e = threadIdx.x; e < nr * other; e += kBlock) {
-        const int i = je + e % nr, c = e / nr;
-        double s = Xg(i, c);
-        for (int l = jb; l < je; ++l) s -= Lat(i, l) * Xg(l, c);
-        Xp(i, c, s);
-      }
-      __syncthreads();
-    }
-  } else {
-    for (int je = n; je > 0; je -= kNb) {
-      const int jb = je - kNb > 0 ? je - kNb : 0;
-      for (int c = threadIdx.x; c < other; c += kBlock)
-        for (int j = je - 1; j >= jb; --j) {
-          double s = Xg(j, c);
-          for (int l = j + 1; l < je; ++l) s -= Lat(l, j) * Xg(l, c);
-          Xp(j, c, Ldiv(s, j));
-        }
-      __syncthreads();
-      for (int e = threadIdx.x; e < jb * other; e += kBlock) {
-        const int i = e % jb, c = e / jb;
-        double s = Xg(i, c);
-        for (int l = jb; l < je; ++l) s -= Lat(l, i) * Xg(l, c);
-        Xp(i, c, s);
-      }
-      __syncthreads();
-    }
-  }
-  if (lds_x) {
-    __syncthreads();
-    for (int e = threadIdx.x; e < xr * xc; e += kBlock) {
-      const int i = e % xr, j = e / xr;
-      X[i + (size_t)j * ldx] = (T)Xs[i + j * xl];
-    }
+// A wavefront solves 16 independent rows / columns of X on its own: X^T (mode
+// 0) or X is cut into 16 x 16 blocks that stay in registers in the layout in
+// which v_mfma_f64_16x16x4f64 returns a tile, which is also its B operand's,
+// so a solved block is the operand of the next products without passing
+// through LDS:
+//   X_p <- inv(L_pp) (X_p - sum_{c < p} L_pc X_c)   (p from the last block in mode 2)
+// The blocks of L come from the L2 (one 128-byte run per 16 lanes, shorter
+// runs for transposed operands), eight of them in flight.  Only the inverted
+// diagonal blocks pass through LDS.  Eight blocks (128 rows) are solved at a
+// time: above that the solved blocks are read back by the lanes that wrote
+// them.
+// Bound: the serial chain of nb (nb + 1) / 2 block products; no barrier after
+// the inversions.  The earlier form kept L and X in LDS, two workgroups per
+// task: leaves above 100 rows did not fit beside X and were substituted row by
+// row, and a block of 2,000 columns had two CUs.  The N = 4,000 system (leaves
+// of 125 rows, inverses of its 2,000-row diagonal blocks for the solve) went
+// from 138.9 to 24.4 ms with this, the tiles of the elementwise tasks and the
+// skipped zero half of the inverses.
+constexpr int kTrsmBlocks = 8;              // blocks solved in registers at a time
+constexpr int kTrsmInvLd = kNb * kNb + 8;   // diagonal blocks in LDS: spread over the banks
+
+// f(0), ..., f(N - 1) with compile-time indices (register arrays)
+template <int I, int N, typename F>
+__device__ __forceinline__ void static_for(F f) {
+  if constexpr (I < N) {
+    f(std::integral_constant<int, I>{});
+    static_for<I + 1, N>(f);
   }
 }
 
-constexpr int kTrsmRegs = 8;  // block-step results per thread: 16 x 8 x 256 covers 128 columns
-
-// Blocked TRSM with L (n x n) and X staged in LDS.  The 16 x 16 diagonal
-// blocks of L are inverted first (one thread per column of each block), then
-// every 16-row (16-column for mode 0) step is a small dense product with that
-// inverse followed by a rank-16 update of the rest, each spread over the whole
-// workgroup: the serial chain is 3 barriers per block instead of one thread
-// walking the whole triangle.
-// Two workgroups per task: the columns of X (its rows in mode 0) are
-// independent, so workgroup h of a task solves the h-th half of them.
-constexpr int kTrsmSplit = 2;
+// row p of the s-th pair (p, c), c < p, in row order
+constexpr int trsm_pair_row(int s) {
+  int p = 1;
+  while (p * (p + 1) / 2 <= s) ++p;
+  return p;
+}
 
 template <typename T>
-__global__ void __launch_bounds__(kBlock) k_trsm(const FTask* tasks, const int* fail) {
-  __shared__ double sh[kShDoubles];
+__global__ void __launch_bounds__(kBlock) k_trsm(const FTask* tasks, const GemmTile* tiles, const int* fail) {
+  __shared__ double inv[kTrsmBlocks * kTrsmInvLd];
+  __shared__ double rdiag[kTrsmBlocks * kNb];
+  __shared__ int perm[kTrsmBlocks * kNb];
+  constexpr int NB = kTrsmBlocks;
   if (*fail) return;
-  FTask t = tasks[blockIdx.x / kTrsmSplit];
-  {
-    const int all = eff(t.m), half = blockIdx.x % kTrsmSplit;
-    const int per = (all + kTrsmSplit - 1) / kTrsmSplit;
-    const int lo = half * per, cnt = all - lo < per ? all - lo : per;
-    if (cnt <= 0) return;
-    t.m.s = cnt;
-    t.m.d = nullptr;
-    t.C = (void*)((T*)t.C + ((t.mode & kTrsmBase) == 0 ? (size_t)lo : (size_t)lo * t.ldc));
-  }
-  const int n = t.n.s;
-  const int other = eff(t.m);
-  if (other <= 0) return;
+  const GemmTile tl = tiles[blockIdx.x];
+  const FTask& t = tasks[tl.task];
+  const int other = eff(t.m), col0 = tl.tm * kTrsmCols, n = t.n.s;
+  if (col0 >= other || n <= 0) return;
+  const int nb = (n + kNb - 1) / kNb;
   const int mode = t.mode & kTrsmBase;
   const bool transa = (t.mode & kTrsmTransA) != 0, unit = (t.mode & kTrsmUnit) != 0;
-  const int nb = (n + kNb - 1) / kNb;
-  const int xr = mode == 0 ? other : n, xc = mode == 0 ? n : other;
-  const int xl = xr | 1;
-  // every block step keeps at most kTrsmRegs results per thread in registers
-  const int64_t need = (int64_t)n * n + (int64_t)nb * kNb * kNb + (int64_t)xl * xc;
-  if (need > kShDoubles || other > kNb * kTrsmRegs) {
-    trsm_rowwise<T>(t, sh);
-    return;
-  }
-  double* Ls = sh;                          // n x n, ld n (L, or U^T with transa)
-  double* Inv = Ls + (size_t)n * n;         // nb blocks of 16 x 16 (ld 16)
-  double* Xs = Inv + (size_t)nb * kNb * kNb;  // xr x xc, ld xl
+  const bool back = mode == 2, pivot = (t.mode & kTrsmPiv) && mode != 0;
   const T* Lg = (const T*)t.A;
-  const int ldl = t.lda;
   T* X = (T*)t.C;
-  const int ldx = t.ldc;
-  if (transa)
-    stage_in(Ls, n, Lg, (long)ldl, 1L, n, n);
-  else
-    stage_in(Ls, n, Lg, 1L, (long)ldl, n, n);
-  __syncthreads();
-  stage_in(Xs, xl, X, 1L, (long)ldx, xr, xc);
-  __syncthreads();
-  if ((t.mode & kTrsmPiv) && mode != 0) {
+  const long li = transa ? (long)t.lda : 1L, lk = transa ? 1L : (long)t.lda;  // strides of L(i, k)
+  const long ai = back ? lk : li, ak = back ? li : lk;  // of the operand: L, or L^T in mode 2
+  const int lane = threadIdx.x & (kWave - 1), w = threadIdx.x / kWave;
+  const int ii = lane & 15, kk = lane >> 4;
+  // this wavefront's 16 columns of X (rows in mode 0): element (row r, column
+  // ii) at Xc[r * xr]
+  const int j = col0 + kNb * w + ii, jc = j < other ? j : other - 1;
+  const bool mine = col0 + kNb * w < other;
+  const long xr = mode == 0 ? (long)t.ldc : 1L;
+  T* Xc = X + (mode == 0 ? (size_t)jc : (size_t)jc * t.ldc);
+  const bool permuted = pivot && nb <= NB;
+  if (permuted && w == 0) {
+    // the interchanges as one permutation, rows lane + 64 q in registers
     const int* piv = (const int*)t.B;
-    for (int c = threadIdx.x; c < other; c += kBlock)
+    constexpr int kQ = NB / 4;
+    int pr[kQ], pv[kQ];
+#pragma unroll
+    for (int q = 0; q < kQ; ++q) {
+      const int r = lane + kWave * q;
+      pr[q] = r;
+      const int p = piv[r < n ? r : n - 1];
+      pv[q] = p < 0 ? 0 : (p >= n ? n - 1 : p);
+    }
+    auto at = [](const int (&v)[kQ], int i) __attribute__((always_inline)) {
+      int x = 0;
+#pragma unroll
+      for (int q = 0; q < kQ; ++q) {
+        const int y = __builtin_amdgcn_readlane(v[q], i & (kWave - 1));
+        x = (i >> 6) == q ? y : x;
+      }
+      return x;
+    };
+    for (int i = 0; i < n; ++i) {
+      const int p = at(pv, i);
+      const int a = at(pr, i), b = at(pr, p);
+#pragma unroll
+      for (int q = 0; q < kQ; ++q) {
+        const int r = lane + kWave * q;
+        pr[q] = r == i ? b : (r == p ? a : pr[q]);
+      }
+    }
+#pragma unroll
+    for (int q = 0; q < kQ; ++q) perm[lane + kWave * q] = pr[q];
+  } else if (pivot && !permuted) {
+    // wide leaves: each thread replays the interchanges on its own column
+    const int* piv = (const int*)t.B;
+    if (threadIdx.x < kTrsmCols && col0 + (int)threadIdx.x < other) {
+      T* xc = X + (size_t)(col0 + threadIdx.x) * t.ldc;
       for (int i = 0; i < n; ++i) {
         int p = piv[i];
         p = p < 0 ? 0 : (p >= n ? n - 1 : p);
         if (p != i) {
-          const double a = Xs[i + c * xl];
-          Xs[i + c * xl] = Xs[p + c * xl];
-          Xs[p + c * xl] = a;
+          const T a = xc[i];
+          xc[i] = xc[p];
+          xc[p] = a;
         }
       }
-  }
-  // inverses of the diagonal blocks: thread (b, c) forms column c of block b
-  // by forward substitution, the column held in registers (rows beyond the
-  // block read a clamped entry and are discarded)
-  for (int w = threadIdx.x; w < nb * kNb; w += kBlock) {
-    const int b = w / kNb, c = w % kNb, r0 = b * kNb;
-    const int bs = n - r0 < kNb ? n - r0 : kNb;
-    double* inv = Inv + (size_t)b * kNb * kNb;
-    if (c >= bs) continue;
-    double x[kNb];
-#pragma unroll
-    for (int r = 0; r < kNb; ++r) {
-      const int rr = r < bs ? r : bs - 1;
-      const double* lrow = Ls + (r0 + rr);
-      double s = r == c ? 1.0 : 0.0;
-#pragma unroll
-      for (int l = 0; l < r; ++l) {
-        // x[l] == 0 for l < c; columns past the matrix only feed discarded rows
-        const int cl = r0 + l < n ? r0 + l : n - 1;
-        s -= lrow[(size_t)cl * n] * x[l];
-      }
-      const double d = unit ? 1.0 : lrow[(size_t)(r0 + rr) * n];
-      x[r] = r < c ? 0.0 : s / d;
     }
-#pragma unroll
-    for (int r = 0; r < kNb; ++r)
-      if (r < bs) inv[r + c * kNb] = x[r];
   }
-  __syncthreads();
-  // Every block step is two small products on the matrix cores (16 x 16
-  // tiles, inner dimension the block's bs <= 16 columns of L): the block of
-  // X times the inverted diagonal block, held in registers across a barrier,
-  // then the rank-bs update of the remaining rows (columns in mode 0).
-  const int lane = threadIdx.x & (kWave - 1), w = threadIdx.x / kWave;
-  const int ot = (other + 15) / 16;  // 16-wide tiles along 'other' (<= 8)
-  for (int step = 0; step < nb; ++step) {
-    const int b = mode == 2 ? nb - 1 - step : step;
-    const int r0 = b * kNb, bs = n - r0 < kNb ? n - r0 : kNb;
-    const double* inv = Inv + (size_t)b * kNb * kNb;
-    hmx_double4 hold[2];
-#pragma unroll
-    for (int q = 0; q < 2; ++q) {
-      const int tt = w + kWaves * q;
-      if (tt >= ot) continue;
-      const int o0 = 16 * tt;
-      if (mode == 1)  // X_b <- inv X_b
-        hold[q] = mfma_tile16(
-            [&](int ii, int k) { const double v = inv[(ii < bs ? ii : bs - 1) + k * kNb]; return ii < bs ? v : 0.0; },
-            [&](int k, int jj) { const int c = o0 + jj < other ? o0 + jj : other - 1; const double v = Xs[(r0 + k) + c * xl]; return o0 + jj < other ? v : 0.0; }, bs);
-      else if (mode == 2)  // X_b <- inv^T X_b
-        hold[q] = mfma_tile16(
-            [&](int ii, int k) { const double v = inv[k + (ii < bs ? ii : bs - 1) * kNb]; return ii < bs ? v : 0.0; },
-            [&](int k, int jj) { const int c = o0 + jj < other ? o0 + jj : other - 1; const double v = Xs[(r0 + k) + c * xl]; return o0 + jj < other ? v : 0.0; }, bs);
-      else  // X_b <- X_b inv^T (rows of X along 'other')
-        hold[q] = mfma_tile16(
-            [&](int ii, int k) { const int r = o0 + ii < other ? o0 + ii : other - 1; const double v = Xs[r + (r0 + k) * xl]; return o0 + ii < other ? v : 0.0; },
-            [&](int k, int jj) { const double v = inv[(jj < bs ? jj : bs - 1) + k * kNb]; return jj < bs ? v : 0.0; }, bs);
+  for (int p0 = 0; p0 < nb; p0 += NB) {
+    const int np = nb - p0 < NB ? nb - p0 : NB;
+    auto block_of = [&](int p) { return back ? nb - 1 - p : p; };
+    __syncthreads();
+    // the diagonal blocks (lower triangles) and the reciprocals of the diagonal
+    for (int e = threadIdx.x; e < np * kNb * kNb; e += kBlock) {
+      const int q = e / (kNb * kNb), r = e % kNb, l = e / kNb % kNb;
+      const int gr = block_of(p0 + q) * kNb + r, gl = gr - r + l;
+      const bool in = gr < n && l <= r;
+      const double v = (double)Lg[(gr < n ? gr : n - 1) * li + (gl < n ? gl : n - 1) * lk];
+      inv[q * kTrsmInvLd + r + l * kNb] = in ? v : 0.0;
+      if (r == l) rdiag[q * kNb + r] = (unit || !in) ? 1.0 : 1.0 / v;
     }
     __syncthreads();
+    // thread (q, c): column c of the inverse of block q by forward
+    // substitution, in registers; written over the block once all are done
+    const int iq = threadIdx.x / kNb, ic = threadIdx.x % kNb;
+    double xi[kNb];
+    if (iq < np) {
+      const double* blk = inv + iq * kTrsmInvLd;
 #pragma unroll
-    for (int q = 0; q < 2; ++q) {
-      const int tt = w + kWaves * q;
-      if (tt >= ot) continue;
-      const int o0 = 16 * tt, jj = lane & 15;
+      for (int r = 0; r < kNb; ++r) {
+        double s = r == ic ? 1.0 : 0.0;
+#pragma unroll
+        for (int l = 0; l < r; ++l) s -= blk[r + l * kNb] * xi[l];
+        xi[r] = r < ic ? 0.0 : s * rdiag[iq * kNb + r];
+      }
+    }
+    __syncthreads();
+    if (iq < np) {
+      double* blk = inv + iq * kTrsmInvLd;
+      const int g0 = block_of(p0 + iq) * kNb;
+#pragma unroll
+      for (int r = 0; r < kNb; ++r) {
+        const double v = (g0 + ic >= n || g0 + r >= n) ? 0.0 : xi[r];
+        blk[back ? ic + r * kNb : r + ic * kNb] = v;  // mode 2 applies the transposed inverse
+      }
+    }
+    __syncthreads();
+    if (!mine) continue;
+    hmx_double4 x[NB];
+#pragma unroll
+    for (int p = 0; p < NB; ++p) {
+      if (p >= np) continue;
+      const int r0 = kNb * block_of(p0 + p);
 #pragma unroll
       for (int v = 0; v < 4; ++v) {
-        const int ii = (lane >> 4) + 4 * v;
-        if (mode == 0) {
-          if (o0 + ii < other && jj < bs) Xs[(o0 + ii) + (r0 + jj) * xl] = hold[q][v];
-        } else {
-          if (ii < bs && o0 + jj < other) Xs[(r0 + ii) + (o0 + jj) * xl] = hold[q][v];
-        }
+        const int r = r0 + kk + 4 * v, rc = r < n ? r : n - 1;
+        const double y = (double)Xc[(permuted ? perm[rc] : rc) * xr];
+        x[p][v] = r < n ? y : 0.0;
       }
     }
-    __syncthreads();
-    // the rest: rows [r0 + bs, n) (mode 1), [0, r0) (mode 2), columns [r0 + bs, n) (mode 0)
-    const int lo = mode == 2 ? 0 : r0 + bs, rest = mode == 2 ? r0 : n - r0 - bs;
-    const int rt = (rest + 15) / 16;
-    for (int tt = w; tt < rt * ot; tt += kWaves) {
-      const int x0 = lo + 16 * (tt % rt), o0 = 16 * (tt / rt);
-      hmx_double4 acc;
-      if (mode == 1)  // X_rest -= L(rest, b) X_b
-        acc = mfma_tile16(
-            [&](int ii, int k) { const int r = x0 + ii < lo + rest ? x0 + ii : lo + rest - 1; const double v = Ls[r + (size_t)(r0 + k) * n]; return x0 + ii < lo + rest ? v : 0.0; },
-            [&](int k, int jj) { const int c = o0 + jj < other ? o0 + jj : other - 1; const double v = Xs[(r0 + k) + c * xl]; return o0 + jj < other ? v : 0.0; }, bs);
-      else if (mode == 2)  // X_rest -= L(b, rest)^T X_b
-        acc = mfma_tile16(
-            [&](int ii, int k) { const int r = x0 + ii < lo + rest ? x0 + ii : lo + rest - 1; const double v = Ls[(r0 + k) + (size_t)r * n]; return x0 + ii < lo + rest ? v : 0.0; },
-            [&](int k, int jj) { const int c = o0 + jj < other ? o0 + jj : other - 1; const double v = Xs[(r0 + k) + c * xl]; return o0 + jj < other ? v : 0.0; }, bs);
-      else  // X(:, rest) -= X_b L(rest, b)^T, rows of X along 'other'
-        acc = mfma_tile16(
-            [&](int ii, int k) { const int r = o0 + ii < other ? o0 + ii : other - 1; const double v = Xs[r + (r0 + k) * xl]; return o0 + ii < other ? v : 0.0; },
-            [&](int k, int jj) { const int c = x0 + jj < lo + rest ? x0 + jj : lo + rest - 1; const double v = Ls[c + (size_t)(r0 + k) * n]; return x0 + jj < lo + rest ? v : 0.0; }, bs);
-      const int jj = lane & 15;
+    // the blocks solved before these eight
+    for (int c = 0; c < p0; ++c) {
+      const int c0 = kNb * block_of(c) + kk;
+      double xs[4], as[NB][4];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int k = c0 + 4 * q, kc = k < n ? k : n - 1;
+        const double y = (double)Xc[kc * xr];
+        xs[q] = k < n ? -y : 0.0;
+#pragma unroll
+        for (int p = 0; p < NB; ++p) {
+          const int r = kNb * block_of(p0 + (p < np ? p : np - 1)) + ii, rc = r < n ? r : n - 1;
+          const double v = (double)Lg[rc * ai + kc * ak];
+          as[p][q] = (r < n && k < n) ? v : 0.0;
+        }
+      }
+#pragma unroll
+      for (int p = 0; p < NB; ++p)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) x[p] = __builtin_amdgcn_mfma_f64_16x16x4f64(as[p][q], xs[q], x[p], 0, 0, 0);
+    }
+    // operand blocks in the order in which they are used, (1, 0), (2, 0),
+    // (2, 1), ...: kAhead of them in flight
+    constexpr int kAhead = 8, kPairs = NB * (NB - 1) / 2;
+    double a[kAhead][4];
+    auto load_block = [&](auto S) __attribute__((always_inline)) {
+      constexpr int s = decltype(S)::value, p = trsm_pair_row(s), c = s - p * (p - 1) / 2;
+      if (p >= np) return;
+      const int r = kNb * block_of(p0 + p) + ii, rc = r < n ? r : n - 1;
+      const int k0 = kNb * block_of(p0 + c) + kk;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int k = k0 + 4 * q, kc = k < n ? k : n - 1;
+        const double v = (double)Lg[rc * ai + kc * ak];
+        a[s % kAhead][q] = (r < n && k < n) ? v : 0.0;
+      }
+    };
+    static_for<0, kAhead < kPairs ? kAhead : kPairs>(load_block);
+    static_for<0, NB>([&](auto P) __attribute__((always_inline)) {
+      constexpr int p = decltype(P)::value;
+      if (p >= np) return;
+      hmx_double4 s0 = x[p], s1 = {0.0, 0.0, 0.0, 0.0};
+      // x of the solved blocks holds the negated result
+      static_for<0, p>([&](auto C) __attribute__((always_inline)) {
+        constexpr int c = decltype(C)::value, s = p * (p - 1) / 2 + c;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          if constexpr (c & 1)
+            s1 = __builtin_amdgcn_mfma_f64_16x16x4f64(a[s % kAhead][q], x[c][q], s1, 0, 0, 0);
+          else
+            s0 = __builtin_amdgcn_mfma_f64_16x16x4f64(a[s % kAhead][q], x[c][q], s0, 0, 0, 0);
+        }
+        if constexpr (s + kAhead < kPairs) load_block(std::integral_constant<int, s + kAhead>{});
+      });
+      const double* blk = inv + p * kTrsmInvLd;
+      hmx_double4 y = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        y = __builtin_amdgcn_mfma_f64_16x16x4f64(blk[q * kWave + lane], s0[q] + s1[q], y, 0, 0, 0);
+      const int r0 = kNb * block_of(p0 + p) + kk;
 #pragma unroll
       for (int v = 0; v < 4; ++v) {
-        const int ii = (lane >> 4) + 4 * v;
-        if (mode == 0) {
-          if (o0 + ii < other && x0 + jj < lo + rest) Xs[(o0 + ii) + (x0 + jj) * xl] -= acc[v];
-        } else {
-          if (x0 + ii < lo + rest && o0 + jj < other) Xs[(x0 + ii) + (o0 + jj) * xl] -= acc[v];
-        }
+        if (r0 + 4 * v < n && j < other) Xc[(r0 + 4 * v) * xr] = (T)y[v];
+        x[p][v] = -y[v];
       }
-    }
-    __syncthreads();
-  }
-  for (int e = threadIdx.x; e < xr * xc; e += kBlock) {
-    const int i = e % xr, j = e / xr;
-    X[i + (size_t)j * ldx] = (T)Xs[i + j * xl];
+    });
   }
 }
 
@@ -822,17 +756,21 @@ __global__ void __launch_bounds__(kBlock) k_trsm(const FTask* tasks, const int* 
 // GEMM split along its inner dimension, added in a fixed order.
 // ---------------------------------------------------------------------------
 template <typename T>
-__global__ void k_sumk(const FTask* tasks, const int* fail) {
+__global__ void k_sumk(const FTask* tasks, const GemmTile* tiles, const int* fail) {
   if (*fail) return;
-  const FTask& t = tasks[blockIdx.x];
+  const GemmTile tl = tiles[blockIdx.x];
+  const FTask& t = tasks[tl.task];
   const int M = eff(t.m), N = eff(t.n), S = t.p.s;
   const T* W = (const T*)t.A;
   T* C = (T*)t.C;
-  for (int e = threadIdx.x; e < M * N; e += blockDim.x) {
-    const int i = e % M, j = e / M;
+  const int64_t hi = std::min<int64_t>((int64_t)M * N, (int64_t)(tl.tm + 1) * kElemsPerTile);
+  for (int64_t e = (int64_t)tl.tm * kElemsPerTile + threadIdx.x; e < hi; e += blockDim.x) {
+    const int i = (int)(e % M), j = (int)(e / M);
     T* pc = C + i + (size_t)j * t.ldc;
+    const T* w = W + i + (size_t)j * t.lda;
     double s = t.mode ? (double)*pc : 0.0;
-    for (int q = 0; q < S; ++q) s += (double)W[i + (size_t)j * t.lda + (size_t)q * t.ldb];
+#pragma unroll 8
+    for (int q = 0; q < S; ++q) s += (double)w[(size_t)q * t.ldb];
     *pc = (T)s;
   }
 }
@@ -841,26 +779,32 @@ __global__ void k_sumk(const FTask* tasks, const int* fail) {
 // zero fill and axpy
 // ---------------------------------------------------------------------------
 template <typename T>
-__global__ void k_zero(const FTask* tasks, const int* fail) {
+__global__ void k_zero(const FTask* tasks, const GemmTile* tiles, const int* fail) {
   if (*fail) return;
-  const FTask& t = tasks[blockIdx.x];
+  const GemmTile tl = tiles[blockIdx.x];
+  const FTask& t = tasks[tl.task];
   T* C = (T*)t.C;
   const int m = t.m.s, n = t.n.s;
   // mode 1: the identity
-  for (int e = threadIdx.x; e < m * n; e += blockDim.x)
-    C[e % m + (size_t)(e / m) * t.ldc] = (t.mode == 1 && e % m == e / m) ? (T)1 : (T)0;
+  const int64_t hi = std::min<int64_t>((int64_t)m * n, (int64_t)(tl.tm + 1) * kElemsPerTile);
+  for (int64_t e = (int64_t)tl.tm * kElemsPerTile + threadIdx.x; e < hi; e += blockDim.x) {
+    const int i = (int)(e % m), j = (int)(e / m);
+    C[i + (size_t)j * t.ldc] = (t.mode == 1 && i == j) ? (T)1 : (T)0;
+  }
 }
 
 template <typename T>
-__global__ void k_axpy(const FTask* tasks, const int* fail) {
+__global__ void k_axpy(const FTask* tasks, const GemmTile* tiles, const int* fail) {
   if (*fail) return;
-  const FTask& t = tasks[blockIdx.x];
+  const GemmTile tl = tiles[blockIdx.x];
+  const FTask& t = tasks[tl.task];
   T* C = (T*)t.C;
   const T* A = (const T*)t.A;
   const int m = eff(t.m), n = eff(t.n);
   const T al = (T)t.alpha;
-  for (int e = threadIdx.x; e < m * n; e += blockDim.x) {
-    const int i = e % m, j = e / m;
+  const int64_t hi = std::min<int64_t>((int64_t)m * n, (int64_t)(tl.tm + 1) * kElemsPerTile);
+  for (int64_t e = (int64_t)tl.tm * kElemsPerTile + threadIdx.x; e < hi; e += blockDim.x) {
+    const int i = (int)(e % m), j = (int)(e / m);
     const T v = t.ta ? A[j + (size_t)i * t.lda] : A[i + (size_t)j * t.lda];
     if (t.mode)
       C[i + (size_t)j * t.ldc] = al * v;
@@ -1724,6 +1668,30 @@ __global__ void __launch_bounds__(kBlock) k_acafull(const FTask* tasks, const in
 
 }  // namespace
 
+bool task_has_tiles(int type) {
+  return type == T_GEMM || type == T_TRSM || type == T_ZERO || type == T_AXPY || type == T_SUMK;
+}
+void append_tiles(const FTask& t, int index, std::vector<GemmTile>& tiles) {
+  switch (t.type) {
+    case T_GEMM:
+      for (int a = 0; a < (t.m.s + TM - 1) / TM; ++a)
+        for (int b = 0; b < (t.n.s + TN - 1) / TN; ++b) tiles.push_back(GemmTile{index, a, b});
+      break;
+    case T_TRSM:
+      for (int a = 0; a < (t.m.s + kTrsmCols - 1) / kTrsmCols; ++a) tiles.push_back(GemmTile{index, a, 0});
+      break;
+    case T_ZERO:
+    case T_AXPY:
+    case T_SUMK: {
+      const int64_t e = (int64_t)t.m.s * t.n.s;
+      for (int64_t a = 0; a * kElemsPerTile < e; ++a) tiles.push_back(GemmTile{index, (int)a, 0});
+      break;
+    }
+    default:
+      break;
+  }
+}
+
 int64_t fadd_workspace(int m, int n, int K) {
   // dense path only when K >= min(m, n); QR path otherwise (K actual < min)
   const int mn = m < n ? m : n;
@@ -1760,7 +1728,7 @@ void launch_fill_int(int* p, size_t n, int v, hipStream_t s) {
 template <typename T>
 void launch_task_kernel(int type, const FTask* tasks, int count, const GemmTile* tiles,
                         int ntiles, double* ws, int* flags, hipStream_t s) {
-  if (count == 0) return;
+  if (count == 0 || (task_has_tiles(type) && ntiles == 0)) return;
   switch (type) {
     case T_GEMM:
       hipLaunchKernelGGL(k_gemm<T>, dim3(ntiles), dim3(256), 0, s, tasks, tiles, flags + 1);
@@ -1769,7 +1737,7 @@ void launch_task_kernel(int type, const FTask* tasks, int count, const GemmTile*
       hipLaunchKernelGGL(k_potrf<T>, dim3(count), dim3(kBlock), 0, s, tasks, flags + 1);
       break;
     case T_TRSM:
-      hipLaunchKernelGGL(k_trsm<T>, dim3(count * kTrsmSplit), dim3(kBlock), 0, s, tasks, flags + 1);
+      hipLaunchKernelGGL(k_trsm<T>, dim3(ntiles), dim3(kBlock), 0, s, tasks, tiles, flags + 1);
       break;
     case T_FADD:
       hipLaunchKernelGGL(k_fadd<T>, dim3(count), dim3(kBlock), 0, s, tasks, ws, flags);
@@ -1784,16 +1752,16 @@ void launch_task_kernel(int type, const FTask* tasks, int count, const GemmTile*
       hipLaunchKernelGGL(k_acafull<T>, dim3(count), dim3(kBlock), 0, s, tasks, flags + 1);
       break;
     case T_ZERO:
-      hipLaunchKernelGGL(k_zero<T>, dim3(count), dim3(256), 0, s, tasks, flags + 1);
+      hipLaunchKernelGGL(k_zero<T>, dim3(ntiles), dim3(256), 0, s, tasks, tiles, flags + 1);
       break;
     case T_AXPY:
-      hipLaunchKernelGGL(k_axpy<T>, dim3(count), dim3(256), 0, s, tasks, flags + 1);
+      hipLaunchKernelGGL(k_axpy<T>, dim3(ntiles), dim3(256), 0, s, tasks, tiles, flags + 1);
       break;
     case T_GETRF:
       hipLaunchKernelGGL(k_getrf<T>, dim3(count), dim3(kBlock), 0, s, tasks, flags + 1);
       break;
     case T_SUMK:
-      hipLaunchKernelGGL(k_sumk<T>, dim3(count), dim3(256), 0, s, tasks, flags + 1);
+      hipLaunchKernelGGL(k_sumk<T>, dim3(ntiles), dim3(256), 0, s, tasks, tiles, flags + 1);
       break;
     case T_LDLT:
       hipLaunchKernelGGL(k_ldlt<T>, dim3(count), dim3(kBlock), 0, s, tasks, flags + 1);

@@ -224,8 +224,11 @@ void SweepSolver::ensure_inverse(const Store<T>& st, hipStream_t s) {
     tasks[q] = t;
   }
   put(trsm_tasks_, tasks, s);
-  launch_task_kernel<T>(T_TRSM, trsm_tasks_.as<FTask>(), nrows_, nullptr, 0, nullptr,
-                        flags_.as<int>(), s);
+  std::vector<GemmTile> tiles;
+  for (int q = 0; q < nrows_; ++q) append_tiles(tasks[q], q, tiles);
+  put(trsm_tiles_, tiles, s);
+  launch_task_kernel<T>(T_TRSM, trsm_tasks_.as<FTask>(), nrows_, trsm_tiles_.as<GemmTile>(),
+                        (int)tiles.size(), nullptr, flags_.as<int>(), s);
   inv_ready_[p] = true;
 }
 

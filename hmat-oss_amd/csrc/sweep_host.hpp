@@ -43,7 +43,7 @@ class SweepSolver {
   int64_t z_elems_ = 0, zpart_elems_ = 0, inv_elems_ = 0;
   DevBuf z_, zpart_, sync_, fail_, flags_;
   DevBuf inv64_, inv32_;
-  DevBuf trsm_tasks_;
+  DevBuf trsm_tasks_, trsm_tiles_;
   bool inv_ready_[2] = {false, false};
   template <typename T>
   void ensure_inverse(const Store<T>& st, hipStream_t s);
