@@ -577,11 +577,12 @@ __device__ inline double group_sum_c(double v) {
 // (r < R) of G (and of V when kV); the loads use clamped rows and a select,
 // the columns are read once per round and written back after the rotation.
 // Requires rows (and cols when kV) <= R kG, kG == group_lanes(pairs, kLanes)
-// and tracked norms.  Without V (kV false) the caller recovers the right
+// and tracked norms; floor_rel as 1e-30 in team_jacobi.  Without V (kV false) the caller recovers the right
 // singular vectors from the input, as G_in^T U.
 template <int kLanes, int R, int kG, bool kV>
 __device__ inline int team_jacobi_rows(double* G, int ldg, int rows, int cols, double* V, int ldv,
-                                       double* sh2, double* nrm, int max_sweeps, double tol2 = 1e-26) {
+                                       double* sh2, double* nrm, int max_sweeps, double tol2 = 1e-26,
+                                       double floor_rel = 1e-30) {
   const int tid = team_tid<kLanes>();
   if constexpr (kV) {
     for (int e = tid; e < cols * cols; e += kLanes) {
@@ -619,7 +620,7 @@ __device__ inline int team_jacobi_rows(double* G, int ldg, int rows, int cols, d
     team_sync<kLanes>();
     double f = 0.0;
     for (int c = 0; c < cols; ++c) f += nrm[c];
-    const double floor2 = 1e-30 * f;
+    const double floor2 = floor_rel * f;
     int rotated = 0;
     for (int rd = 0; rd < rounds; ++rd) {
       for (int pk = grp; pk < half; pk += ngrp) {

@@ -45,18 +45,121 @@ __global__ void __launch_bounds__(kBlock) k_table_full(const LeafDesc* desc, con
 
 constexpr int kSvdMax = 99;  // compressionMinLeafSize - 1
 
+// Largest of v over the wavefront, in every lane.
+__device__ inline double wave_max(double v) {
+  v = fmax(v, dpp_swap<0xB1>(v));
+  v = fmax(v, dpp_swap<0x4E>(v));
+  v = fmax(v, dpp_swap<0x141>(v));
+  v = fmax(v, dpp_swap<0x140>(v));
+  return fmax(fmax(lane_read(v, 0), lane_read(v, 16)), fmax(lane_read(v, 32), lane_read(v, 48)));
+}
+
+// Pivoted Gram-Schmidt of G (gr x gc, gc <= gr <= 2 kR, at W with ld gr) in
+// registers: threads 2 c and 2 c + 1 hold the two halves of column c.  Step
+// s takes the largest remaining column as the direction q, and row s of R,
+// r_c = q . g_c for every c (columns in their own order, not the pivots'),
+// goes to W[c + s ldw] (over G).  Stops where the largest remaining column is at most
+// tol ||G||_F.  Returns the number of steps; G = Q W^T to working precision,
+// and the singular values and right vectors of G are those of W^T (the R of
+// modified Gram-Schmidt is that of a matrix within rounding of G).
+template <int kR>
+__device__ int pivoted_rows(int gr, int gc, double tol, double* W, int ldw) {
+  __shared__ double q[2 * kR];
+  __shared__ double top[2][kWaves];
+  __shared__ int who[2][kWaves];
+  const int tid = threadIdx.x, lane = tid & (kWave - 1), w = tid / kWave;
+  const int c = tid >> 1, h = tid & 1, i0 = h * kR;
+  double g[kR];
+  double n2 = 0.0;
+#pragma unroll
+  for (int r = 0; r < kR; ++r) {
+    const int i = i0 + r < gr ? i0 + r : gr - 1;
+    const double v = W[i + (c < gc ? c : gc - 1) * gr];
+    g[r] = (c < gc && i0 + r < gr) ? v : 0.0;
+    n2 += g[r] * g[r];
+  }
+  __syncthreads();
+  n2 += dpp_swap<0xB1>(n2);
+  double stop = 0.0;
+  int s = 0;
+  for (; s < gc; ++s) {
+    const int b = s & 1;
+    const double m = wave_max(n2);
+    const uint64_t at = __ballot(n2 == m);
+    if (lane == 0) {
+      top[b][w] = m;
+      who[b][w] = at ? c + ((int)__builtin_ctzll(at) >> 1) : -1;
+    }
+    if (s == 0) {
+      // every column counts twice (both halves hold its norm)
+      const double f = wave_sum(n2);
+      if (lane == 0) q[w] = f;
+    }
+    __syncthreads();
+    double best = top[b][0];
+    int piv = who[b][0];
+#pragma unroll
+    for (int u = 1; u < kWaves; ++u)
+      if (top[b][u] > best) {
+        best = top[b][u];
+        piv = who[b][u];
+      }
+    if (s == 0) {
+      stop = tol * tol * 0.5 * ((q[0] + q[1]) + (q[2] + q[3]));
+      __syncthreads();
+    }
+    if (!(best > stop) || piv < 0) break;
+    if (c == piv) {
+      const double inv = 1.0 / sqrt(best);
+#pragma unroll
+      for (int r = 0; r < kR; ++r) q[i0 + r] = g[r] * inv;
+    }
+    __syncthreads();
+    double d0 = 0.0, d1 = 0.0;
+#pragma unroll
+    for (int r = 0; r < kR; ++r) {
+      if (r & 1)
+        d1 += q[i0 + r] * g[r];
+      else
+        d0 += q[i0 + r] * g[r];
+    }
+    double d = d0 + d1;
+    d += dpp_swap<0xB1>(d);
+    if (h == 0 && c < gc) W[c + s * ldw] = d;
+    n2 = 0.0;
+#pragma unroll
+    for (int r = 0; r < kR; ++r) {
+      g[r] -= d * q[i0 + r];
+      n2 += g[r] * g[r];
+    }
+    n2 += dpp_swap<0xB1>(n2);
+    if (c == piv) n2 = 0.0;  // what is left of the pivot is rounding
+  }
+  __syncthreads();
+  return s;
+}
+
+// Truncated SVD of a small admissible leaf (compression.cpp:224-251).  The
+// block's numerical rank is well below its size, so it is first reduced to W
+// (pivoted_rows, cut at 1e-14 of its norm), and the one-sided Jacobi runs on
+// W's columns, already graded from the largest to the smallest, without
+// accumulating rotations: its columns become sigma_j v_j, and u_j = G v_j /
+// sigma_j from the block's entries evaluated once more (A B^T is then G's exact
+// projection on the kept v_j).  Bound: the serial steps of the reduction and
+// of the Jacobi rounds.  2,407 blocks of 98 x 98 (N = 50,000): 2.3 ms; 107 ms
+// with the Jacobi on the whole blocks and its rotations accumulated.
 template <typename T>
-__global__ void __launch_bounds__(kBlock) k_svd_compress(const LeafDesc* desc, const int* list,
+__global__ void __launch_bounds__(kBlock, 2) k_svd_compress(const LeafDesc* desc, const int* list,
                                                          T* arena, int* ranks, int* overflow,
                                                          PointSet rp, PointSet cp,
                                                          KernelParams kp, double eps,
                                                          const int64_t* tab_off,
                                                          const double* table) {
-  __shared__ double G[kSvdMax * kSvdMax];
-  __shared__ double V[kSvdMax * kSvdMax];
+  // 80 KB of LDS: two workgroups per CU (sig also holds the Jacobi's norms)
+  __shared__ double W[kSvdMax * kSvdMax];
   __shared__ double sig[kSvdMax];
   __shared__ int order[kSvdMax];
-  __shared__ int flag;
+  __shared__ double sh2[2 + kWaves];
   const int leaf = list[blockIdx.x];
   const LeafDesc d = desc[leaf];
   // G = A (m >= n) or A^T (m < n), so that G has min(m, n) columns.
@@ -64,42 +167,62 @@ __global__ void __launch_bounds__(kBlock) k_svd_compress(const LeafDesc* desc, c
   const int gr = tr ? d.n : d.m, gc = tr ? d.m : d.n;
   // entries from the kernel, or from a block staged by the host (tab_off)
   const double* tab = tab_off ? table + tab_off[blockIdx.x] : nullptr;
-  for (int e = threadIdx.x; e < d.m * d.n; e += kBlock) {
-    const int i = e % d.m, j = e / d.m;
-    const double v = tab ? tab[e] : entry(rp, cp, kp, d.r0 + i, d.c0 + j);
-    if (tr)
-      G[j + i * gr] = v;
-    else
-      G[i + j * gr] = v;
-  }
+  auto get = [&](int r, int c) -> double {
+    const int i = tr ? c : r, j = tr ? r : c;
+    return tab ? tab[i + (size_t)j * d.m] : entry(rp, cp, kp, d.r0 + i, d.c0 + j);
+  };
+  const int ldw = gc | 1;  // odd: the rounds' strided accesses spread over the banks
+  const double tol = fmin(1e-14, 1e-2 * eps);
+  for (int e = threadIdx.x; e < gr * gc; e += kBlock) W[e] = get(e % gr, e / gr);
   __syncthreads();
-  jacobi_svd(G, gr, gr, gc, V, gc, &flag);
-  sorted_norms(G, gr, gr, gc, sig, order);
-  int k = find_k(sig, order, gc, eps);
+  const int r = gr <= 52 ? pivoted_rows<26>(gr, gc, tol, W, ldw) : pivoted_rows<50>(gr, gc, tol, W, ldw);
+  // pairs whose inner product is below 1e-16 eps^2 ||G||^2 turn a kept column by
+  // less than 1e-16
+  const double floor_rel = fmax(1e-30, 1e-16 * eps * eps);
+  if (r <= 32)
+    team_jacobi_rows<kBlock, 7, 16, false>(W, ldw, gc, r, nullptr, 0, sh2, sig, 40, 1e-26, floor_rel);
+  else if (r <= 64)
+    team_jacobi_rows<kBlock, 13, 8, false>(W, ldw, gc, r, nullptr, 0, sh2, sig, 40, 1e-26, floor_rel);
+  else
+    team_jacobi_rows<kBlock, 25, 4, false>(W, ldw, gc, r, nullptr, 0, sh2, sig, 40, 1e-26, floor_rel);
+  sorted_norms(W, ldw, gc, r, sig, order);
+  int k = find_k(sig, order, r, eps);
   if (k > d.cap) {
     if (threadIdx.x == 0) atomicOr(overflow, 1);
     k = d.cap;
   }
   // G = U S V^T.  A = U sqrt(S), B = V sqrt(S) (or swapped when transposed).
-  T* A = arena + d.a;
-  T* B = arena + d.b;
-  for (int e = threadIdx.x; e < k * gr; e += kBlock) {
-    const int i = e % gr, c = e / gr;
-    const int j = order[c];
-    const double v = G[i + j * gr] / sqrt(sig[j]);
-    if (tr)
-      B[i + (size_t)c * d.n] = (T)v;
-    else
-      A[i + (size_t)c * d.m] = (T)v;
-  }
+  T* pu = arena + (tr ? d.b : d.a);  // gr x k
+  T* pv = arena + (tr ? d.a : d.b);  // gc x k
   for (int e = threadIdx.x; e < k * gc; e += kBlock) {
-    const int i = e % gc, c = e / gc;
-    const int j = order[c];
-    const double v = V[i + j * gc] * sqrt(sig[j]);
-    if (tr)
-      A[i + (size_t)c * d.m] = (T)v;
-    else
-      B[i + (size_t)c * d.n] = (T)v;
+    const int i = e % gc, c = e / gc, j = order[c];
+    pv[e] = (T)(W[i + j * ldw] / sqrt(sig[j]));
+  }
+  // u: threads 2 i and 2 i + 1 take the halves of row i's columns
+  constexpr int kC = 8;
+  const int row = threadIdx.x >> 1, h = threadIdx.x & 1, half = (gc + 1) / 2;
+  for (int c0 = 0; c0 < k; c0 += kC) {
+    const double* wj[kC];
+    double acc[kC];
+#pragma unroll
+    for (int b = 0; b < kC; ++b) {
+      wj[b] = W + order[c0 + b < k ? c0 + b : k - 1] * ldw;
+      acc[b] = 0.0;
+    }
+    if (row < gr)
+      for (int c = h * half; c < (h ? gc : half); ++c) {
+        const double v = get(row, c);
+#pragma unroll
+        for (int b = 0; b < kC; ++b) acc[b] += v * wj[b][c];
+      }
+#pragma unroll
+    for (int b = 0; b < kC; ++b) {
+      const double v = acc[b] + dpp_swap<0xB1>(acc[b]);
+      if (h == 0 && row < gr && c0 + b < k) {
+        const double sj = sig[order[c0 + b]];
+        pu[row + (size_t)(c0 + b) * gr] = (T)(v / (sj * sqrt(sj)));
+      }
+    }
   }
   if (threadIdx.x == 0) ranks[leaf] = k;
 }
