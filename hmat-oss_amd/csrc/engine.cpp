@@ -660,44 +660,78 @@ void Matrix::assemble_host_pass(const HostFunctions& f, const CompressionSpec& c
 // The item lists hold offsets in units of one right-hand side (the offsets for
 // nrhs right-hand sides are nrhs times these; the kernels scale them), so one
 // plan serves every nrhs and only the scratch buffers depend on it.
+//
+// The contributions of a destination range (a leaf cluster, or a piece of at
+// most kYRows rows of a wider one) are cut into runs of about 'grain' entries,
+// one workgroup each.  A run writes its own partial sums, so a smaller grain
+// costs slots (128 rows written and read again) and a larger one leaves the
+// device idle: grain = the entries over 2,048 (eight workgroups for each of
+// the 256 CUs), at least 4,096 entries (below that a workgroup is all launch
+// and metadata) and at most 32,768 (above it, the last runs of a long launch
+// are what is left running).
 void Matrix::build_gemv_plan() {
   GemvPlan& P = plan_;
-  P.max_rows = 0;
-  // the y pass takes destination leaf clusters of at most 512 rows: a matrix
-  // with wider ones has no H-gemv plan (its gemv reports it, the rest works)
+  // the plan takes leaf clusters of at most 512 rows: a matrix with wider ones
+  // has no H-gemv plan (its gemv reports it, the rest works)
   P.built = false;
   for (const Cluster* c : rows->leaves)
     if (c->size > 512) return;
-  const int nrhs = 1;
   const auto& D = s64.hdesc;
   const int nleaf = (int)D.size();
-  const int chunk = kZChunk;
+  // ranks as a hint for the sizes of the runs (they may change later)
+  std::vector<int> rk(nleaf, 0);
+  const DevBuf& rb = s64.ranks.p ? s64.ranks : s32.ranks;
+  if (rb.p && nleaf) {
+    HMX_CHECK(hipMemcpyAsync(rk.data(), rb.p, rk.size() * sizeof(int), hipMemcpyDeviceToHost, stream));
+    HMX_CHECK(hipStreamSynchronize(stream));
+  }
   std::vector<ZItem> zi;
   std::vector<ZReduce> zr;
-  std::vector<int64_t> zoff_side0(nleaf, -1), zoff_side1(nleaf, -1);
-  int64_t zpart = 0, zbuf = 0;
+  std::vector<int64_t> zoff[2] = {std::vector<int64_t>(nleaf, -1), std::vector<int64_t>(nleaf, -1)};
+  int64_t zpart = 0, zbuf = 0, counted_parts = 0;
   for (int l = 0; l < nleaf; ++l) {
     const LeafDesc& L = D[l];
     if (L.kind != 1) continue;
     const bool mir = bt->leaves[l]->mirrored() && lower_sym;
     for (int side = 0; side < (mir ? 2 : 1); ++side) {
       const int len = side == 0 ? L.n : L.m;
-      ZReduce red{l, (int)zi.size(), 0, 0, zbuf};
-      for (int r = 0; r < len; r += chunk) {
-        zi.push_back(ZItem{l, side, r, std::min(chunk, len - r), zpart});
-        zpart += (int64_t)L.cap * nrhs;
+      const int nch = (len + kZChunk - 1) / kZChunk;
+      const int64_t base = side == 0 ? L.b : L.a;
+      const int x0 = side == 0 ? L.c0 : L.r0;
+      if (nch > 1) zr.push_back(ZReduce{l, L.cap, nch, 0, zpart, zbuf});
+      for (int r = 0; r < len; r += kZChunk) {
+        zi.push_back(ZItem{base + r, nch > 1 ? zpart : zbuf, l, len, std::min(kZChunk, len - r), x0 + r, L.cap,
+                           nch > 1 ? 1 : 0});
+        if (nch > 1) zpart += L.cap;
       }
-      red.end = (int)zi.size();
-      zr.push_back(red);
-      (side == 0 ? zoff_side0 : zoff_side1)[l] = zbuf;
-      zbuf += (int64_t)L.cap * nrhs;
+      counted_parts += (int64_t)nch * L.cap;
+      zoff[side][l] = zbuf;
+      zbuf += L.cap;
     }
   }
-  // y pass: contributions grouped by destination leaf cluster of the rows tree
-  const auto& RL = rows->leaves;
-  std::vector<std::vector<YContrib>> per(RL.size());
-  std::vector<std::vector<int64_t>> slots_for(RL.size());
-  int64_t slot = 0;
+  // the chunks that take a workgroup first, then those of one wavefront; the
+  // longest of each first, so that the last ones running are short
+  P.nzlong = 0;
+  for (const ZItem& z : zi) P.nzlong += z.rows > kZChunk / 4;
+  std::stable_sort(zi.begin(), zi.end(), [&](const ZItem& a, const ZItem& b) {
+    const bool la = a.rows > kZChunk / 4, lb = b.rows > kZChunk / 4;
+    if (la != lb) return la;
+    return (int64_t)a.rows * rk[a.leaf] > (int64_t)b.rows * rk[b.leaf];
+  });
+  // y pass: contributions by destination range of the rows tree
+  struct Range {
+    int r0, len;
+  };
+  std::vector<Range> ranges;
+  std::vector<int> first_range;  // of a leaf cluster
+  for (const Cluster* c : rows->leaves) {
+    first_range.push_back((int)ranges.size());
+    for (int r = 0; r < c->size; r += kYRows) ranges.push_back(Range{c->offset + r, std::min(kYRows, c->size - r)});
+  }
+  first_range.push_back((int)ranges.size());
+  std::vector<std::vector<YContrib>> per(ranges.size());
+  std::vector<std::vector<int64_t>> slots_for(ranges.size());
+  int64_t slot = 0, counted_slots = 0, total = 0;
   for (int l = 0; l < nleaf; ++l) {
     const Block* b = bt->leaves[l];
     const LeafDesc& L = D[l];
@@ -705,72 +739,110 @@ void Matrix::build_gemv_plan() {
     if (L.kind == 0) {
       if (!b->rows->is_leaf() || !b->cols->is_leaf())
         throw std::runtime_error("gemv: full leaf spanning several leaf clusters");
-      YContrib c{l, 0, 0, 0, -1};
-      if (mir) {
-        c.z = slot;
-        slots_for[b->cols->leaf_index].push_back(slot);
-        slot += (int64_t)L.n * nrhs;
+      total += (int64_t)L.m * L.n;
+      if (mir) counted_slots += L.n;
+      for (int q = first_range[b->rows->leaf_index]; q < first_range[b->rows->leaf_index + 1]; ++q) {
+        // M^T x of these rows: one slot per range of the columns' cluster
+        const int row0 = ranges[q].r0 - L.r0;
+        const int qd = mir ? first_range[b->cols->leaf_index] : 0;
+        for (int c0 = 0; c0 < L.n; c0 += kYRows) {
+          const int nc = std::min(kYRows, L.n - c0);
+          int64_t z = -1;
+          if (mir) {
+            z = slot;
+            slot += nc;
+            slots_for[qd + c0 / kYRows].push_back(z);
+          }
+          for (int j = 0; j < nc; j += kYCols)
+            per[q].push_back(YContrib{L.a + row0 + (int64_t)(c0 + j) * L.m, z, -1, L.m, std::min(kYCols, nc - j),
+                                      L.c0 + c0 + j, nc, j});
+        }
       }
-      per[b->rows->leaf_index].push_back(c);
     } else {
-      for (int q = b->rows->first_leaf; q < b->rows->first_leaf + b->rows->nleaves; ++q)
-        per[q].push_back(YContrib{l, 2, RL[q]->offset - L.r0, 0, zoff_side0[l]});
-      if (mir)
-        for (int q = b->cols->first_leaf; q < b->cols->first_leaf + b->cols->nleaves; ++q)
-          per[q].push_back(YContrib{l, 3, RL[q]->offset - L.c0, 0, zoff_side1[l]});
+      total += (int64_t)rk[l] * ((int64_t)L.m + (mir ? L.n : 0));
+      for (int side = 0; side < (mir ? 2 : 1); ++side) {
+        // side 0: A z into the rows, side 1: B z' into the columns
+        const Cluster* c = side == 0 ? b->rows : b->cols;
+        const int64_t base = side == 0 ? L.a : L.b;
+        for (int q = first_range[c->first_leaf]; q < first_range[c->first_leaf + c->nleaves]; ++q)
+          per[q].push_back(YContrib{base + ranges[q].r0 - c->offset, zoff[side][l], l, c->size, 0, 0, L.cap, 0});
+      }
     }
   }
+  auto cost = [&](const YContrib& c, int len) {
+    // entries, plus the latency of an Rk slice however small its rank
+    return c.leaf < 0 ? (int64_t)len * c.n : (int64_t)len * (rk[c.leaf] + 2);
+  };
+  P.counted1 = counted_parts + zbuf + counted_slots + rows->n;
   std::vector<YItem> yi;
   std::vector<YContrib> contrib;
+  std::vector<YFinal> yf;
   std::vector<int64_t> slist;
-  for (size_t q = 0; q < RL.size(); ++q) {
-    P.max_rows = std::max(P.max_rows, RL[q]->size);
-    YItem it{RL[q]->offset, RL[q]->size, (int)contrib.size(), 0, (int)slist.size(), 0};
-    // full leaves first, then the Rk slices, which the y pass stages in batches
-    std::stable_partition(per[q].begin(), per[q].end(), [](const YContrib& c) { return c.kind == 0; });
-    contrib.insert(contrib.end(), per[q].begin(), per[q].end());
-    slist.insert(slist.end(), slots_for[q].begin(), slots_for[q].end());
-    it.end = (int)contrib.size();
-    it.send = (int)slist.size();
-    yi.push_back(it);
+  const int64_t array = (int64_t)(kNoAllocArrayBytes / sizeof(double)), admit = (int64_t)(kNoAllocScratchBytes / sizeof(double));
+  int64_t slots_used = 0;
+  for (int64_t grain = std::min<int64_t>(32768, std::max<int64_t>(4096, total / 2048));; grain *= 2) {
+    yi.clear();
+    contrib.clear();
+    yf.clear();
+    slist.clear();
+    slots_used = slot;
+    for (size_t q = 0; q < ranges.size(); ++q) {
+      const int len = ranges[q].len;
+      YFinal fin{ranges[q].r0, len, (int)slist.size(), 0};
+      size_t i = 0;
+      while (i < per[q].size()) {
+        YItem it{ranges[q].r0, len, (int)contrib.size(), 0, slots_used, 0, 0};
+        for (int64_t c = 0; i < per[q].size() && (c == 0 || c + cost(per[q][i], len) <= grain); ++i) {
+          c += cost(per[q][i], len);
+          if (per[q][i].leaf < 0 && per[q][i].z >= 0) it.mirrored = 1;
+          contrib.push_back(per[q][i]);
+        }
+        it.end = (int)contrib.size();
+        yi.push_back(it);
+        slist.push_back(slots_used);
+        slots_used += len;
+      }
+      slist.insert(slist.end(), slots_for[q].begin(), slots_for[q].end());
+      fin.end = (int)slist.size();
+      yf.push_back(fin);
+    }
+    // the allocation-free entry point admits nrhs by counted1 and must hold
+    // this plan's scratch then: fewer, longer runs where it would not
+    const int64_t most = std::max<int64_t>(admit / std::max<int64_t>(P.counted1, 1), 1);
+    if ((zpart + zbuf + slots_used) * most <= array || P.counted1 > admit || (int64_t)yi.size() <= (int64_t)ranges.size())
+      break;
   }
   upload(P.zitems, zi.data(), zi.size() * sizeof(ZItem), stream);
   upload(P.zred, zr.data(), zr.size() * sizeof(ZReduce), stream);
   upload(P.yitems, yi.data(), yi.size() * sizeof(YItem), stream);
   upload(P.contrib, contrib.data(), contrib.size() * sizeof(YContrib), stream);
+  upload(P.yfinal, yf.data(), yf.size() * sizeof(YFinal), stream);
   upload(P.slotlist, slist.data(), slist.size() * sizeof(int64_t), stream);
   P.zpart1 = zpart;
   P.z1 = zbuf;
-  P.slot1 = slot;
+  P.slot1 = slots_used;
   P.nz = (int)zi.size();
   P.nzred = (int)zr.size();
   P.ny = (int)yi.size();
+  P.nfinal = (int)yf.size();
   P.built = true;
   P.nrhs = 0;
   HMX_CHECK(hipStreamSynchronize(stream));
 }
 
-size_t Matrix::gemv_scratch_elems(int nrhs) const {
-  const GemvPlan& P = plan_;
-  return (size_t)(P.zpart1 + P.z1 + P.slot1 + rows->n) * (size_t)nrhs;
-}
+size_t Matrix::gemv_scratch_elems(int nrhs) const { return (size_t)plan_.counted1 * (size_t)nrhs; }
 
 template <typename T>
 void Matrix::gemv_launch(double alpha, const T* x, double beta, T* y, int nrhs, int ldx, int ldy,
-                         const Store<T>& st, double* zpart, double* z, double* slots,
-                         double* acc) {
+                         const Store<T>& st, double* zpart, double* z, double* slots) {
   const GemvPlan& P = plan_;
-  const LeafDesc* desc = st.desc.template as<LeafDesc>();
   const int* ranks = st.ranks.template as<int>();
-  launch_gemv_zpass<T>(desc, ranks, st.data(), P.zitems.as<ZItem>(), P.nz, x, ldx, nrhs, zpart,
-                       stream);
-  launch_gemv_zreduce(P.zred.as<ZReduce>(), P.nzred, ranks, zpart, P.zitems.as<ZItem>(), nrhs,
-                      desc, z, stream);
-  launch_gemv_ypass<T>(desc, ranks, st.data(), P.yitems.as<YItem>(), P.ny,
-                       P.contrib.as<YContrib>(), z, slots, x, ldx, nrhs, acc, rows->n, P.max_rows,
-                       stream);
-  launch_gemv_yfinal<T>(P.yitems.as<YItem>(), P.ny, P.slotlist.as<int64_t>(), slots, acc,
-                        rows->n, y, ldy, nrhs, alpha, beta, stream);
+  launch_gemv_zpass<T>(ranks, st.data(), P.zitems.as<ZItem>(), P.nzlong, P.nz, x, ldx, nrhs, zpart, z, stream);
+  launch_gemv_zreduce(P.zred.as<ZReduce>(), P.nzred, ranks, zpart, nrhs, z, stream);
+  launch_gemv_ypass<T>(ranks, st.data(), P.yitems.as<YItem>(), P.ny, P.contrib.as<YContrib>(), z, slots, x,
+                       ldx, nrhs, stream);
+  launch_gemv_yfinal<T>(P.yfinal.as<YFinal>(), P.nfinal, P.slotlist.as<int64_t>(), slots, y, ldy, nrhs,
+                        alpha, beta, stream);
 }
 
 template <typename T>
@@ -786,11 +858,10 @@ void Matrix::gemv_device(double alpha, const T* x, double beta, T* y, int nrhs, 
     P.zpart.ensure(std::max<int64_t>(P.zpart1 * nrhs, 1) * sizeof(double));
     P.z.ensure(std::max<int64_t>(P.z1 * nrhs, 1) * sizeof(double));
     P.slots.ensure(std::max<int64_t>(P.slot1 * nrhs, 1) * sizeof(double));
-    P.acc.ensure((size_t)rows->n * nrhs * sizeof(double));
     P.nrhs = nrhs;
   }
   gemv_launch<T>(alpha, x, beta, y, nrhs, ldx, ldy, st, P.zpart.as<double>(), P.z.as<double>(),
-                 P.slots.as<double>(), P.acc.as<double>());
+                 P.slots.as<double>());
 }
 
 template <typename T>
@@ -800,17 +871,17 @@ void Matrix::gemv_device_scratch(double alpha, const T* x, double beta, T* y, in
   if (!plan_.built)
     throw std::runtime_error("gemv: no H-gemv plan (matrix not assembled, or leaf clusters above 512 rows)");
   if (nrhs < 1) throw std::runtime_error("gemv: nrhs must be positive");
+  const GemvPlan& P = plan_;
   const size_t need = gemv_scratch_elems(nrhs);
-  if (need > scratch_elems)
+  if (need * sizeof(double) > kNoAllocScratchBytes ||
+      (size_t)(P.zpart1 + P.z1 + P.slot1) * (size_t)nrhs > scratch_elems)
     throw std::runtime_error("gemv: needs " + std::to_string(need * sizeof(double)) +
                              " bytes of scratch, the allocation-free entry point has " +
-                             std::to_string(scratch_elems * sizeof(double)));
-  const GemvPlan& P = plan_;
+                             std::to_string(kNoAllocScratchBytes));
   double* zpart = scratch;
   double* z = zpart + P.zpart1 * nrhs;
   double* slots = z + P.z1 * nrhs;
-  double* acc = slots + P.slot1 * nrhs;
-  gemv_launch<T>(alpha, x, beta, y, nrhs, n_cols(), n_rows(), st, zpart, z, slots, acc);
+  gemv_launch<T>(alpha, x, beta, y, nrhs, n_cols(), n_rows(), st, zpart, z, slots);
 }
 template void Matrix::gemv_device_scratch<double>(double, const double*, double, double*, int,
                                                   const Store<double>&, double*, size_t);

@@ -78,11 +78,11 @@ struct KernelSpec {
 struct GemvPlan {
   bool built = false;
   int nrhs = 0;       // scratch buffers below hold this many right-hand sides
-  DevBuf zitems, zred, yitems, contrib, slotlist;
-  int nz = 0, nzred = 0, ny = 0;
-  int max_rows = 0;   // rows of the largest destination leaf cluster
+  DevBuf zitems, zred, yitems, contrib, yfinal, slotlist;
+  int nz = 0, nzlong = 0, nzred = 0, ny = 0, nfinal = 0;
   int64_t zpart1 = 0, z1 = 0, slot1 = 0;  // scratch doubles per right-hand side
-  DevBuf zpart, z, slots, acc;
+  int64_t counted1 = 0;  // the count by which the allocation-free entry point admits products
+  DevBuf zpart, z, slots;
 };
 
 struct Stats {
@@ -290,7 +290,7 @@ class Matrix {
   void build_gemv_plan();
   template <typename T>
   void gemv_launch(double alpha, const T* x, double beta, T* y, int nrhs, int ldx, int ldy,
-                   const Store<T>& st, double* zpart, double* z, double* slots, double* acc);
+                   const Store<T>& st, double* zpart, double* z, double* slots);
   GemvPlan plan_;
   DevBuf overflow_;
   std::shared_ptr<struct FactorState> fstate_;

@@ -68,35 +68,47 @@ void launch_aca(const LeafDesc* desc, const AcaTask* tasks, int count, T* arena,
                 const double* table = nullptr);
 
 // ---- H-gemv -----------------------------------------------------------------
-// Work items of the z pass: z_part = P^T x over a row range of a panel of at
-// most kZChunk rows.
+// Offsets into z, zpart and the slots are per right-hand side: the data of a
+// record sits at nrhs times its offset, one column of 'cap' (z) or the slot's
+// rows (slots) per right-hand side.
+//
+// z pass: P^T x over at most kZChunk rows of a panel, into z, or into zpart
+// where the panel has several chunks.
 constexpr int kZChunk = 1024;
 struct ZItem {
-  int leaf;
-  int side;       // 0: B panel against x[cols]  (z),  1: A panel against x[rows] (z')
-  int row0, rows; // local row range inside the panel
-  int64_t zslot;  // output slot offset per right-hand side (the slot holds cap * nrhs doubles
-                  // at nrhs * zslot)
+  int64_t p;        // first row of the chunk in the arena
+  int64_t z;        // output offset
+  int leaf, ld, rows;
+  int x0;           // the chunk's first entry of x
+  int cap, part;
 };
-// y pass: one work item per destination leaf cluster.  Contributions:
-//   kind 0: full leaf with rows == destination: acc += M x[cols]; if the leaf is
-//           mirrored (symmetric storage) also slot[fslot] = M^T x[rows]
-//   kind 2: Rk A panel rows [row0, row0+len): acc += A z
-//   kind 3: Rk B panel rows [row0, row0+len) (mirrored Rk): acc += B z'
-// and the final pass adds the mirrored-full slots that target the cluster:
-//   y[r0:r0+len] = beta y + alpha (acc + sum slots)
+// z = sum of a panel's chunks, at part, part + cap, ...
+struct ZReduce {
+  int leaf, cap, count, pad;
+  int64_t part, z;
+};
+// y pass: one work item per run of a destination range's contributions:
+//   leaf < 0: n columns of a full leaf's rows, acc += M x; with z >= 0 also
+//             slot z (cap rows), rows [col0, col0 + n) = M^T x[range]
+//   else    : the range's rows of an Rk panel, acc += P z
+// acc goes to the slot 'out' (len rows); the final pass adds the slots that
+// target a range: y[r0:r0+len] = beta y + alpha sum.
+constexpr int kYRows = 128;  // rows of a destination range (at most)
+constexpr int kYCols = 32;   // columns of a full leaf's contribution (at most)
 struct YItem {
-  int r0, len;
+  int x0, len;      // the range's first row (entry of x for M^T x) and its rows
   int beg, end;     // contribution range
-  int sbeg, send;   // slot-list range (indices into slot_list)
+  int64_t out;
+  int mirrored, pad;  // 1: some contribution has a slot
 };
 struct YContrib {
-  int leaf;
-  int kind;
-  int row0;
-  int pad;
-  int64_t z;       // z / z' offset for rk, slot offset for mirrored full (doubles per
-                   // right-hand side: the data sits at nrhs * z), else -1
+  int64_t p;        // first entry in the arena
+  int64_t z;
+  int leaf, ld, n, x0, cap, col0;
+};
+struct YFinal {
+  int r0, len;
+  int beg, end;     // slot-list range
 };
 
 // ---- whole-matrix leaf operations (k_ops.hip); one workgroup per listed leaf
@@ -134,34 +146,27 @@ void launch_gauss(double* out, size_t n, uint64_t seed, hipStream_t s);
 void launch_pick_scale(const double* V, int ldv, int rows, int first, int count,
                        const double* lam, double e, double* out, hipStream_t s);
 
-// Fixed device scratch of the allocation-free H-gemv (64 MiB per GPU); returns
-// its device address on the current device (looked up once per device).
+// Fixed device scratch of the allocation-free H-gemv: products of up to
+// kNoAllocScratchBytes of temporaries by gemv_scratch_elems' count are taken;
+// the array holds the most that the present plan lays out for such a product.
+// Returns its device address on the current device (looked up once per device).
 constexpr size_t kNoAllocScratchBytes = size_t(64) << 20;
+constexpr size_t kNoAllocArrayBytes = 4 * kNoAllocScratchBytes;
 double* noalloc_gemv_scratch(size_t* elems);
 
 template <typename T>
-void launch_gemv_zpass(const LeafDesc* desc, const int* ranks, const T* arena, const ZItem* items,
-                       int count, const T* x, int ldx, int nrhs, double* zpart, hipStream_t s);
-// Sums z partial slots per (leaf, side): z[z] = sum of slots of items [beg, end).
-struct ZReduce {
-  int leaf;
-  int beg, end;
-  int pad;
-  int64_t z;
-};
-void launch_gemv_zreduce(const ZReduce* red, int count, const int* ranks, const double* zpart,
-                         const ZItem* items, int nrhs, const LeafDesc* desc, double* z,
-                         hipStream_t s);
+// (the first nlong items have more than kZChunk / 4 rows, the others at most that)
+void launch_gemv_zpass(const int* ranks, const T* arena, const ZItem* items, int nlong, int count,
+                       const T* x, int ldx, int nrhs, double* zpart, double* z, hipStream_t s);
+void launch_gemv_zreduce(const ZReduce* red, int count, const int* ranks, const double* zpart, int nrhs,
+                         double* z, hipStream_t s);
 template <typename T>
-// (max_rows: the largest destination leaf cluster, at most 512 rows)
-void launch_gemv_ypass(const LeafDesc* desc, const int* ranks, const T* arena, const YItem* items,
-                       int count, const YContrib* contrib, const double* z, double* slots,
-                       const T* x, int ldx, int nrhs, double* acc, int ldacc, int max_rows,
-                       hipStream_t s);
+void launch_gemv_ypass(const int* ranks, const T* arena, const YItem* items, int count,
+                       const YContrib* contrib, const double* z, double* slots, const T* x, int ldx,
+                       int nrhs, hipStream_t s);
 template <typename T>
-void launch_gemv_yfinal(const YItem* items, int count, const int64_t* slot_list,
-                        const double* slots, const double* acc, int ldacc, T* y, int ldy,
-                        int nrhs, double alpha, double beta, hipStream_t s);
+void launch_gemv_yfinal(const YFinal* items, int count, const int64_t* slot_list, const double* slots,
+                        T* y, int ldy, int nrhs, double alpha, double beta, hipStream_t s);
 
 // Refinement helpers on column-major N x nrhs vectors (ld = n).
 void launch_vec_add_f2d(double* x, const float* d, size_t n, hipStream_t s);   // x += d
