@@ -346,7 +346,9 @@ int init_engine() {
     if (n < 1) throw std::runtime_error("no HIP device");
   });
 }
-int finalize_engine() { return 0; }
+int finalize_engine() {
+  return guard([] { hmx::release_kept_memory(); });
+}
 
 int get_info(hmat_matrix_t* h, hmat_info_t* info) {
   return guard([&] { M(h)->info(*info); });
@@ -988,8 +990,7 @@ int hmx_run_batch(hmat_matrix_t** ms, hmat_assemble_context_t** ctx, int count, 
     if (count < 0 || threads < 1) throw std::runtime_error("hmx_run_batch: bad count or thread count");
     // several host threads submit at once: each system keeps to its own stream
     // and to its share of the device memory for temporaries
-    size_t freeb = 0, total = 0;
-    HMX_CHECK(hipMemGetInfo(&freeb, &total));
+    const size_t freeb = hmx::device_free_bytes();
     const int workers = std::min(threads, std::max(count, 1));
     const size_t share = std::min((size_t)(0.5 * (double)freeb / workers), (size_t)96 << 30);
     for (int i = 0; i < count; ++i) {

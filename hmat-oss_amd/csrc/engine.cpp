@@ -6,13 +6,90 @@
 
 #include "factor_kernels.hpp"
 #include <chrono>
+#include <list>
+#include <mutex>
 #include <cstring>
 #include <functional>
 #include <stdexcept>
 
 namespace hmx {
 
+// ---- device buffers kept between objects --------------------------------------
+// A buffer given up by a DevBuf is kept for the next one of its size instead
+// of going back to the driver, which clears device memory before it hands it
+// out again: a program that builds, factorises and drops one matrix after the
+// other (a likelihood per hyperparameter, a batch of systems) spent most of
+// its time there (N = 50,000: assembly 12 ms of kernels, 474 ms a pass; an
+// 8,000-point likelihood and gradient 107 ms with clean memory at hand, 204 ms
+// without).  At most kept_limit() bytes are kept per process and device, the
+// oldest go first; all of them go back when an allocation fails and at
+// hmat_interface_t.finalize.
+//
+// release() waits for the device, as hipFree does, so that a kept buffer has
+// no work of any stream left on it; the lists are guarded by a mutex.
+namespace {
+struct KeptBuffer {
+  void* p;
+  size_t bytes;
+  int dev;
+};
+std::mutex kept_mutex;
+std::list<KeptBuffer>& kept_list() {  // oldest first; never destroyed (the runtime may end before it)
+  static auto* l = new std::list<KeptBuffer>;
+  return *l;
+}
+size_t kept_bytes = 0;
+
+// an eighth of the device's memory: 36 GB of 288
+size_t kept_limit() {
+  size_t freeb = 0, total = 0;
+  if (hipMemGetInfo(&freeb, &total) != hipSuccess) return 0;
+  return total / 8;
+}
+
+// sizes are rounded up to an eighth of their power of two, so that buffers of
+// similar objects fit each other
+size_t rounded_size(size_t n) {
+  size_t step = 256;
+  while (step * 16 <= n) step *= 2;
+  return (n + step - 1) / step * step;
+}
+}  // namespace
+
+void release_kept_memory() {
+  std::lock_guard<std::mutex> lock(kept_mutex);
+  for (const KeptBuffer& k : kept_list()) (void)hipFree(k.p);
+  kept_list().clear();
+  kept_bytes = 0;
+}
+
+size_t device_free_bytes() {
+  size_t freeb = 0, total = 0;
+  HMX_CHECK(hipMemGetInfo(&freeb, &total));
+  int dev = 0;
+  HMX_CHECK(hipGetDevice(&dev));
+  std::lock_guard<std::mutex> lock(kept_mutex);
+  for (const KeptBuffer& k : kept_list())
+    if (k.dev == dev) freeb += k.bytes;
+  return freeb;
+}
+
 void DevBuf::release() {
+  if (p && hipDeviceSynchronize() == hipSuccess) {
+    static const size_t limit = kept_limit();
+    std::lock_guard<std::mutex> lock(kept_mutex);
+    if (bytes <= limit) {
+      auto& l = kept_list();
+      l.push_back(KeptBuffer{p, bytes, dev});
+      kept_bytes += bytes;
+      while (kept_bytes > limit) {
+        (void)hipFree(l.front().p);
+        kept_bytes -= l.front().bytes;
+        l.pop_front();
+      }
+      p = nullptr;
+    }
+  }
   if (p) (void)hipFree(p);
   p = nullptr;
   bytes = 0;
@@ -20,9 +97,35 @@ void DevBuf::release() {
 
 void DevBuf::alloc(size_t nbytes) {
   release();
-  if (nbytes == 0) nbytes = 256;
-  HMX_CHECK(hipMalloc(&p, nbytes));
-  bytes = nbytes;
+  const size_t want = rounded_size(std::max<size_t>(nbytes, 1));
+  int d = 0;
+  HMX_CHECK(hipGetDevice(&d));
+  {
+    std::lock_guard<std::mutex> lock(kept_mutex);
+    auto& l = kept_list();
+    auto best = l.end();
+    for (auto it = l.begin(); it != l.end(); ++it)
+      if (it->dev == d && it->bytes >= want && it->bytes <= want + want / 4 &&
+          (best == l.end() || it->bytes < best->bytes))
+        best = it;
+    if (best != l.end()) {
+      p = best->p;
+      bytes = best->bytes;
+      dev = d;
+      kept_bytes -= bytes;
+      l.erase(best);
+      return;
+    }
+  }
+  hipError_t e = hipMalloc(&p, want);
+  if (e != hipSuccess) {
+    (void)hipGetLastError();
+    release_kept_memory();
+    p = nullptr;
+    HMX_CHECK(hipMalloc(&p, want));
+  }
+  bytes = want;
+  dev = d;
 }
 
 void DevBuf::ensure(size_t nbytes) {
@@ -274,8 +377,7 @@ int aca_kmax(const LeafDesc& L) {
 // memory, between 4 and 64 GiB (a larger launch runs more blocks side by side;
 // each launch lasts as long as its slowest block)
 int64_t aca_budget_doubles() {
-  size_t freeb = 0, total = 0;
-  HMX_CHECK(hipMemGetInfo(&freeb, &total));
+  const size_t freeb = device_free_bytes();
   const int64_t lo = (int64_t)4 << 30, hi = (int64_t)64 << 30;
   return std::min(hi, std::max(lo, (int64_t)(freeb / 4))) / (int64_t)sizeof(double);
 }
@@ -305,8 +407,7 @@ void Matrix::assemble_pass(const KernelSpec& k, const CompressionSpec& comp) {
   // device memory stays with partial ACA)
   std::vector<int> giant;
   if (embedded && comp.method != 0) {
-    size_t freeb = 0, total = 0;
-    HMX_CHECK(hipMemGetInfo(&freeb, &total));
+    const size_t freeb = device_free_bytes();
     for (size_t i = 0; i < bt->leaves.size(); ++i) {
       const LeafDesc& L = s64.hdesc[i];
       if (L.kind == 1 && std::min(L.m, L.n) >= giant_rows &&
@@ -420,33 +521,58 @@ void Matrix::assemble_pass(const KernelSpec& k, const CompressionSpec& comp) {
     }
   }
   // ACA blocks, the largest first, in launches bounded by a workspace budget.
+  // Most blocks stop far below the room their leaf's capacity would give
+  // (ranks of 5 to 25 in panels of 320 columns, 16 GB of workspace at
+  // N = 50,000): a first round with panels of kAcaRoom columns, and the blocks
+  // that fill them run again, from their start, with four times the room up to
+  // their full one.
+  const int kAcaRoom = embedded ? 128 : 32;
   std::vector<AcaTask> acat;
-  for (int l : aca) acat.push_back(AcaTask{l, aca_kmax(s64.hdesc[l]), 0});
-  sort_aca_by_size(acat, s64.hdesc);
+  for (int l : aca) {
+    const int full_room = aca_kmax(s64.hdesc[l]), room = std::min(full_room, kAcaRoom);
+    acat.push_back(AcaTask{l, room, 0, -1, room == full_room});
+  }
   const int64_t budget = acat.empty() ? 0 : aca_budget_doubles();
   const int partial = comp.method == 2;
-  size_t i = 0;
   DevBuf ws, dt;
   const int nleaf = (int)bt->leaves.size();
-  while (i < acat.size()) {
-    HMX_CHECK(hipStreamSynchronize(stream));
-    report_assembly(nleaf - (int)(acat.size() - i), nleaf);
-    std::vector<AcaTask> batch;
-    int64_t used = 0;
+  while (!acat.empty()) {
+    sort_aca_by_size(acat, s64.hdesc);
+    bool again = false;
+    size_t i = 0;
     while (i < acat.size()) {
-      const LeafDesc& L = s64.hdesc[acat[i].leaf];
-      const int64_t need = aca_workspace(L.m, L.n, acat[i].kmax);
-      if (!batch.empty() && used + need > budget) break;
-      batch.push_back(AcaTask{acat[i].leaf, acat[i].kmax, used});
-      used += need;
-      ++i;
+      HMX_CHECK(hipStreamSynchronize(stream));
+      report_assembly(nleaf - (int)(acat.size() - i), nleaf);
+      std::vector<AcaTask> batch;
+      int64_t used = 0;
+      while (i < acat.size()) {
+        const LeafDesc& L = s64.hdesc[acat[i].leaf];
+        const int64_t need = aca_workspace(L.m, L.n, acat[i].kmax);
+        if (!batch.empty() && used + need > budget) break;
+        batch.push_back(acat[i]);
+        batch.back().ws = used;
+        again |= !acat[i].last;
+        used += need;
+        ++i;
+      }
+      ws.ensure((size_t)used * sizeof(double));
+      upload(dt, batch.data(), batch.size() * sizeof(AcaTask), stream);
+      launch_aca<double>(s64.desc.as<LeafDesc>(), dt.as<AcaTask>(), (int)batch.size(), s64.data(),
+                         s64.ranks.as<int>(), overflow_.as<int>(), ws.as<double>(), rp, cp, kp,
+                         comp.eps, lowrank_eps, partial, stream);
     }
-    HMX_CHECK(hipStreamSynchronize(stream));
-    ws.ensure((size_t)used * sizeof(double));
-    upload(dt, batch.data(), batch.size() * sizeof(AcaTask), stream);
-    launch_aca<double>(s64.desc.as<LeafDesc>(), dt.as<AcaTask>(), (int)batch.size(), s64.data(),
-                       s64.ranks.as<int>(), overflow_.as<int>(), ws.as<double>(), rp, cp, kp,
-                       comp.eps, lowrank_eps, partial, stream);
+    std::vector<AcaTask> more;
+    if (again) {
+      std::vector<int> rk(nleaf);
+      HMX_CHECK(hipMemcpyAsync(rk.data(), s64.ranks.p, rk.size() * sizeof(int), hipMemcpyDeviceToHost, stream));
+      HMX_CHECK(hipStreamSynchronize(stream));
+      for (const AcaTask& t : acat)
+        if (rk[t.leaf] == kAcaRoomFull) {
+          const int full_room = aca_kmax(s64.hdesc[t.leaf]), room = std::min(full_room, 4 * t.kmax);
+          more.push_back(AcaTask{t.leaf, room, 0, -1, room == full_room});
+        }
+    }
+    acat.swap(more);
   }
 }
 
@@ -910,16 +1036,25 @@ void gemv_host_t(Matrix& M, const void* alpha, void* x, const void* beta, void* 
   const int n = M.n_rows(), nc = M.n_cols();
   std::vector<T> hx((size_t)nc * nrhs), hy((size_t)n * nrhs);
   const T a = *(const T*)alpha, b = *(const T*)beta;
+  const bool read_y = b != (T)0;
   if (permute) {
     permute_in((const T*)x, hx.data(), M.cols->indices, nc, nrhs);
-    permute_in((const T*)y, hy.data(), M.rows->indices, n, nrhs);
+    if (read_y) permute_in((const T*)y, hy.data(), M.rows->indices, n, nrhs);
   } else {
     std::memcpy(hx.data(), x, hx.size() * sizeof(T));
-    std::memcpy(hy.data(), y, hy.size() * sizeof(T));
+    if (read_y) std::memcpy(hy.data(), y, hy.size() * sizeof(T));
   }
-  DevBuf dx, dy;
-  upload(dx, hx.data(), hx.size() * sizeof(T), M.stream);
-  upload(dy, hy.data(), hy.size() * sizeof(T), M.stream);
+  // device copies kept with the matrix; hx and hy outlive the copies on every
+  // way out, so the call waits once
+  struct Wait {
+    hipStream_t s;
+    ~Wait() { (void)hipStreamSynchronize(s); }
+  } wait{M.stream};
+  DevBuf &dx = M.host_x, &dy = M.host_y;
+  dx.ensure(hx.size() * sizeof(T));
+  dy.ensure(hy.size() * sizeof(T));
+  HMX_CHECK(hipMemcpyAsync(dx.p, hx.data(), hx.size() * sizeof(T), hipMemcpyHostToDevice, M.stream));
+  if (read_y) HMX_CHECK(hipMemcpyAsync(dy.p, hy.data(), hy.size() * sizeof(T), hipMemcpyHostToDevice, M.stream));
   M.gemv_device<T>((double)a, dx.as<T>(), (double)b, dy.as<T>(), nrhs, nc, n, M.store<T>());
   HMX_CHECK(hipMemcpyAsync(hy.data(), dy.p, hy.size() * sizeof(T), hipMemcpyDeviceToHost, M.stream));
   HMX_CHECK(hipStreamSynchronize(M.stream));

@@ -17,10 +17,12 @@
 
 namespace hmx {
 
-// Owning device allocation.
+// Owning device allocation.  Buffers given up are kept for later ones, within
+// a bound (see engine.cpp); the content of a new one is undefined.
 struct DevBuf {
   void* p = nullptr;
   size_t bytes = 0;
+  int dev = 0;
   DevBuf() = default;
   DevBuf(const DevBuf&) = delete;
   DevBuf& operator=(const DevBuf&) = delete;
@@ -33,6 +35,11 @@ struct DevBuf {
 };
 
 void upload(DevBuf& b, const void* src, size_t bytes, hipStream_t s);
+
+// Gives the kept buffers back to the driver.
+void release_kept_memory();
+// Free memory of the current device, the kept buffers included.
+size_t device_free_bytes();
 
 // Leaf storage of one precision.
 template <typename T>
@@ -193,6 +200,8 @@ class Matrix {
   DevBuf hodlr_buf, hodlr_logdet;
   int overflow = 0;
   Stats stats;
+
+  DevBuf host_x, host_y;  // device copies of the vectors of gemv_host
 
   // points of the kernel, hmat order (rows tree), SoA, plus user indices
   DevBuf pts_rows, user_rows;

@@ -275,8 +275,7 @@ class Exec {
     eps_ = M.lowrank_eps;
     cap_max_ = M.rk_cap_max;
     if (fs_.temp_budget == 0) {
-      size_t freeb = 0, total = 0;
-      HMX_CHECK(hipMemGetInfo(&freeb, &total));
+      const size_t freeb = device_free_bytes();
       fs_.temp_budget = std::min((size_t)(0.5 * (double)freeb), (size_t)96 << 30);
       if (M.temp_budget_limit) fs_.temp_budget = std::min(fs_.temp_budget, M.temp_budget_limit);
     }

@@ -595,6 +595,10 @@ __global__ void __launch_bounds__(kBlock) k_aca(const LeafDesc* desc, const AcaT
     k = aca_partial(c, w, t.kmax, aca_eps, red, rv, ri, tmp);
   else
     k = aca_plus(c, w, t.kmax, aca_eps, red, rv, ri, tmp);
+  if (k >= t.kmax && !t.last) {
+    if (threadIdx.x == 0) ranks[t.leaf] = kAcaRoomFull;
+    return;
+  }
   // stopped by the panel room rather than by the criterion: the host grows
   // the capacities and assembles again
   const int room = d.m < d.n ? d.m : d.n;

@@ -53,7 +53,9 @@ struct AcaTask {
   int kmax;       // capacity of the ACA panels
   int64_t ws;     // offset (doubles) of this task's workspace
   int64_t tab = -1;  // offset of the block staged by the host in the table, or -1
+  int last = 1;      // 0: a block that fills its panels gets rank kAcaRoomFull (it runs again)
 };
+constexpr int kAcaRoomFull = -2;
 
 // Workspace (doubles) needed by one ACA task followed by its truncation.
 int64_t aca_workspace(int m, int n, int kmax);

@@ -1,0 +1,77 @@
+"""Device buffers that outlive their matrix, and the ACA's panel rooms.
+
+* Matrices of changing sizes and types built, factorised and dropped one after
+  the other, in one thread and in four, reuse each other's buffers: every
+  product equals that of the matrix's own leaves (4 N u |A| |x|), every solve
+  leaves the compression's residual.
+* hmat_interface_t.finalize gives the kept buffers back.
+* Blocks whose ACA needs more columns than its first room (32) run again: at
+  eps 1e-13 the ranks are above it and the matrix is within 1,000 eps of the
+  exact kernel's."""
+import threading
+
+import numpy as np
+import pytest
+
+hmat_amd = pytest.importorskip("hmat_amd")
+
+pytestmark = pytest.mark.gpu
+
+
+def _points(n, seed, height=1.5):
+    u = np.random.default_rng(seed).random((n, 2))
+    return np.column_stack([np.cos(2 * np.pi * u[:, 0]), np.sin(2 * np.pi * u[:, 0]), height * u[:, 1]])
+
+
+def _one(n, seed, leaf, factor):
+    t = hmat_amd.ClusterTree(_points(n, seed), leaf)
+    h = hmat_amd.HMatrix(t)
+    h.assemble(length=0.5, nugget=1e-1, eps=1e-6)
+    A = h.to_dense()
+    x = np.random.default_rng(seed).standard_normal((n, 3))
+    y = h.gemv(x, permute=False)
+    assert (np.abs(y - A @ x) <= 4 * n * 2.0 ** -53 * (np.abs(A) @ np.abs(x))).all()
+    if factor:
+        h.factorize(hmat_amd.FACT_LLT, mixed=(seed % 2 == 1))
+        if seed % 2 == 0:
+            s = h.solve(x, permute=False)
+            assert np.linalg.norm(A @ s - x) <= 1e-2 * np.linalg.norm(x)
+    h.close()
+
+
+def test_buffers_reused_and_given_back():
+    import torch
+    for seed, (n, leaf) in enumerate([(1500, 64), (900, 32), (1600, 64), (1500, 64), (400, 100), (1550, 64)]):
+        _one(n, seed, leaf, factor=True)
+    errors = []
+
+    def work(seed):
+        try:
+            for k in range(3):
+                _one(700 + 50 * seed + k, seed, 64, factor=False)
+        except Exception as e:  # noqa: BLE001 - reported below
+            errors.append(e)
+    threads = [threading.Thread(target=work, args=(s,)) for s in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not errors, errors
+    before = torch.cuda.mem_get_info()[0]
+    assert hmat_amd.interface().finalize() == 0
+    assert torch.cuda.mem_get_info()[0] > before
+    _one(1000, 8, 64, factor=True)
+
+
+def test_aca_rooms():
+    n = 1600
+    pts = _points(n, 5)
+    t = hmat_amd.ClusterTree(pts, 100)
+    h = hmat_amd.HMatrix(t, lowrank_eps=1e-13)
+    h.assemble(length=0.5, nugget=0.0, eps=1e-13)
+    tab = h.leaf_table()
+    assert tab[(tab[:, 4] == 1) & (np.maximum(tab[:, 0], tab[:, 1]) >= 100)][:, 5].max() > 32
+    P = pts[t.indices]
+    K = np.exp(-np.sqrt(((P[:, None] - P[None]) ** 2).sum(axis=2)) / 0.5)
+    assert np.linalg.norm(h.to_dense() - K) <= 1e-10 * np.linalg.norm(K)
+    h.close()
