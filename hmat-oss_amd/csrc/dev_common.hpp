@@ -8,6 +8,7 @@
 #include <cstdio>
 #include <stdexcept>
 #include <string>
+#include <type_traits>
 
 #define HMX_CHECK(expr)                                                                    \
   do {                                                                                     \
@@ -88,6 +89,26 @@ __host__ __device__ inline double kernel_value(const KernelParams& k, double dx,
   return v;
 }
 
+// ---- address spaces ----------------------------------------------------------
+// Pointers read from memory (task records) or passed between functions are
+// generic, and their accesses flat: slower, and counted with the LDS accesses,
+// so that every wait for LDS also waits for the loads in flight.  Operands
+// known to be in global memory or in LDS are cast to these types first.
+template <typename T>
+struct InGlobal {
+  typedef T __attribute__((address_space(1))) type;
+};
+template <typename T>
+using gptr = typename InGlobal<T>::type*;
+template <typename T>
+using cgptr = const typename InGlobal<T>::type*;
+template <typename T>
+struct InLds {
+  typedef T __attribute__((address_space(3))) type;
+};
+template <typename T>
+using lptr = typename InLds<T>::type*;
+
 // ---- staging global -> LDS ----------------------------------------------------
 // Copies an m x n block into LDS, dst[i + j * ldd] = src[i * si + j * sj] for
 // i < mv, j < nv and 0 elsewhere.  Each thread issues kStage independent loads
@@ -97,9 +118,11 @@ __host__ __device__ inline double kernel_value(const KernelParams& k, double dx,
 // whole leaf takes a larger kS so that it is one or two round trips.
 constexpr int kStage = 8;
 
-template <typename D, typename S, int kS = kStage>
-__device__ inline void stage_in(D* dst, int ldd, const S* src, long si, long sj, int m, int n,
+template <typename PD, typename PS, int kS = kStage>
+__device__ inline void stage_in(PD dst, int ldd, PS src, long si, long sj, int m, int n,
                                 int mv, int nv, double scale = 1.0) {
+  using D = std::decay_t<decltype(dst[0] + 0)>;  // values, whatever the address spaces
+  using S = std::decay_t<decltype(src[0] + 0)>;
   const int total = m * n;
   if (total <= 0) return;
   // element e = i + j m of thread t is t + kBlock u: the row and column step by
@@ -135,9 +158,9 @@ __device__ inline void stage_in(D* dst, int ldd, const S* src, long si, long sj,
     }
   }
 }
-template <typename D, typename S, int kS = kStage>
-__device__ inline void stage_in(D* dst, int ldd, const S* src, long si, long sj, int m, int n) {
-  stage_in<D, S, kS>(dst, ldd, src, si, sj, m, n, m, n);
+template <typename PD, typename PS, int kS = kStage>
+__device__ inline void stage_in(PD dst, int ldd, PS src, long si, long sj, int m, int n) {
+  stage_in<PD, PS, kS>(dst, ldd, src, si, sj, m, n, m, n);
 }
 
 // ---- reductions -------------------------------------------------------------
@@ -190,6 +213,15 @@ __device__ inline T wave_sum(T v) {
   v += dpp_swap<0x141>(v);
   v += dpp_swap<0x140>(v);
   return (lane_read(v, 0) + lane_read(v, 16)) + (lane_read(v, 32) + lane_read(v, 48));
+}
+
+// Largest of v over the wavefront, in every lane.
+__device__ inline double wave_max(double v) {
+  v = fmax(v, dpp_swap<0xB1>(v));
+  v = fmax(v, dpp_swap<0x4E>(v));
+  v = fmax(v, dpp_swap<0x141>(v));
+  v = fmax(v, dpp_swap<0x140>(v));
+  return fmax(fmax(lane_read(v, 0), lane_read(v, 16)), fmax(lane_read(v, 32), lane_read(v, 48)));
 }
 
 // Sum over the whole workgroup (blockDim.x == kBlock).  All threads get the result.

@@ -45,7 +45,8 @@ __device__ inline int group_lanes(int items, int lanes) {
 }
 
 // sum_{i = i0, i0+g, ... < m} x[i] y[i]; four loads in flight per operand.
-__device__ inline double strided_dot(const double* x, const double* y, int i0, int m, int g) {
+template <typename PX, typename PY>
+__device__ inline double strided_dot(PX x, PY y, int i0, int m, int g) {
   double s0 = 0.0, s1 = 0.0;
   int i = i0;
   for (; i + 3 * g < m; i += 4 * g) {
@@ -61,7 +62,8 @@ __device__ inline double strided_dot(const double* x, const double* y, int i0, i
 }
 
 // y[i] -= f x[i] for i = i0, i0+g, ... < m (x and y distinct columns).
-__device__ inline void strided_axpy(double* y, double f, const double* x, int i0, int m, int g) {
+template <typename PY, typename PX>
+__device__ inline void strided_axpy(PY y, double f, PX x, int i0, int m, int g) {
   int i = i0;
   for (; i + 3 * g < m; i += 4 * g) {
     const double x0 = x[i], x1 = x[i + g], x2 = x[i + 2 * g], x3 = x[i + 3 * g];
@@ -77,7 +79,7 @@ __device__ inline void strided_axpy(double* y, double f, const double* x, int i0
 // Sum over the whole team; every thread gets the same value.  'red' holds
 // kWaves doubles (workgroup team only).
 template <int kLanes>
-__device__ inline double team_sum(double v, double* red) {
+__device__ inline double team_sum(double v, lptr<double> red) {
   v = wave_sum(v);
   if constexpr (kLanes == kWave) {
     return v;
@@ -98,16 +100,16 @@ __device__ inline double team_sum(double v, double* red) {
 // On exit R is in the upper triangle, v_j below the diagonal, tau[j] set.
 // The whole team forms each reflector (norm, scaling); trailing column c
 // belongs to lane group c mod (kLanes / g), which applies the reflector to it.
-template <int kLanes>
-__device__ inline void team_house_qr(double* A, int lda, int m, int k, double* tau) {
+template <int kLanes, typename PA, typename PT>
+__device__ inline void team_house_qr(PA A, int lda, int m, int k, PT tau) {
   __shared__ double red[kWaves];
   const int tid = team_tid<kLanes>();
   const int steps = m < k ? m : k;
   const int g = group_lanes(k, kLanes), ngrp = kLanes / g, grp = tid / g, sub = tid % g;
   for (int j = 0; j < steps; ++j) {
-    double* v = A + (size_t)j * lda;
+    const PA v = A + (size_t)j * lda;
     double s = strided_dot(v, v, j + 1 + tid, m, kLanes);
-    s = team_sum<kLanes>(s, red);
+    s = team_sum<kLanes>(s, (lptr<double>)red);
     const double alpha = v[j];
     double t = 0.0, beta = alpha;
     if (s != 0.0) {
@@ -125,7 +127,7 @@ __device__ inline void team_house_qr(double* A, int lda, int m, int k, double* t
     if (t != 0.0) {
       int c = j + 1 + ((grp - (j + 1) % ngrp) + ngrp) % ngrp;
       for (; c < k; c += ngrp) {
-        double* a = A + (size_t)c * lda;
+        const PA a = A + (size_t)c * lda;
         double d = strided_dot(v, a, j + 1 + sub, m, g);
         d = group_sum(d, g) + a[j];
         const double f = t * d;
@@ -150,7 +152,7 @@ __device__ inline void team_house_qr(double* A, int lda, int m, int k, double* t
 constexpr int kQrRows = 8;
 
 template <int kLanes, int kC>
-__device__ inline void team_sum_n(double (&v)[kC], double* red) {
+__device__ inline void team_sum_n(double (&v)[kC], lptr<double> red) {
 #pragma unroll
   for (int c = 0; c < kC; ++c) v[c] = wave_sum(v[c]);
   if constexpr (kLanes != kWave) {
@@ -172,13 +174,15 @@ __device__ inline void team_sum_n(double (&v)[kC], double* red) {
   }
 }
 
-// Element type of a panel known to be in global memory: loads and stores then
-// use a uniform base and 32-bit offsets instead of 64-bit flat addresses.
-typedef __attribute__((address_space(1))) double gdouble;
-
-template <int kLanes, int R, typename E = double>
-__device__ inline void team_house_qr_rows(E* A, int lda, int m, int k, double* tau) {
+// (one array for all instantiations in a kernel; wavefronts use their own part)
+__device__ inline lptr<double> qr_red() {
   __shared__ double red[4 * kWaves];
+  return (lptr<double>)red;
+}
+
+template <int kLanes, int R, typename PA, typename PT>
+__device__ inline void team_house_qr_rows(PA A, int lda, int m, int k, PT tau) {
+  const lptr<double> red = qr_red();
   const int tid = team_tid<kLanes>();
   const int steps = m < k ? m : k;
   // rows of this thread; loads use a clamped row and a select instead of a
@@ -190,7 +194,7 @@ __device__ inline void team_house_qr_rows(E* A, int lda, int m, int k, double* t
     rc[r] = row[r] < m ? row[r] : m - 1;
   }
   for (int j = 0; j < steps; ++j) {
-    E* vcol = A + (size_t)j * lda;
+    const PA vcol = A + (size_t)j * lda;
     double v[R];
     double s1[1] = {0.0};
 #pragma unroll
@@ -226,7 +230,7 @@ __device__ inline void team_house_qr_rows(E* A, int lda, int m, int k, double* t
 #pragma unroll
         for (int c = 0; c < 4; ++c) {
           const int cc = c0 + c < k ? c0 + c : k - 1;
-          const E* ac = A + (size_t)cc * lda;
+          const PA ac = A + (size_t)cc * lda;
           aj[c] = ac[j];  // read by all before thread 0 rewrites it
 #pragma unroll
           for (int r = 0; r < R; ++r) a[c][r] = ac[rc[r]];
@@ -242,7 +246,7 @@ __device__ inline void team_house_qr_rows(E* A, int lda, int m, int k, double* t
 #pragma unroll
         for (int c = 0; c < 4; ++c) {
           if (c0 + c >= k) continue;
-          E* ac = A + (size_t)(c0 + c) * lda;
+          const PA ac = A + (size_t)(c0 + c) * lda;
           const double f = t * (d[c] + aj[c]);
 #pragma unroll
           for (int r = 0; r < R; ++r)
@@ -260,8 +264,8 @@ __device__ inline void team_house_qr_rows(E* A, int lda, int m, int k, double* t
 
 // Picks the rows-per-thread count for m (m <= kQrRows * kLanes for a
 // wavefront, 2 * kQrRows * kLanes for larger teams).
-template <int kLanes>
-__device__ inline void team_house_qr_rows(double* A, int lda, int m, int k, double* tau) {
+template <int kLanes, typename PA, typename PT>
+__device__ inline void team_house_qr_any_rows(PA A, int lda, int m, int k, PT tau) {
   if (m <= 2 * kLanes)
     team_house_qr_rows<kLanes, 2>(A, lda, m, k, tau);
   else if (m <= 4 * kLanes)
@@ -272,29 +276,16 @@ __device__ inline void team_house_qr_rows(double* A, int lda, int m, int k, doub
     team_house_qr_rows<kLanes, 2 * kQrRows>(A, lda, m, k, tau);
 }
 
-// The rows QR of a panel in global memory (m <= 16 kLanes).
-template <int kLanes>
-__device__ inline void team_house_qr_rows_global(double* A, int lda, int m, int k, double* tau) {
-  gdouble* G = (gdouble*)A;
-  if (m <= 2 * kLanes)
-    team_house_qr_rows<kLanes, 2, gdouble>(G, lda, m, k, tau);
-  else if (m <= 4 * kLanes)
-    team_house_qr_rows<kLanes, 4, gdouble>(G, lda, m, k, tau);
-  else if (m <= 8 * kLanes)
-    team_house_qr_rows<kLanes, kQrRows, gdouble>(G, lda, m, k, tau);
-  else
-    team_house_qr_rows<kLanes, 2 * kQrRows, gdouble>(G, lda, m, k, tau);
-}
-
 // Householder QR of two global panels at once, one per half of the
 // workgroup (rows <= 16 * 128 each, k columns each, k <= min(m, n)).  Both
 // halves take the same k steps, so their workgroup barriers pair up.
-__device__ inline void house_qr_pair(double* A, int lda, int m, double* tau_a, double* B, int ldb, int n,
-                                     double* tau_b, int k) {
+template <typename PT>
+__device__ inline void house_qr_pair(gptr<double> A, int lda, int m, PT tau_a, gptr<double> B, int ldb, int n,
+                                     PT tau_b, int k) {
   if (threadIdx.x < kBlock / 2)
-    team_house_qr_rows_global<kBlock / 2>(A, lda, m, k, tau_a);
+    team_house_qr_any_rows<kBlock / 2>(A, lda, m, k, tau_a);
   else
-    team_house_qr_rows_global<kBlock / 2>(B, ldb, n, k, tau_b);
+    team_house_qr_any_rows<kBlock / 2>(B, ldb, n, k, tau_b);
   __syncthreads();
 }
 
@@ -325,8 +316,8 @@ __device__ inline void team_apply_q(const double* V, int ldv, int m, int nref, c
 // T of team_larft from the strict upper triangle of S = V^T V: T[j, j] = tau_j,
 // T[l, j] = -tau_j sum_{r=l}^{j-1} T[l, r] S[r, j].  The recurrence runs on
 // the team's first wavefront; row l of T is written by lane l mod 64 only.
-template <int kLanes>
-__device__ inline void larft_recurrence(int k, const double* tau, const double* S, double* T) {
+template <int kLanes, typename PT>
+__device__ inline void larft_recurrence(int k, PT tau, PT S, PT T) {
   const int tid = team_tid<kLanes>();
   if (tid < kWave) {
     for (int j = 0; j < k; ++j) {
@@ -348,9 +339,8 @@ __device__ inline void larft_recurrence(int k, const double* tau, const double* 
 // T[l, j] = -tau_j sum_{r=l}^{j-1} T[l, r] S[r, j], T[j, j] = tau_j.
 // The recurrence runs on the team's first wavefront; row l of T is written
 // by lane l mod 64 only, so its steps need no cross-lane exchange.
-template <int kLanes>
-__device__ inline void team_larft(const double* V, int ldv, int m, int k, const double* tau,
-                                  double* S, double* T) {
+template <int kLanes, typename PV, typename PT>
+__device__ inline void team_larft(PV V, int ldv, int m, int k, PT tau, PT S, PT T) {
   const int tid = team_tid<kLanes>();
   const int npairs = k * (k - 1) / 2;
   if (npairs > 0) {
@@ -360,8 +350,8 @@ __device__ inline void team_larft(const double* V, int ldv, int m, int k, const 
       while (j * (j - 1) / 2 > p) --j;
       while ((j + 1) * j / 2 <= p) ++j;
       const int l = p - j * (j - 1) / 2;
-      const double* vl = V + (size_t)l * ldv;
-      const double* vj = V + (size_t)j * ldv;
+      const PV vl = V + (size_t)l * ldv;
+      const PV vj = V + (size_t)j * ldv;
       double d = strided_dot(vl, vj, j + 1 + sub, m, g);
       d = group_sum(d, g) + vl[j];
       if (sub == 0) S[l + (size_t)j * k] = d;
@@ -371,11 +361,11 @@ __device__ inline void team_larft(const double* V, int ldv, int m, int k, const 
   larft_recurrence<kLanes>(k, tau, S, T);
 }
 
-// Workgroup-wide wrappers (the workgroup's own reduction scratch is unused).
-__device__ inline void house_qr(double* A, int lda, int m, int k, double* tau, double* = nullptr,
-                                double* = nullptr) {
+// Workgroup-wide wrappers.
+template <typename PA, typename PT>
+__device__ inline void house_qr(PA A, int lda, int m, int k, PT tau) {
   if (m <= 2 * kQrRows * kBlock)
-    team_house_qr_rows<kBlock>(A, lda, m, k, tau);
+    team_house_qr_any_rows<kBlock>(A, lda, m, k, tau);
   else
     team_house_qr<kBlock>(A, lda, m, k, tau);
 }
@@ -383,16 +373,13 @@ __device__ inline void apply_q(const double* V, int ldv, int m, int nref, const 
                                double* Y, int ldy, int r, double* = nullptr, double* = nullptr) {
   team_apply_q<kBlock>(V, ldv, m, nref, tau, Y, ldy, r);
 }
-// Single-wavefront versions (operands in LDS).
-__device__ inline void wave_house_qr(double* A, int lda, int m, int k, double* tau) {
+// Single-wavefront version.
+template <typename PA, typename PT>
+__device__ inline void wave_house_qr(PA A, int lda, int m, int k, PT tau) {
   if (m <= kQrRows * kWave)
-    team_house_qr_rows<kWave>(A, lda, m, k, tau);
+    team_house_qr_any_rows<kWave>(A, lda, m, k, tau);
   else
     team_house_qr<kWave>(A, lda, m, k, tau);
-}
-__device__ inline void wave_apply_q(const double* V, int ldv, int m, int nref, const double* tau,
-                                    double* Y, int ldy, int r) {
-  team_apply_q<kWave>(V, ldv, m, nref, tau, Y, ldy, r);
 }
 
 constexpr int kJacobiMaxCols = 256;  // columns whose norms the Jacobi keeps in scratch
@@ -434,9 +421,9 @@ __device__ inline void jacobi_rot(double a, double b, double c2, double& t, doub
   s = y * t;
 }
 
-template <int kLanes>
-__device__ inline int team_jacobi(double* G, int ldg, int rows, int cols, double* V, int ldv,
-                                  double* sh2, double* nrm, int max_sweeps, double tol2 = 1e-26) {
+template <int kLanes, typename PG>
+__device__ inline int team_jacobi(PG G, int ldg, int rows, int cols, PG V, int ldv,
+                                  lptr<double> sh2, lptr<double> nrm, int max_sweeps, double tol2 = 1e-26) {
   const int tid = team_tid<kLanes>();
   if (V != nullptr)
     for (int e = tid; e < cols * cols; e += kLanes) {
@@ -475,7 +462,7 @@ __device__ inline int team_jacobi(double* G, int ldg, int rows, int cols, double
         const double x = G[e % rows + (size_t)(e / rows) * ldg];
         f += x * x;
       }
-      f = team_sum<kLanes>(f, sh2 ? sh2 + 2 : nullptr);
+      f = team_sum<kLanes>(f, sh2 ? sh2 + 2 : lptr<double>(nullptr));
     }
     const double floor2 = 1e-30 * f;
     int rotated = 0;
@@ -497,8 +484,8 @@ __device__ inline int team_jacobi(double* G, int ldg, int rows, int cols, double
           q = tmp;
         }
         if (q >= cols) continue;
-        double* gp = G + (size_t)p * ldg;
-        double* gq = G + (size_t)q * ldg;
+        const PG gp = G + (size_t)p * ldg;
+        const PG gq = G + (size_t)q * ldg;
         double c2 = 0.0, a, b;
         if (track) {
           c2 = group_sum(strided_dot(gp, gq, sub, rows, g), g);
@@ -526,8 +513,8 @@ __device__ inline int team_jacobi(double* G, int ldg, int rows, int cols, double
           gq[i] = s * x + c * y;
         }
         if (V != nullptr) {
-          double* vp = V + (size_t)p * ldv;
-          double* vq = V + (size_t)q * ldv;
+          const PG vp = V + (size_t)p * ldv;
+          const PG vq = V + (size_t)q * ldv;
           for (int i = sub; i < cols; i += g) {
             const double x = vp[i], y = vq[i];
             vp[i] = c * x - s * y;
@@ -579,9 +566,9 @@ __device__ inline double group_sum_c(double v) {
 // Requires rows (and cols when kV) <= R kG, kG == group_lanes(pairs, kLanes)
 // and tracked norms; floor_rel as 1e-30 in team_jacobi.  Without V (kV false) the caller recovers the right
 // singular vectors from the input, as G_in^T U.
-template <int kLanes, int R, int kG, bool kV>
-__device__ inline int team_jacobi_rows(double* G, int ldg, int rows, int cols, double* V, int ldv,
-                                       double* sh2, double* nrm, int max_sweeps, double tol2 = 1e-26,
+template <int kLanes, int R, int kG, bool kV, typename PG>
+__device__ inline int team_jacobi_rows(PG G, int ldg, int rows, int cols, PG V, int ldv,
+                                       lptr<double> sh2, lptr<double> nrm, int max_sweeps, double tol2 = 1e-26,
                                        double floor_rel = 1e-30) {
   const int tid = team_tid<kLanes>();
   if constexpr (kV) {
@@ -640,8 +627,8 @@ __device__ inline int team_jacobi_rows(double* G, int ldg, int rows, int cols, d
           q = tmp;
         }
         if (q >= cols) continue;
-        double* gp = G + (size_t)p * ldg;
-        double* gq = G + (size_t)q * ldg;
+        const PG gp = G + (size_t)p * ldg;
+        const PG gq = G + (size_t)q * ldg;
         // all loads of the pair issued before the first wait
         double xp[R], xq[R], up[R], uq[R];
 #pragma unroll
@@ -650,8 +637,8 @@ __device__ inline int team_jacobi_rows(double* G, int ldg, int rows, int cols, d
           xq[r] = gq[rgc[r]];
         }
         if constexpr (kV) {
-          const double* vp = V + (size_t)p * ldv;
-          const double* vq = V + (size_t)q * ldv;
+          const PG vp = V + (size_t)p * ldv;
+          const PG vq = V + (size_t)q * ldv;
 #pragma unroll
           for (int r = 0; r < R; ++r) {
             up[r] = vp[rvc[r]];
@@ -674,8 +661,8 @@ __device__ inline int team_jacobi_rows(double* G, int ldg, int rows, int cols, d
           }
         }
         if constexpr (kV) {
-          double* vp = V + (size_t)p * ldv;
-          double* vq = V + (size_t)q * ldv;
+          const PG vp = V + (size_t)p * ldv;
+          const PG vq = V + (size_t)q * ldv;
 #pragma unroll
           for (int r = 0; r < R; ++r) {
             if (rg[r] < cols) {
@@ -714,9 +701,9 @@ __device__ inline int team_jacobi_rows(double* G, int ldg, int rows, int cols, d
 
 // Dispatch on the group size and rows per lane; V == nullptr skips the
 // accumulation of V.  Shapes outside the instantiated ones use team_jacobi.
-template <int kLanes, bool kV>
-__device__ inline int team_jacobi_sel(double* G, int ldg, int rows, int cols, double* V, int ldv,
-                                      double* sh2, double* nrm, int max_sweeps, double tol2 = 1e-26) {
+template <int kLanes, bool kV, typename PG>
+__device__ inline int team_jacobi_sel(PG G, int ldg, int rows, int cols, PG V, int ldv,
+                                      lptr<double> sh2, lptr<double> nrm, int max_sweeps, double tol2 = 1e-26) {
   const int half = ((cols + 1) & ~1) / 2;
   const int g = group_lanes(half, kLanes);
   const int span = kV ? (rows > cols ? rows : cols) : rows;
@@ -724,22 +711,15 @@ __device__ inline int team_jacobi_sel(double* G, int ldg, int rows, int cols, do
 #define HMX_JR(G_, R_)                                                                             \
   if (g == G_ && need <= R_)                                                                       \
     return team_jacobi_rows<kLanes, R_, G_, kV>(G, ldg, rows, cols, V, ldv, sh2, nrm, max_sweeps, tol2);
-  if constexpr (kLanes == kWave) {
-    HMX_JR(16, 1)
-    HMX_JR(8, 2)
-    HMX_JR(4, 6)
-    HMX_JR(4, 8)
-  } else {
-    HMX_JR(16, 2)
-    HMX_JR(8, 8)
-  }
+  HMX_JR(16, 2)
+  HMX_JR(8, 8)
 #undef HMX_JR
   return team_jacobi<kLanes>(G, ldg, rows, cols, V, ldv, sh2, nrm, max_sweeps, tol2);
 }
 
-template <int kLanes>
-__device__ inline int team_jacobi_any(double* G, int ldg, int rows, int cols, double* V, int ldv,
-                                      double* sh2, double* nrm, int max_sweeps, double tol2 = 1e-26) {
+template <int kLanes, typename PG>
+__device__ inline int team_jacobi_any(PG G, int ldg, int rows, int cols, PG V, int ldv,
+                                      lptr<double> sh2, lptr<double> nrm, int max_sweeps, double tol2 = 1e-26) {
   if (nrm != nullptr && cols <= kJacobiMaxCols && cols >= 2 && rows >= 1) {
     if (V != nullptr)
       return team_jacobi_sel<kLanes, true>(G, ldg, rows, cols, V, ldv, sh2, nrm, max_sweeps, tol2);
@@ -748,30 +728,174 @@ __device__ inline int team_jacobi_any(double* G, int ldg, int rows, int cols, do
   return team_jacobi<kLanes>(G, ldg, rows, cols, V, ldv, sh2, nrm, max_sweeps, tol2);
 }
 
-// Workgroup version used by the existing call sites (cols <= kJacobiMaxCols);
-// V == nullptr leaves V out.
-__device__ inline void jacobi_svd(double* G, int ldg, int rows, int cols, double* V, int ldv,
-                                  int* /*flag*/, int max_sweeps = 40, double tol2 = 1e-26) {
-  __shared__ double sh2[2 + kWaves];
+// The norms of the workgroup's Jacobi: one array for every instantiation.
+__device__ inline lptr<double> jacobi_norms() {
   __shared__ double nrm[kJacobiMaxCols];
-  team_jacobi_any<kBlock>(G, ldg, rows, cols, V, ldv, sh2, nrm, max_sweeps, tol2);
+  return (lptr<double>)nrm;
 }
 
-// Single-wavefront version (G, V in LDS; cols <= kJacobiMaxCols); V == nullptr
-// leaves V out.
-__device__ inline int wave_jacobi_svd(double* G, int ldg, int rows, int cols, double* V, int ldv,
-                                      int max_sweeps = 40, double tol2 = 1e-26) {
-  __shared__ double nrm[kJacobiMaxCols];
-  return team_jacobi_any<kWave>(G, ldg, rows, cols, V, ldv, nullptr, nrm, max_sweeps, tol2);
+// Workgroup version used by the existing call sites (cols <= kJacobiMaxCols);
+// V == nullptr leaves V out.
+template <typename PG>
+__device__ inline void jacobi_svd(PG G, int ldg, int rows, int cols, PG V, int ldv,
+                                  int* /*flag*/, int max_sweeps = 40, double tol2 = 1e-26) {
+  __shared__ double sh2[2 + kWaves];
+  team_jacobi_any<kBlock>(G, ldg, rows, cols, V, ldv, (lptr<double>)sh2, jacobi_norms(), max_sweeps, tol2);
+}
+
+// ---------------------------------------------------------------------------
+// Core SVD of the recompressions: G (rows x cols, both at most kCoreMax) on one
+// wavefront.  A one-sided Jacobi on the core itself took 7 to 14 sweeps of
+// rounds whose index arithmetic, masks and branches cost 2,000 cycles each (88 us
+// for 13 columns, the larger part of a recompression: an average launch of FADD
+// went from 166 to 147 us in a 40,000-point FP32 Cholesky and from 137 to 110 us
+// in a 6,000-point FP64 LU, RKRK from 53 to 41 and from 41 to 34 us).  Here:
+//  1. Pivoted Gram-Schmidt of the rows of G in registers (lane c holds row c):
+//     G = W Q^T, the columns of W graded, their number the numerical rank (cut at
+//     1e-15 of the norm, the level below which the Jacobi rotates nothing).
+//  2. Jacobi on the columns of W, which being graded needs about half the
+//     sweeps, in a tournament whose columns move between fixed slots: every lane
+//     reads and writes the same LDS addresses in every round, rows are padded
+//     with zeros, a pair below the threshold gets the identity rotation, and the
+//     norms come from the registers.
+// On exit the first r columns of G hold sigma_j u_j; returns r.
+// Bound: the instructions of one wavefront (about 100 per round).
+// ---------------------------------------------------------------------------
+constexpr int kCoreMax = 32;
+
+__device__ inline lptr<double> core_buffer() {
+  __shared__ double w[kCoreMax * (kCoreMax + 1)];
+  return (lptr<double>)w;
+}
+
+// kG lanes per pair, kR rows per lane (rows <= kG kR), cols <= 128 / kG; W has
+// cols rounded up to even columns, ld rows >= kG kR, zero outside the matrix.
+template <int kG, int kR>
+__device__ inline void slot_jacobi(lptr<double> W, int ld, int cols, double tol2, double floor_rel) {
+  const int lane = threadIdx.x & (kWave - 1);
+  const int h = (cols + 1) / 2, rounds = 2 * h - 1;
+  const int i = lane / kG, sub = lane % kG;
+  const bool act = i < h;
+  const int ic = act ? i : 0;
+  // slots: top column i of pair i, bottom column h + i.  The top of pair 0 stays,
+  // the others move up through the tops and back through the bottoms.
+  const int top_to = ic == 0 ? 0 : (ic < h - 1 ? ic + 1 : 2 * h - 1);
+  const int bot_to = ic == 0 ? (h > 1 ? 1 : h) : h + ic - 1;
+  const lptr<double> xt = W + ic * ld + sub, xb = W + (h + ic) * ld + sub;
+  const lptr<double> yt = W + top_to * ld + sub, yb = W + bot_to * ld + sub;
+  double floor2 = 0.0;
+  for (int sweep = 0; sweep < 40; ++sweep) {
+    bool rotated = false;
+    for (int rd = 0; rd < rounds; ++rd) {
+      double x[kR], y[kR];
+#pragma unroll
+      for (int r = 0; r < kR; ++r) {
+        x[r] = xt[kG * r];
+        y[r] = xb[kG * r];
+      }
+      double a = 0.0, b = 0.0, c2 = 0.0;
+#pragma unroll
+      for (int r = 0; r < kR; ++r) {
+        a += x[r] * x[r];
+        b += y[r] * y[r];
+        c2 += x[r] * y[r];
+      }
+      a = group_sum_c<kG>(a);
+      b = group_sum_c<kG>(b);
+      c2 = group_sum_c<kG>(c2);
+      if (sweep == 0 && rd == 0) floor2 = floor_rel * wave_sum(act && sub == 0 ? a + b : 0.0);
+      const bool turn = c2 * c2 > tol2 * a * b && fabs(c2) > floor2;
+      double t, c, s;
+      jacobi_rot(a, b, c2, t, c, s);
+      c = turn ? c : 1.0;
+      s = turn ? s : 0.0;
+      rotated |= turn && act;
+      __builtin_amdgcn_wave_barrier();
+      if (act) {
+#pragma unroll
+        for (int r = 0; r < kR; ++r) {
+          yt[kG * r] = c * x[r] - s * y[r];
+          yb[kG * r] = s * x[r] + c * y[r];
+        }
+      }
+      __builtin_amdgcn_wave_barrier();
+    }
+    if (__ballot(rotated) == 0) break;
+  }
+}
+
+template <int kN>
+__device__ inline int core_rows(lptr<double> G, int ldg, int rows, int cols, lptr<double> W, int ld) {
+  const int lane = threadIdx.x & (kWave - 1);
+  const int lc = lane < rows ? lane : rows - 1;
+  double g[kN];
+  double n2 = 0.0;
+#pragma unroll
+  for (int r = 0; r < kN; ++r) {
+    const double v = G[lc + (r < cols ? r : cols - 1) * ldg];
+    g[r] = (lane < rows && r < cols) ? v : 0.0;
+    n2 += g[r] * g[r];
+  }
+  const double total = wave_sum(n2);
+  if (!(total < __builtin_inf())) {  // infinities and NaN go on as NaN
+    if (lane < ld) W[lane] = __builtin_nan("");
+    return 1;
+  }
+  const double stop = 1e-30 * total;
+  const int most = rows < cols ? rows : cols;
+  int s = 0;
+  for (; s < most; ++s) {
+    const double m = wave_max(n2);
+    if (!(m > stop)) break;
+    const int p = __builtin_ctzll(__ballot(n2 == m));
+    const double inv = 1.0 / sqrt(m);
+    double q[kN], d = 0.0;
+#pragma unroll
+    for (int r = 0; r < kN; ++r) {
+      q[r] = lane_read(g[r], p) * inv;
+      d += q[r] * g[r];
+    }
+    if (lane < ld) W[lane + s * ld] = d;
+    n2 = 0.0;
+#pragma unroll
+    for (int r = 0; r < kN; ++r) {
+      g[r] = lane == p ? 0.0 : g[r] - d * q[r];  // what is left of the pivot is rounding
+      n2 += g[r] * g[r];
+    }
+  }
+  if ((s & 1) && lane < ld) W[lane + s * ld] = 0.0;
+  return s;
+}
+
+// (one wavefront; rows, cols <= kCoreMax)
+__device__ inline int wave_core_svd(lptr<double> G, int ldg, int rows, int cols, double tol2, double floor_rel) {
+  const lptr<double> W = core_buffer();
+  const int lane = threadIdx.x & (kWave - 1);
+  int r;
+  int ld = 17;  // odd: the columns' rows spread over the banks
+  if (rows <= 16) {
+    r = cols <= 16 ? core_rows<16>(G, ldg, rows, cols, W, ld) : core_rows<32>(G, ldg, rows, cols, W, ld);
+    __builtin_amdgcn_wave_barrier();
+    if (r > 1) slot_jacobi<8, 2>(W, ld, r, tol2, floor_rel);
+  } else {
+    ld = 33;
+    r = cols <= 24 ? core_rows<24>(G, ldg, rows, cols, W, ld) : core_rows<32>(G, ldg, rows, cols, W, ld);
+    __builtin_amdgcn_wave_barrier();
+    if (r > 1) slot_jacobi<4, 8>(W, ld, r, tol2, floor_rel);
+  }
+  __builtin_amdgcn_wave_barrier();
+  for (int e = lane; e < rows * r; e += kWave) G[e % rows + e / rows * ldg] = W[e % rows + e / rows * ld];
+  __builtin_amdgcn_wave_barrier();
+  return r;
 }
 
 // Column norms of G into sig[0..cols), then order[] = permutation sorting
 // sig descending (ties by index).  Returns nothing; ends with a barrier.
-__device__ inline void sorted_norms(const double* G, int ldg, int rows, int cols, double* sig,
-                                    int* order) {
+template <typename PG, typename PS, typename PI>
+__device__ inline void sorted_norms(PG G, int ldg, int rows, int cols, PS sig, PI order) {
   const int lane = threadIdx.x & (kWave - 1), w = threadIdx.x / kWave;
   for (int j = w; j < cols; j += kWaves) {
-    const double* g = G + (size_t)j * ldg;
+    const PG g = G + (size_t)j * ldg;
     double s = 0.0;
     for (int i = lane; i < rows; i += kWave) s += g[i] * g[i];
     s = wave_sum(s);
@@ -794,7 +918,8 @@ __device__ inline void sorted_norms(const double* G, int ldg, int rows, int cols
 
 // findK scalar_array.cpp:98-116: number of sigma (descending) with
 // sigma[i] > eps * sigma[0].
-__device__ inline int find_k(const double* sig, const int* order, int n, double eps) {
+template <typename PS, typename PI>
+__device__ inline int find_k(PS sig, PI order, int n, double eps) {
   if (n == 0) return 0;
   const double thr = sig[order[0]] * eps;
   int k = 0;

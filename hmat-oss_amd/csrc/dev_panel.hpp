@@ -14,7 +14,8 @@ typedef double hmx_double4 __attribute__((ext_vector_type(4)));
 
 // Entry (r, c) of the unit lower trapezoidal reflector matrix stored in V
 // (m x K, ld ldv: reflector entries below the diagonal), zero outside.
-__device__ inline double refl_entry(const double* V, int ldv, int m, int K, int r, int c) {
+template <typename PV>
+__device__ inline double refl_entry(PV V, int ldv, int m, int K, int r, int c) {
   const int rc = r < m ? r : m - 1, cc = c < K ? c : K - 1;
   const double x = V[rc + (size_t)cc * ldv];
   return (r >= m || c >= K) ? 0.0 : (r > c ? x : (r == c ? 1.0 : 0.0));
@@ -27,8 +28,8 @@ __device__ inline double refl_entry(const double* V, int ldv, int m, int K, int 
 // j + 16 (i mod 4), element i / 4.  The four wavefronts take interleaved
 // slabs; their tiles go through 'part' (4 * kNb (kNb + 1) / 2 * 256
 // doubles of LDS) and are summed in a fixed order.
-template <int kNb>
-__device__ void wg_reflector_gram(const double* V, int ldv, int m, int K, double* S, double* part) {
+template <int kNb, typename PV, typename PT>
+__device__ void wg_reflector_gram(PV V, int ldv, int m, int K, PT S, lptr<double> part) {
   constexpr int kTiles = kNb * (kNb + 1) / 2;
   const int lane = threadIdx.x & (kWave - 1), w = threadIdx.x / kWave;
   const int kk = lane >> 4, ii = lane & 15;
@@ -77,7 +78,8 @@ __host__ __device__ constexpr int gram_part(int K) {
   return 4 * (((K + 15) / 16) * ((K + 15) / 16 + 1) / 2) * 256;
 }
 
-__device__ inline void wg_reflector_gram_any(const double* V, int ldv, int m, int K, double* S, double* part) {
+template <typename PV, typename PT>
+__device__ inline void wg_reflector_gram_any(PV V, int ldv, int m, int K, PT S, lptr<double> part) {
   switch ((K + 15) / 16) {
     case 1: wg_reflector_gram<1>(V, ldv, m, K, S, part); break;
     case 2: wg_reflector_gram<2>(V, ldv, m, K, S, part); break;
@@ -91,13 +93,13 @@ __device__ inline void wg_reflector_gram_any(const double* V, int ldv, int m, in
 namespace hmx {
 
 // G = X^T Y (kx x ky; G[i + j ldg], or G[j + i ldg] when 'trans') for X
-// (p x kx, ld ldx) and Y (p x ky, ld ldy) of element type T, on the matrix
+// (p x kx, ld ldx) and Y (p x ky, ld ldy), pointers PX, on the matrix
 // cores as wg_reflector_gram: 16-column blocks of X are the A operand, of Y
 // the B operand, tile (a, b) accumulates over 4-row slabs, the wavefronts'
 // tiles meet in 'part' (4 kNa kNb 256 doubles of LDS).
-template <typename T, int kNa, int kNb>
-__device__ void wg_xty(const T* X, int ldx, int kx, const T* Y, int ldy, int ky, int p, double* G, int ldg,
-                       bool trans, double* part) {
+template <int kNa, int kNb, typename PX, typename PG>
+__device__ void wg_xty(PX X, int ldx, int kx, PX Y, int ldy, int ky, int p, PG G, int ldg,
+                       bool trans, lptr<double> part) {
   constexpr int kTiles = kNa * kNb;
   const int lane = threadIdx.x & (kWave - 1), w = threadIdx.x / kWave;
   const int kk = lane >> 4, ii = lane & 15;
@@ -153,14 +155,14 @@ __device__ void wg_xty(const T* X, int ldx, int kx, const T* Y, int ldy, int ky,
 __host__ __device__ constexpr int xty_part(int kx, int ky) { return 4 * ((kx + 15) / 16) * ((ky + 15) / 16) * 256; }
 
 // kx, ky <= 32; returns false (nothing done) otherwise.
-template <typename T>
-__device__ inline bool wg_xty_any(const T* X, int ldx, int kx, const T* Y, int ldy, int ky, int p, double* G,
-                                  int ldg, bool trans, double* part) {
+template <typename PX, typename PG>
+__device__ inline bool wg_xty_any(PX X, int ldx, int kx, PX Y, int ldy, int ky, int p, PG G,
+                                  int ldg, bool trans, lptr<double> part) {
   const int na = (kx + 15) / 16, nb = (ky + 15) / 16;
-  if (na == 1 && nb == 1) wg_xty<T, 1, 1>(X, ldx, kx, Y, ldy, ky, p, G, ldg, trans, part);
-  else if (na == 1 && nb == 2) wg_xty<T, 1, 2>(X, ldx, kx, Y, ldy, ky, p, G, ldg, trans, part);
-  else if (na == 2 && nb == 1) wg_xty<T, 2, 1>(X, ldx, kx, Y, ldy, ky, p, G, ldg, trans, part);
-  else if (na == 2 && nb == 2) wg_xty<T, 2, 2>(X, ldx, kx, Y, ldy, ky, p, G, ldg, trans, part);
+  if (na == 1 && nb == 1) wg_xty<1, 1>(X, ldx, kx, Y, ldy, ky, p, G, ldg, trans, part);
+  else if (na == 1 && nb == 2) wg_xty<1, 2>(X, ldx, kx, Y, ldy, ky, p, G, ldg, trans, part);
+  else if (na == 2 && nb == 1) wg_xty<2, 1>(X, ldx, kx, Y, ldy, ky, p, G, ldg, trans, part);
+  else if (na == 2 && nb == 2) wg_xty<2, 2>(X, ldx, kx, Y, ldy, ky, p, G, ldg, trans, part);
   else return false;
   return true;
 }
@@ -168,19 +170,19 @@ __device__ inline bool wg_xty_any(const T* X, int ldx, int kx, const T* Y, int l
 // out (rows x nk, ld ldo) = M (rows x k, ld ldm) C (k x nk, ld ldc; LDS or
 // global): each thread owns rows and streams a row of M once per eight
 // output columns.
-template <typename T, typename TO = T>
-__device__ void rows_times_small(const T* M, int ldm, int rows, int k, const double* C, int ldc, int nk, TO* out,
+template <typename TO, typename PM, typename PC, typename PO>
+__device__ void rows_times_small(PM M, int ldm, int rows, int k, PC C, int ldc, int nk, PO out,
                                  int ldo) {
   constexpr int kC = 8;
   for (int c0 = 0; c0 < nk; c0 += kC) {
-    const double* cc[kC];
+    PC cc[kC];
 #pragma unroll
     for (int b = 0; b < kC; ++b) cc[b] = C + (size_t)(c0 + b < nk ? c0 + b : nk - 1) * ldc;
     for (int i = threadIdx.x; i < rows; i += kBlock) {
       double acc[kC];
 #pragma unroll
       for (int b = 0; b < kC; ++b) acc[b] = 0.0;
-      const T* mi = M + i;
+      const PM mi = M + i;
       int l = 0;
       for (; l + 8 <= k; l += 8) {
         double v[8];

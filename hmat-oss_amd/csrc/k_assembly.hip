@@ -45,15 +45,6 @@ __global__ void __launch_bounds__(kBlock) k_table_full(const LeafDesc* desc, con
 
 constexpr int kSvdMax = 99;  // compressionMinLeafSize - 1
 
-// Largest of v over the wavefront, in every lane.
-__device__ inline double wave_max(double v) {
-  v = fmax(v, dpp_swap<0xB1>(v));
-  v = fmax(v, dpp_swap<0x4E>(v));
-  v = fmax(v, dpp_swap<0x141>(v));
-  v = fmax(v, dpp_swap<0x140>(v));
-  return fmax(fmax(lane_read(v, 0), lane_read(v, 16)), fmax(lane_read(v, 32), lane_read(v, 48)));
-}
-
 // Pivoted Gram-Schmidt of G (gr x gc, gc <= gr <= 2 kR, at W with ld gr) in
 // registers: threads 2 c and 2 c + 1 hold the two halves of column c.  Step
 // s takes the largest remaining column as the direction q, and row s of R,
@@ -178,13 +169,14 @@ __global__ void __launch_bounds__(kBlock, 2) k_svd_compress(const LeafDesc* desc
   const int r = gr <= 52 ? pivoted_rows<26>(gr, gc, tol, W, ldw) : pivoted_rows<50>(gr, gc, tol, W, ldw);
   // pairs whose inner product is below 1e-16 eps^2 ||G||^2 turn a kept column by
   // less than 1e-16
+  const lptr<double> w3 = (lptr<double>)W;
   const double floor_rel = fmax(1e-30, 1e-16 * eps * eps);
   if (r <= 32)
-    team_jacobi_rows<kBlock, 7, 16, false>(W, ldw, gc, r, nullptr, 0, sh2, sig, 40, 1e-26, floor_rel);
+    team_jacobi_rows<kBlock, 7, 16, false>(w3, ldw, gc, r, lptr<double>(nullptr), 0, (lptr<double>)sh2, (lptr<double>)sig, 40, 1e-26, floor_rel);
   else if (r <= 64)
-    team_jacobi_rows<kBlock, 13, 8, false>(W, ldw, gc, r, nullptr, 0, sh2, sig, 40, 1e-26, floor_rel);
+    team_jacobi_rows<kBlock, 13, 8, false>(w3, ldw, gc, r, lptr<double>(nullptr), 0, (lptr<double>)sh2, (lptr<double>)sig, 40, 1e-26, floor_rel);
   else
-    team_jacobi_rows<kBlock, 25, 4, false>(W, ldw, gc, r, nullptr, 0, sh2, sig, 40, 1e-26, floor_rel);
+    team_jacobi_rows<kBlock, 25, 4, false>(w3, ldw, gc, r, lptr<double>(nullptr), 0, (lptr<double>)sh2, (lptr<double>)sig, 40, 1e-26, floor_rel);
   sorted_norms(W, ldw, gc, r, sig, order);
   int k = find_k(sig, order, r, eps);
   if (k > d.cap) {
@@ -539,8 +531,9 @@ template <typename T>
 __device__ int truncate_panels(double* A, int m, double* B, int n, int k, const AcaWs& w,
                                double eps, T* outA, T* outB, int cap, int* overflow, double* red,
                                int* flag) {
-  house_qr(A, m, m, k, w.taua, red, w.sig);
-  house_qr(B, n, n, k, w.taub, red, w.sig);
+  const auto ga = (gptr<double>)A, gb = (gptr<double>)B;
+  house_qr(ga, m, m, k, (gptr<double>)w.taua);
+  house_qr(gb, n, n, k, (gptr<double>)w.taub);
   // g = Ra Rb^T (k x k), Ra, Rb upper triangular
   for (int e = threadIdx.x; e < k * k; e += kBlock) {
     const int i = e % k, j = e / k;
@@ -550,7 +543,7 @@ __device__ int truncate_panels(double* A, int m, double* B, int n, int k, const 
     w.g[i + (size_t)j * k] = s;
   }
   __syncthreads();
-  jacobi_svd(w.g, k, k, k, w.v, k, flag);
+  jacobi_svd((gptr<double>)w.g, k, k, k, (gptr<double>)w.v, k, flag);
   sorted_norms(w.g, k, k, k, w.sig, w.order);
   int nk = find_k(w.sig, w.order, k, eps);
   if (nk > cap) {

@@ -42,6 +42,15 @@ __device__ inline MfmaAcc<float>::type mfma16x16x4(float a, float b, MfmaAcc<flo
   return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
 }
 
+// f(0), ..., f(N - 1) with compile-time indices (register arrays)
+template <int I, int N, typename F>
+__device__ __forceinline__ void static_for(F f) {
+  if constexpr (I < N) {
+    f(std::integral_constant<int, I>{});
+    static_for<I + 1, N>(f);
+  }
+}
+
 // ---------------------------------------------------------------------------
 // GEMM: C (m x n, ldc) = beta C + alpha op(A) op(B), 64 x 64 tiles.
 // ---------------------------------------------------------------------------
@@ -58,9 +67,9 @@ __global__ void __launch_bounds__(256) k_gemm(const FTask* tasks, const GemmTile
   const int M = eff(t.m), N = eff(t.n), P = eff(t.p);
   const int i0 = tl.tm * TM, j0 = tl.tn * TN;
   if (i0 >= M || j0 >= N) return;
-  const T* A = (const T*)t.A;
-  const T* B = (const T*)t.B;
-  T* C = (T*)t.C;
+  const auto A = (cgptr<T>)t.A;
+  const auto B = (cgptr<T>)t.B;
+  const auto C = (gptr<T>)t.C;
   // wavefront w computes the 32 x 32 quadrant (w & 1, w >> 1) of the tile as
   // 2 x 2 matrix-core tiles of 16 x 16: A[i][k] comes from lane i + 16 k,
   // B[k][j] from lane j + 16 k (inner dimension 4 per instruction)
@@ -128,7 +137,7 @@ __global__ void __launch_bounds__(256) k_gemm(const FTask* tasks, const GemmTile
       for (int v = 0; v < 4; ++v) {
         const int i = i0 + qi + 16 * a + MfmaAcc<T>::row(lane, v), j = j0 + qj + 16 * b + li;
         if (i >= M || j >= N) continue;
-        T* pc = C + i + (size_t)j * t.ldc;
+        const auto pc = C + i + (size_t)j * t.ldc;
         *pc = t.mode ? *pc + alpha * acc[a][b][v] : alpha * acc[a][b][v];
       }
 }
@@ -195,21 +204,206 @@ __device__ void potrf_body(T* L, int ld, int n, int* info) {
   }
 }
 
+// Reciprocal, quotient and square root for the serial chains of the leaf
+// factorisations: hardware estimates with Newton / Goldschmidt steps and
+// Markstein's final corrections (P. Markstein, IBM J. Res. Dev. 34, 1990), a
+// power of two taken out first.  About a third of the dependent steps of the
+// library forms.
+__device__ inline double chain_rcp(double d) {
+  const int e = __builtin_amdgcn_frexp_exp(d);
+  const double s = __builtin_amdgcn_ldexp(d, -e);
+  double y = __builtin_amdgcn_rcp(s);
+  y = fma(fma(-s, y, 1.0), y, y);
+  y = fma(fma(-s, y, 1.0), y, y);
+  return fabs(d) <= 1.79e308 ? __builtin_amdgcn_ldexp(y, -e) : 1.0 / d;
+}
+// a / d with y = 1 / d: the product corrected by its remainder (a == d gives 1)
+__device__ inline double chain_div(double a, double d, double y) {
+  const double q = a * y;
+  return fabs(d) <= 1.79e308 ? fma(fma(-q, d, a), y, q) : q;
+}
+// sqrt(d)
+__device__ inline double chain_sqrt(double d) {
+  const int e = __builtin_amdgcn_frexp_exp(d) & ~1;
+  const double s = __builtin_amdgcn_ldexp(d, -e);
+  const double y = __builtin_amdgcn_rsq(s);
+  double g = s * y, h = 0.5 * y;
+  double r = fma(-h, g, 0.5);
+  g = fma(g, r, g);
+  h = fma(h, r, h);
+  r = fma(-h, g, 0.5);
+  g = fma(g, r, g);
+  h = fma(h, r, h);
+  g = fma(fma(-g, g, s), h, g);
+  return (d > 0.0 && d <= 1.79e308) ? __builtin_amdgcn_ldexp(g, e >> 1) : d;
+}
+
+// The 16 x 16 tiles t = w, w + 4, ... < count of a trailing update by 16
+// columns, four at a time so that their LDS reads and products overlap:
+// tile(t, x0, y0) gives the tile's offsets, A(i, k) and B(k, j) the operands'
+// entries, and the block itself (ld ld, n x n) is the accumulator.
+template <typename FT, typename FA, typename FB>
+__device__ inline void panel_update(double* P, int ld, int n, int count, FT tile, FA A, FB B) {
+  constexpr int kBatch = 4;
+  const int lane = threadIdx.x & (kWave - 1), w = threadIdx.x / kWave, ii = lane & 15, kk = lane >> 4;
+  for (int t0 = w; t0 < count; t0 += kBatch * kWaves) {
+    int x0[kBatch], y0[kBatch];
+    double a[kBatch][4], b[kBatch][4];
+    hmx_double4 acc[kBatch];
+#pragma unroll
+    for (int u = 0; u < kBatch; ++u) {
+      const int t = t0 + u * kWaves;
+      tile(t < count ? t : t0, x0[u], y0[u]);
+      const int xr = x0[u] + ii < n ? x0[u] + ii : n - 1, yc = y0[u] + ii < n ? y0[u] + ii : n - 1;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        a[u][q] = -A(xr, 4 * q + kk);
+        b[u][q] = B(4 * q + kk, yc);
+        const int i = x0[u] + kk + 4 * q;
+        acc[u][q] = P[(i < n ? i : n - 1) + yc * ld];
+      }
+    }
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+#pragma unroll
+      for (int u = 0; u < kBatch; ++u) acc[u] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[u][q], b[u][q], acc[u], 0, 0, 0);
+#pragma unroll
+    for (int u = 0; u < kBatch; ++u)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        const int i = x0[u] + kk + 4 * v, j = y0[u] + ii;
+        if (t0 + u * kWaves < count && i < n && j < n) P[i + j * ld] = acc[u][v];
+      }
+  }
+}
+
+// n x n (n <= 128) between global memory (ld lda) and LDS (ld n): a wavefront
+// per column, no index divisions, 16 columns' loads in flight.
+template <typename T>
+__device__ inline void leaf_in(double* L, cgptr<T> A, int lda, int n) {
+  const int lane = threadIdx.x & (kWave - 1), w = threadIdx.x / kWave;
+  constexpr int kC = 16;
+  const int i1 = lane < n ? lane : n - 1, i2 = lane + kWave < n ? lane + kWave : n - 1;
+  for (int j0 = w; j0 < n; j0 += kC * kWaves) {
+    T v[kC][2];
+#pragma unroll
+    for (int c = 0; c < kC; ++c) {
+      const int j = j0 + kWaves * c < n ? j0 + kWaves * c : n - 1;
+      v[c][0] = A[(size_t)j * lda + i1];
+      v[c][1] = A[(size_t)j * lda + i2];
+    }
+#pragma unroll
+    for (int c = 0; c < kC; ++c) {
+      const int j = j0 + kWaves * c;
+      if (j >= n) continue;
+      if (lane < n) L[j * n + lane] = (double)v[c][0];
+      if (lane + kWave < n) L[j * n + lane + kWave] = (double)v[c][1];
+    }
+  }
+}
+template <typename T>
+__device__ inline void leaf_out(gptr<T> A, int lda, const double* L, int n, bool lower) {
+  const int lane = threadIdx.x & (kWave - 1), w = threadIdx.x / kWave;
+#pragma unroll 4
+  for (int j = w; j < n; j += kWaves)
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const int i = lane + kWave * h;
+      if (i < n) A[(size_t)j * lda + i] = (lower && i < j) ? (T)0 : (T)L[j * n + i];
+    }
+}
+
+// Blocked Cholesky of a leaf of at most 128 rows in LDS (FP64).  Per 16
+// columns: the diagonal block on one wavefront with a row per lane in registers
+// (the other lanes' entries by readlane: no LDS round trip and no barrier in its
+// 16 steps), in the square-root-free form, so that a step's chain is one
+// reciprocal, the roots being taken for all 16 columns at once; the rows below
+// by one thread each with the block's multipliers; the trailing lower triangle
+// on the matrix cores.  Bound: the chain of reciprocals and rank-1 steps of the
+// diagonal blocks.  125 rows: 244 us (FP64) and 167 us (FP32 storage) with a column
+// per step of the whole workgroup, 90 us now.
+__device__ void potrf_lds(double* L, int ld, int n, int* info) {
+  __shared__ double mult[kNb * kNb];  // a_cj / d_j at c + 16 j
+  __shared__ double root[kNb], rroot[kNb];
+  const int lane = threadIdx.x & (kWave - 1), w = threadIdx.x / kWave, i = lane & 15;
+  for (int r0 = 0; r0 < n; r0 += kNb) {
+    const int bs = n - r0 < kNb ? n - r0 : kNb;
+    if (w == 0) {
+      double a[kNb];
+      const int ir = r0 + (i < bs ? i : bs - 1);
+#pragma unroll
+      for (int c = 0; c < kNb; ++c) {
+        const double v = L[ir + (r0 + (c < bs ? c : bs - 1)) * ld];
+        a[c] = (i < bs && c < bs) ? v : (i == c ? 1.0 : 0.0);
+      }
+      bool bad = false;
+      double diag = 1.0;
+      static_for<0, kNb>([&](auto J) __attribute__((always_inline)) {
+        constexpr int j = decltype(J)::value;
+        const double d = lane_read(a[j], j);
+        bad |= !(d > 0.0);
+        diag = i == j ? a[j] : diag;
+        const double m = a[j] * chain_rcp(d);
+        if (lane < kNb) mult[i + kNb * j] = m;
+#pragma unroll
+        for (int c = j + 1; c < kNb; ++c) a[c] -= m * lane_read(a[j], c);
+      });
+      if (bad && lane == 0) atomicOr(info, 1);
+      const double p = chain_sqrt(diag), y = chain_rcp(p);
+      if (lane < kNb) {
+        root[i] = p;
+        rroot[i] = y;
+      }
+#pragma unroll
+      for (int c = 0; c < kNb; ++c) {
+        const double pc = lane_read(p, c), l = i == c ? pc : chain_div(a[c], pc, lane_read(y, c));
+        if (lane < bs && c <= i) L[r0 + i + (r0 + c) * ld] = l;
+      }
+    }
+    __syncthreads();
+    const int below = n - r0 - kNb;
+    if (below <= 0) break;
+    if ((int)threadIdx.x < below) {
+      double* row = L + r0 + kNb + threadIdx.x + r0 * ld;
+      double x[kNb];
+#pragma unroll
+      for (int c = 0; c < kNb; ++c) x[c] = row[c * ld];
+      static_for<0, kNb>([&](auto J) __attribute__((always_inline)) {
+        constexpr int j = decltype(J)::value;
+#pragma unroll
+        for (int c = j + 1; c < kNb; ++c) x[c] -= x[j] * mult[c + kNb * j];
+      });
+#pragma unroll
+      for (int c = 0; c < kNb; ++c) row[c * ld] = chain_div(x[c], root[c], rroot[c]);
+    }
+    __syncthreads();
+    const int nt = (below + kNb - 1) / kNb;
+    panel_update(
+        L, ld, n, nt * (nt + 1) / 2,
+        [&](int t, int& x0, int& y0) {
+          int tj = 0;
+          while (t >= nt - tj) t -= nt - tj++;
+          x0 = r0 + kNb * (tj + t + 1);
+          y0 = r0 + kNb * (tj + 1);
+        },
+        [&](int r, int k) { return L[r + (r0 + k) * ld]; }, [&](int k, int c) { return L[c + (r0 + k) * ld]; });
+    __syncthreads();
+  }
+}
+
 template <typename T>
 __global__ void __launch_bounds__(kBlock) k_potrf(const FTask* tasks, int* info) {
-  __shared__ T lds[kLdsDense * kLdsDense];
+  __shared__ double lds[kLdsDense * kLdsDense];
   const FTask& t = tasks[blockIdx.x];
   const int n = t.m.s;
   T* A = (T*)t.A;
   const int lda = t.lda;
   if (n <= kLdsDense) {
-    stage_in(lds, n, A, 1L, (long)lda, n, n);
+    leaf_in<T>(lds, (cgptr<T>)A, lda, n);
     __syncthreads();
-    potrf_body(lds, n, n, info);
-    for (int e = threadIdx.x; e < n * n; e += kBlock) {
-      const int i = e % n, j = e / n;
-      A[i + (size_t)j * lda] = (i >= j) ? lds[i + j * n] : (T)0;
-    }
+    potrf_lds(lds, n, n, info);
+    __syncthreads();
+    leaf_out<T>((gptr<T>)A, lda, lds, n, true);
   } else {
     potrf_body(A, lda, n, info);
     for (int e = threadIdx.x; e < n * n; e += kBlock) {
@@ -258,7 +452,7 @@ __global__ void __launch_bounds__(kBlock) k_ldlt(const FTask* tasks, int* info) 
   T* D = (T*)t.B;
   const int lda = t.lda;
   if (n <= kLdsDense) {
-    stage_in(lds, n, A, 1L, (long)lda, n, n);
+    stage_in(lds, n, (cgptr<T>)A, 1L, (long)lda, n, n);
     __syncthreads();
     ldlt_body(lds, n, n, dl, info);
     for (int e = threadIdx.x; e < n * n; e += kBlock) {
@@ -285,9 +479,9 @@ __global__ void k_dscale(const FTask* tasks, const int* fail) {
   if (*fail) return;
   const FTask& t = tasks[blockIdx.x / kDscaleSplit];
   const int part = blockIdx.x % kDscaleSplit;
-  const T* A = (const T*)t.A;
-  const T* d = (const T*)t.B;
-  T* C = (T*)t.C;
+  const auto A = (cgptr<T>)t.A;
+  const auto d = (cgptr<T>)t.B;
+  const auto C = (gptr<T>)t.C;
   const int m = eff(t.m), n = eff(t.n);
   const bool cols = t.mode & kDscaleCols, inv = t.mode & kDscaleInv;
   const int64_t total = (int64_t)m * n;
@@ -360,20 +554,171 @@ __device__ void getrf_body(T* P, int ld, int n, int* piv, int* info) {
   }
 }
 
+// Blocked LU of a leaf of at most 128 rows in LDS (FP64), the same pivots.  Per
+// 16 columns: the panel on one wavefront with two rows per lane in registers;
+// rows stay where they are and carry their position (the interchanges move
+// positions), the pivot row reaches the others by readlane, so a step has no
+// barrier.  Then the interchanges on the other columns and the 16 rows of U by
+// one thread per column, and the trailing block on the matrix cores.  Bound:
+// the chain of pivot searches and divisions.  94 rows in FP64: 231 us with a
+// column per step of the whole workgroup, 127 us now.
+__device__ void getrf_lds(double* P, int ld, int n, int* piv, int* info) {
+  __shared__ int swap[kNb];
+  __shared__ int from[2 * kWave];  // the row that the panel's interchanges bring to a position
+  __shared__ int stop;
+  const int lane = threadIdx.x & (kWave - 1), w = threadIdx.x / kWave;
+  if (threadIdx.x == 0) stop = 0;
+  __syncthreads();
+  for (int r0 = 0; r0 < n; r0 += kNb) {
+    const int bs = n - r0 < kNb ? n - r0 : kNb, rows = n - r0;
+    if (w == 0) {
+      // rows r0 + lane + 64 h, columns r0 .. r0 + bs
+      double a[2][kNb];
+      int pos[2];
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        pos[h] = lane + kWave * h;
+        const int r = r0 + (pos[h] < rows ? pos[h] : rows - 1);
+#pragma unroll
+        for (int c = 0; c < kNb; ++c) a[h][c] = P[r + (r0 + (c < bs ? c : bs - 1)) * ld];
+      }
+      bool fail = false;
+      static_for<0, kNb>([&](auto J) __attribute__((always_inline)) {
+        constexpr int j = decltype(J)::value;
+        if (j >= bs || fail) return;
+        // largest |a_ij| among the rows at positions >= j, the first of equals
+        double v[2];
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          const bool in = pos[h] >= j && pos[h] < rows;
+          const double x = fabs(a[h][j]);
+          v[h] = (in && x == x) ? x : -1.0;
+        }
+        double m = v[0] > v[1] ? v[0] : v[1];
+        m = fmax(m, dpp_swap<0xB1>(m));
+        m = fmax(m, dpp_swap<0x4E>(m));
+        m = fmax(m, dpp_swap<0x141>(m));
+        m = fmax(m, dpp_swap<0x140>(m));
+        m = fmax(fmax(lane_read(m, 0), lane_read(m, 16)), fmax(lane_read(m, 32), lane_read(m, 48)));
+        int pp = 0x7fffffff;  // its position
+        uint64_t at0 = __ballot(m >= 0.0 && v[0] == m), at1 = __ballot(m >= 0.0 && v[1] == m);
+        if (__popcll(at0) + __popcll(at1) == 1) {
+          pp = at0 ? __builtin_amdgcn_readlane(pos[0], __builtin_ctzll(at0))
+                   : __builtin_amdgcn_readlane(pos[1], __builtin_ctzll(at1));
+        } else {
+          for (uint64_t b = at0; b; b &= b - 1) pp = min(pp, __builtin_amdgcn_readlane(pos[0], __builtin_ctzll(b)));
+          for (uint64_t b = at1; b; b &= b - 1) pp = min(pp, __builtin_amdgcn_readlane(pos[1], __builtin_ctzll(b)));
+          if (pp == 0x7fffffff) pp = j;  // a column of NaNs: the pivot test below fails
+        }
+        // the lane and half that hold position pp
+        const uint64_t w0 = __ballot(pos[0] == pp), w1 = __ballot(pos[1] == pp);
+        const bool second = w0 == 0;
+        const int src = __builtin_ctzll(second ? w1 : w0);
+        double u[kNb];
+#pragma unroll
+        for (int c = j; c < kNb; ++c) u[c] = second ? lane_read(a[1][c], src) : lane_read(a[0][c], src);
+        if (lane == 0) swap[j] = pp;
+        const double d = u[j];
+        if (d == 0.0 || !isfinite(d)) {
+          fail = true;
+          return;
+        }
+        // a quotient and not a product with 1 / d: the multiplier of a row equal to
+        // the pivot's is then exactly 1, and a singular leaf ends on an exact zero
+        const double y = chain_rcp(d);
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          // interchange of the positions j and pp
+          pos[h] = pos[h] == pp ? j : (pos[h] == j ? pp : pos[h]);
+          if (pos[h] > j) {
+            const double l = chain_div(a[h][j], d, y);
+            a[h][j] = l;
+#pragma unroll
+            for (int c = j + 1; c < kNb; ++c) a[h][c] -= l * u[c];
+          }
+        }
+      });
+      if (fail) {
+        if (lane == 0) {
+          atomicOr(info, 1);
+          stop = 1;
+        }
+      } else {
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+          if (lane + kWave * h < rows)
+#pragma unroll
+            for (int c = 0; c < kNb; ++c)
+              if (c < bs) P[r0 + pos[h] + (r0 + c) * ld] = a[h][c];
+        if (lane < bs) piv[r0 + lane] = r0 + swap[lane];
+        from[pos[0]] = lane;
+        from[pos[1]] = lane + kWave;
+      }
+    }
+    __syncthreads();
+    if (stop) return;
+    // the interchanges on the other columns; right of the panel also
+    // U12 = L11^{-1} A12
+    const int c = threadIdx.x;
+    if (c < n && (c < r0 || c >= r0 + bs)) {
+      double* col = P + c * ld + r0;
+      // the rows that move are those at positions j < 16 and swap[j]: all loads
+      // first, then the stores (equal positions get equal values)
+      double x[kNb], z[kNb];
+      int at[kNb];
+#pragma unroll
+      for (int j = 0; j < kNb; ++j) {
+        at[j] = swap[j < bs ? j : bs - 1];
+        x[j] = col[from[j < bs ? j : bs - 1]];
+        z[j] = col[from[at[j]]];
+      }
+#pragma unroll
+      for (int j = 0; j < kNb; ++j) {
+        col[at[j]] = z[j];
+        if (j < bs) col[j] = x[j];
+      }
+      if (c >= r0 + bs) {
+        // (bs == 16 here)
+        const double* blk = P + r0 + r0 * ld;
+        static_for<1, kNb>([&](auto J) __attribute__((always_inline)) {
+          constexpr int j = decltype(J)::value;
+#pragma unroll
+          for (int l = 0; l < j; ++l) x[j] -= blk[j + l * ld] * x[l];
+          col[j] = x[j];
+        });
+      }
+    }
+    __syncthreads();
+    const int rest = n - r0 - kNb;
+    if (rest <= 0) break;
+    const int nt = (rest + kNb - 1) / kNb;
+    // an entry takes its 16 terms one after the other, as in the panel and in U:
+    // a row that equals an earlier pivot's ends on exact zeros here too
+    panel_update(
+        P, ld, n, nt * nt,
+        [&](int t, int& x0, int& y0) {
+          x0 = r0 + kNb * (t % nt + 1);
+          y0 = r0 + kNb * (t / nt + 1);
+        },
+        [&](int r, int k) { return P[r + (r0 + k) * ld]; }, [&](int k, int c) { return P[r0 + k + c * ld]; });
+    __syncthreads();
+  }
+}
+
 template <typename T>
 __global__ void __launch_bounds__(kBlock) k_getrf(const FTask* tasks, int* info) {
-  __shared__ T lds[kLdsDense * kLdsDense];
+  __shared__ double lds[kLdsDense * kLdsDense];
   const FTask& t = tasks[blockIdx.x];
   const int n = t.m.s;
   T* A = (T*)t.A;
   const int lda = t.lda;
   int* piv = (int*)t.B;
   if (n <= kLdsDense) {
-    stage_in(lds, n, A, 1L, (long)lda, n, n);
+    leaf_in<T>(lds, (cgptr<T>)A, lda, n);
     __syncthreads();
-    getrf_body(lds, n, n, piv, info);
+    getrf_lds(lds, n, n, piv, info);
     __syncthreads();
-    for (int e = threadIdx.x; e < n * n; e += kBlock) A[e % n + (size_t)(e / n) * lda] = lds[e];
+    leaf_out<T>((gptr<T>)A, lda, lds, n, false);
   } else {
     getrf_body(A, lda, n, piv, info);
   }
@@ -515,7 +860,7 @@ __global__ void __launch_bounds__(kBlock) k_hodlr(const FTask* tasks, double* ws
 // Rows (mode 0) / columns (modes 1, 2) of X are independent: a task is cut
 // into tiles of kTrsmCols of them, one workgroup each.
 // ---------------------------------------------------------------------------
-constexpr int kShDoubles = 19456;  // 152 KiB of LDS per workgroup
+constexpr int kShDoubles = 18432;  // 144 KiB of LDS per workgroup, beside the core SVD's buffer
 
 // A wavefront solves 16 independent rows / columns of X on its own: X^T (mode
 // 0) or X is cut into 16 x 16 blocks that stay in registers in the layout in
@@ -537,15 +882,6 @@ constexpr int kShDoubles = 19456;  // 152 KiB of LDS per workgroup
 // skipped zero half of the inverses.
 constexpr int kTrsmBlocks = 8;              // blocks solved in registers at a time
 constexpr int kTrsmInvLd = kNb * kNb + 8;   // diagonal blocks in LDS: spread over the banks
-
-// f(0), ..., f(N - 1) with compile-time indices (register arrays)
-template <int I, int N, typename F>
-__device__ __forceinline__ void static_for(F f) {
-  if constexpr (I < N) {
-    f(std::integral_constant<int, I>{});
-    static_for<I + 1, N>(f);
-  }
-}
 
 // row p of the s-th pair (p, c), c < p, in row order
 constexpr int trsm_pair_row(int s) {
@@ -569,8 +905,8 @@ __global__ void __launch_bounds__(kBlock) k_trsm(const FTask* tasks, const GemmT
   const int mode = t.mode & kTrsmBase;
   const bool transa = (t.mode & kTrsmTransA) != 0, unit = (t.mode & kTrsmUnit) != 0;
   const bool back = mode == 2, pivot = (t.mode & kTrsmPiv) && mode != 0;
-  const T* Lg = (const T*)t.A;
-  T* X = (T*)t.C;
+  const auto Lg = (cgptr<T>)t.A;
+  const auto X = (gptr<T>)t.C;
   const long li = transa ? (long)t.lda : 1L, lk = transa ? 1L : (long)t.lda;  // strides of L(i, k)
   const long ai = back ? lk : li, ak = back ? li : lk;  // of the operand: L, or L^T in mode 2
   const int lane = threadIdx.x & (kWave - 1), w = threadIdx.x / kWave;
@@ -580,11 +916,11 @@ __global__ void __launch_bounds__(kBlock) k_trsm(const FTask* tasks, const GemmT
   const int j = col0 + kNb * w + ii, jc = j < other ? j : other - 1;
   const bool mine = col0 + kNb * w < other;
   const long xr = mode == 0 ? (long)t.ldc : 1L;
-  T* Xc = X + (mode == 0 ? (size_t)jc : (size_t)jc * t.ldc);
+  const auto Xc = X + (mode == 0 ? (size_t)jc : (size_t)jc * t.ldc);
   const bool permuted = pivot && nb <= NB;
   if (permuted && w == 0) {
     // the interchanges as one permutation, rows lane + 64 q in registers
-    const int* piv = (const int*)t.B;
+    const auto piv = (cgptr<int>)t.B;
     constexpr int kQ = NB / 4;
     int pr[kQ], pv[kQ];
 #pragma unroll
@@ -616,9 +952,9 @@ __global__ void __launch_bounds__(kBlock) k_trsm(const FTask* tasks, const GemmT
     for (int q = 0; q < kQ; ++q) perm[lane + kWave * q] = pr[q];
   } else if (pivot && !permuted) {
     // wide leaves: each thread replays the interchanges on its own column
-    const int* piv = (const int*)t.B;
+    const auto piv = (cgptr<int>)t.B;
     if (threadIdx.x < kTrsmCols && col0 + (int)threadIdx.x < other) {
-      T* xc = X + (size_t)(col0 + threadIdx.x) * t.ldc;
+      const auto xc = X + (size_t)(col0 + threadIdx.x) * t.ldc;
       for (int i = 0; i < n; ++i) {
         int p = piv[i];
         p = p < 0 ? 0 : (p >= n ? n - 1 : p);
@@ -761,13 +1097,13 @@ __global__ void k_sumk(const FTask* tasks, const GemmTile* tiles, const int* fai
   const GemmTile tl = tiles[blockIdx.x];
   const FTask& t = tasks[tl.task];
   const int M = eff(t.m), N = eff(t.n), S = t.p.s;
-  const T* W = (const T*)t.A;
-  T* C = (T*)t.C;
+  const auto W = (cgptr<T>)t.A;
+  const auto C = (gptr<T>)t.C;
   const int64_t hi = std::min<int64_t>((int64_t)M * N, (int64_t)(tl.tm + 1) * kElemsPerTile);
   for (int64_t e = (int64_t)tl.tm * kElemsPerTile + threadIdx.x; e < hi; e += blockDim.x) {
     const int i = (int)(e % M), j = (int)(e / M);
-    T* pc = C + i + (size_t)j * t.ldc;
-    const T* w = W + i + (size_t)j * t.lda;
+    const auto pc = C + i + (size_t)j * t.ldc;
+    const auto w = W + i + (size_t)j * t.lda;
     double s = t.mode ? (double)*pc : 0.0;
 #pragma unroll 8
     for (int q = 0; q < S; ++q) s += (double)w[(size_t)q * t.ldb];
@@ -783,7 +1119,7 @@ __global__ void k_zero(const FTask* tasks, const GemmTile* tiles, const int* fai
   if (*fail) return;
   const GemmTile tl = tiles[blockIdx.x];
   const FTask& t = tasks[tl.task];
-  T* C = (T*)t.C;
+  const auto C = (gptr<T>)t.C;
   const int m = t.m.s, n = t.n.s;
   // mode 1: the identity
   const int64_t hi = std::min<int64_t>((int64_t)m * n, (int64_t)(tl.tm + 1) * kElemsPerTile);
@@ -798,8 +1134,8 @@ __global__ void k_axpy(const FTask* tasks, const GemmTile* tiles, const int* fai
   if (*fail) return;
   const GemmTile tl = tiles[blockIdx.x];
   const FTask& t = tasks[tl.task];
-  T* C = (T*)t.C;
-  const T* A = (const T*)t.A;
+  const auto C = (gptr<T>)t.C;
+  const auto A = (cgptr<T>)t.A;
   const int m = eff(t.m), n = eff(t.n);
   const T al = (T)t.alpha;
   const int64_t hi = std::min<int64_t>((int64_t)m * n, (int64_t)(tl.tm + 1) * kElemsPerTile);
@@ -820,9 +1156,12 @@ __global__ void k_axpy(const FTask* tasks, const GemmTile* tiles, const int* fai
 // block to compress; V, sig, order scratch (gc^2, gc, gc).  Truncated SVD at
 // eps into out (A = U sqrt(S) on the row side of D).
 template <typename T>
-__device__ int dense_to_rk(double* G, int gr, int gc, bool tr, double* V, double* sig, int* order,
+__device__ int dense_to_rk(double* G, bool in_lds, int gr, int gc, bool tr, double* V, double* sig, int* order,
                            double eps, RkRef out, int* overflow, int* flag) {
-  jacobi_svd(G, gr, gr, gc, V, gc, flag);
+  if (in_lds)
+    jacobi_svd((lptr<double>)G, gr, gr, gc, (lptr<double>)V, gc, flag);
+  else
+    jacobi_svd((gptr<double>)G, gr, gr, gc, (gptr<double>)V, gc, flag);
   sorted_norms(G, gr, gr, gc, sig, order);
   int k = find_k(sig, order, gc, eps);
   if (k > out.cap) {
@@ -852,31 +1191,32 @@ __device__ int dense_to_rk(double* G, int gr, int gc, bool tr, double* V, double
   return k;
 }
 
-// Widest core SVD done by one wavefront; wider cores use the workgroup (a
-// barrier per round, but a quarter of the rows per lane).
-constexpr int kWaveJacobiMax = 16;
-
 // Scratch of the QR recompression (all K x K blocks ld K).
+// (P double pointers, PI int pointers: LDS or global)
+template <typename P, typename PI>
 struct QrScratch {
-  double *taua, *taub;  // K each
-  double *g, *v;        // core SVD: G = Ra Rb^T -> U Sigma, and its V
-  double *ta, *tb;      // block-reflector factors of the two panels
-  double *x, *w;        // K x nk work blocks of the back-transformation
-  double *sig, *scale;  // K each
-  int* order;           // K
+  P taua, taub;  // K each
+  P g, v;        // core SVD: G = Ra Rb^T -> U Sigma, and its input
+  P ta, tb;      // block-reflector factors of the two panels
+  P x, w;        // K x nk work blocks of the back-transformation
+  P sig, scale;  // K each
+  PI order;      // K
 };
+using LdsScratch = QrScratch<lptr<double>, lptr<int>>;
+using GlobalScratch = QrScratch<gptr<double>, gptr<int>>;
 
 // doubles of the scratch above
 __device__ inline int64_t qr_core(int K) { return 6 * (int64_t)K * K + 5 * (int64_t)K; }
 
-__device__ inline QrScratch carve_qr(double* core, int K) {
+template <typename W, typename P>
+__device__ inline W carve_qr(P core, int K) {
   const size_t K2 = (size_t)K * K;
-  QrScratch w;
+  W w;
   w.taua = core;
   w.taub = core + K;
   w.sig = core + 2 * K;
   w.scale = core + 3 * K;
-  w.order = (int*)(core + 4 * K);
+  w.order = (decltype(w.order))(core + 4 * K);
   w.g = core + 5 * K;
   w.v = w.g + K2;
   w.ta = w.v + K2;
@@ -889,10 +1229,10 @@ __device__ inline QrScratch carve_qr(double* core, int K) {
 // Rows of one side of the formatted sum, concatenated: the target's panel
 // followed by every live part's panel placed at its row offset (zero
 // elsewhere); alpha_i scales the A side.  dst is rows x K, ld ld.
-template <typename T>
-__device__ void concat_side(double* dst, int ld, int rows, bool bside, const FTask& t, int kt) {
+template <typename T, typename PD>
+__device__ void concat_side(PD dst, int ld, int rows, bool bside, const FTask& t, int kt) {
   const RkRef& tg = t.tgt;
-  const T* src = (const T*)(bside ? tg.b : tg.a);
+  const auto src = (cgptr<T>)(bside ? tg.b : tg.a);
   const int lds = bside ? tg.lb : tg.la;
   stage_in(dst, ld, src, 1L, (long)lds, rows, kt);
   int off = kt;
@@ -900,13 +1240,13 @@ __device__ void concat_side(double* dst, int ld, int rows, bool bside, const FTa
     const Part& p = t.parts[q];
     const int kq = rank_of(p.rk);
     if (!(kq > 0 && p.alpha != 0.0 && p.rk.m > 0 && p.rk.n > 0)) continue;
-    const T* P = (const T*)(bside ? p.rk.b : p.rk.a);
+    const auto P = (cgptr<T>)(bside ? p.rk.b : p.rk.a);
     const int ldp = bside ? p.rk.lb : p.rk.la;
     const int o = bside ? p.coff : p.roff, pr = bside ? p.rk.n : p.rk.m;
     const double f = bside ? 1.0 : p.alpha;
     // the part covers rows [o, o + pr) of the target; zero elsewhere
     const int r_lo = o > 0 ? o : 0, r_hi = o + pr < rows ? o + pr : rows;
-    double* col0 = dst + (size_t)off * ld;
+    const PD col0 = dst + (size_t)off * ld;
     if (r_hi > r_lo)
       stage_in(col0 + r_lo, ld, P + (r_lo - o), 1L, (long)ldp, r_hi - r_lo, kq, r_hi - r_lo, kq, f);
     const int nz = rows - (r_hi > r_lo ? r_hi - r_lo : 0);
@@ -921,8 +1261,8 @@ __device__ void concat_side(double* dst, int ld, int rows, bool bside, const FTa
 }
 
 // G (K x K) = Ra Rb^T with Ra, Rb the upper triangles of two panels.
-__device__ inline void core_product(const double* Ra, int lra, const double* Rb, int lrb, int K,
-                                    double* G) {
+template <typename PA, typename PB, typename PG>
+__device__ inline void core_product(PA Ra, int lra, PB Rb, int lrb, int K, PG G) {
   for (int e = threadIdx.x; e < K * K; e += kBlock) {
     const int i = e % K, j = e / K;
     double s = 0.0;
@@ -937,9 +1277,9 @@ __device__ inline void core_product(const double* Ra, int lra, const double* Rb,
 // ld K): X = V1^T U, W = Tq X (K x nk, from the unit lower K x K top V1 of V
 // staged in w.w), then out = [U; 0] - V W with each thread owning rows and
 // streaming a row of V once per eight output columns.
-template <typename T>
-__device__ void wy_apply_out(const double* V, int ldv, int rows, int K, const double* Tq,
-                             const double* src, const QrScratch& w, int nk, T* out, int ldo) {
+template <typename T, typename PV, typename PS, typename W>
+__device__ void wy_apply_out(PV V, int ldv, int rows, int K, PS Tq, PS src, const W& w, int nk, gptr<T> out,
+                             int ldo) {
   for (int e = threadIdx.x; e < K * K; e += kBlock) {
     const int i = e % K, l = e / K;
     w.w[e] = i > l ? V[i + (size_t)l * ldv] : (i == l ? 1.0 : 0.0);
@@ -947,8 +1287,8 @@ __device__ void wy_apply_out(const double* V, int ldv, int rows, int K, const do
   __syncthreads();
   for (int e = threadIdx.x; e < K * nk; e += kBlock) {
     const int l = e % K, c = e / K;
-    const double* u = src + (size_t)w.order[c] * K;
-    const double* vl = w.w + (size_t)l * K;
+    const PS u = src + (size_t)w.order[c] * K;
+    const PS vl = w.w + (size_t)l * K;
     double s = 0.0;
     for (int i = l; i < K; ++i) s += vl[i] * u[i];
     w.x[l + (size_t)c * K] = s * w.scale[c];
@@ -963,7 +1303,7 @@ __device__ void wy_apply_out(const double* V, int ldv, int rows, int K, const do
   __syncthreads();
   constexpr int kC = 8;
   for (int c0 = 0; c0 < nk; c0 += kC) {
-    const double* wc[kC];
+    PS wc[kC];
 #pragma unroll
     for (int b = 0; b < kC; ++b) wc[b] = w.w + (size_t)(c0 + b < nk ? c0 + b : nk - 1) * K;
     // two rows per thread at a time (the second one kBlock further), so that
@@ -977,8 +1317,8 @@ __device__ void wy_apply_out(const double* V, int ldv, int rows, int K, const do
       for (int b = 0; b < kC; ++b) acc[0][b] = acc[1][b] = 0.0;
       // entries strictly below the unit diagonal: l < min(i, K)
       const int la = ia < K ? ia : K, lb = ib < K ? ib : K, lmax = la > lb ? la : lb;
-      const double* va = V + ia;
-      const double* vb = V + ib;
+      const PV va = V + ia;
+      const PV vb = V + ib;
       int l = 0;
       for (; l + 8 <= lmax; l += 8) {
         double xa[8], xb[8];
@@ -1024,39 +1364,53 @@ __device__ void wy_apply_out(const double* V, int ldv, int rows, int K, const do
 
 // After QR of both panels (reflectors Va, Vb, factors ta, tb) and G = Ra Rb^T
 // in w.g: SVD of G, cut at eps, write Qa U sqrt(S) and Qb V sqrt(S) to out.
-// stage: free LDS of kShDoubles doubles when the core lives in global memory
-// (nullptr otherwise): a core of at most kShDoubles entries is rotated there.
-template <typename T>
-__device__ void qr_finish(const double* Va, int lda, int m, const double* Vb, int ldb, int n, int K,
-                          const QrScratch& w, bool wave_core, double eps, RkRef out, int* overflow,
-                          int* flag, int* sweeps_out, double* stage = nullptr) {
-  __shared__ int sweeps;
+// stage: free LDS of kShDoubles doubles when the core lives in global memory:
+// a core of at most kShDoubles entries is rotated there.
+template <typename T, typename PV, typename P, typename PI>
+__device__ void qr_finish(PV Va, int lda, int m, PV Vb, int ldb, int n, int K, const QrScratch<P, PI>& w,
+                          double eps, RkRef out, int* overflow, int* flag, lptr<double> stage) {
+  constexpr bool kInLds = std::is_same_v<P, lptr<double>>;
+  __shared__ int core_rank;
+  int r = K;  // columns of the rotated core
   // one-sided Jacobi on G without V: G_in (kept in w.v) gives the right side
   // afterwards as G_in^T U, so the rounds only rotate G
   for (int e = threadIdx.x; e < K * K; e += kBlock) w.v[e] = w.g[e];
   __syncthreads();
-  if (stage != nullptr && K * K <= kShDoubles) {
+  if (K <= kCoreMax) {
+    // in LDS, a global core through its free part
+    lptr<double> g;
+    if constexpr (kInLds) {
+      g = w.g;
+    } else {
+      g = stage;
+      for (int e = threadIdx.x; e < K * K; e += kBlock) g[e] = w.g[e];
+      __syncthreads();
+    }
+    if (threadIdx.x < kWave) {
+      const int c = wave_core_svd(g, K, K, K, 1e-26, fmax(1e-30, 1e-16 * eps * eps));
+      if (threadIdx.x == 0) core_rank = c;
+    }
+    __syncthreads();
+    r = core_rank;
+    if constexpr (!kInLds) {
+      for (int e = threadIdx.x; e < K * r; e += kBlock) w.g[e] = g[e];
+      __syncthreads();
+    }
+  } else if constexpr (kInLds) {
+    jacobi_svd(w.g, K, K, K, P(nullptr), K, flag);
+  } else if (K * K <= kShDoubles) {
     // the rounds' loads and stores hit LDS instead of the L2
     for (int e = threadIdx.x; e < K * K; e += kBlock) stage[e] = w.g[e];
     __syncthreads();
-    jacobi_svd(stage, K, K, K, nullptr, K, flag);
+    jacobi_svd(stage, K, K, K, lptr<double>(nullptr), K, flag);
     for (int e = threadIdx.x; e < K * K; e += kBlock) w.g[e] = stage[e];
-    if (threadIdx.x == 0) sweeps = 0;
-    __syncthreads();
-  } else if (wave_core) {
-    if (threadIdx.x < kWave) {
-      const int sw = wave_jacobi_svd(w.g, K, K, K, nullptr, K);
-      if (threadIdx.x == 0) sweeps = sw;
-    }
     __syncthreads();
   } else {
-    jacobi_svd(w.g, K, K, K, nullptr, K, flag);
-    if (threadIdx.x == 0) sweeps = 0;
+    jacobi_svd(w.g, K, K, K, P(nullptr), K, flag);
     __syncthreads();
   }
-  if (sweeps_out) *sweeps_out = sweeps;
-  sorted_norms(w.g, K, K, K, w.sig, w.order);
-  int nk = find_k(w.sig, w.order, K, eps);
+  sorted_norms(w.g, K, K, r, w.sig, w.order);
+  int nk = find_k(w.sig, w.order, r, eps);
   if (nk > out.cap) {
     if (threadIdx.x == 0) atomicOr(overflow, 1);
     nk = out.cap;
@@ -1064,21 +1418,53 @@ __device__ void qr_finish(const double* Va, int lda, int m, const double* Vb, in
   // A = Qa U sqrt(S): column j of the rotated G is sigma_j u_j
   for (int c = threadIdx.x; c < nk; c += kBlock) w.scale[c] = 1.0 / sqrt(w.sig[w.order[c]]);
   __syncthreads();
-  wy_apply_out<T>(Va, lda, m, K, w.ta, w.g, w, nk, (T*)out.a, out.la);
+  wy_apply_out<T>(Va, lda, m, K, w.ta, w.g, w, nk, (gptr<T>)out.a, out.la);
   // B = Qb V sqrt(S) with v_j sigma_j = G_in^T u_j, u_j = g_j / sigma_j: column j
   // of w.ta (the A side's block factor is done) gets G_in^T u_j, and the same
   // scale 1 / sqrt(sigma_j) as the A side applies
   for (int e = threadIdx.x; e < K * nk; e += kBlock) {
     const int i = e % K, j = w.order[e / K];
-    const double* gi = w.v + (size_t)i * K;
-    const double* gj = w.g + (size_t)j * K;
+    const P gi = w.v + (size_t)i * K;
+    const P gj = w.g + (size_t)j * K;
     double s = 0.0;
     for (int l = 0; l < K; ++l) s += gi[l] * gj[l];
     w.ta[i + (size_t)j * K] = s / w.sig[j];
   }
   __syncthreads();
-  wy_apply_out<T>(Vb, ldb, n, K, w.tb, w.ta, w, nk, (T*)out.b, out.lb);
+  wy_apply_out<T>(Vb, ldb, n, K, w.tb, w.ta, w, nk, (gptr<T>)out.b, out.lb);
   if (threadIdx.x == 0) *out.rank = nk;
+}
+
+// QR form with both concatenated panels in global memory (Va m x K, Vb n x K);
+// part: part_size doubles of free LDS.
+template <typename T, typename W>
+__device__ void qr_global(gptr<double> Va, int m, gptr<double> Vb, int n, int K, const W& w, lptr<double> part,
+                          int64_t part_size, double eps, RkRef out, int* overflow, int* flag, lptr<double> stage) {
+  // V^T V of the global panels on the matrix cores when its LDS staging fits
+  const bool mfma_gram = K <= 64 && gram_part(K) <= part_size;
+  // both panels at once, one per half of the workgroup, when each has at
+  // most 16 rows per thread
+  const bool pair = m <= 16 * (kBlock / 2) && n <= 16 * (kBlock / 2);
+  if (pair)
+    house_qr_pair(Va, m, m, w.taua, Vb, n, n, w.taub, K);
+  else
+    house_qr(Va, m, m, K, w.taua);
+  if (mfma_gram) {
+    wg_reflector_gram_any(Va, m, m, K, w.x, part);
+    larft_recurrence<kBlock>(K, w.taua, w.x, w.ta);
+  } else {
+    team_larft<kBlock>(Va, m, m, K, w.taua, w.x, w.ta);
+  }
+  if (!pair) house_qr(Vb, n, n, K, w.taub);
+  if (mfma_gram) {
+    wg_reflector_gram_any(Vb, n, n, K, w.x, part);
+    larft_recurrence<kBlock>(K, w.taub, w.x, w.tb);
+  } else {
+    team_larft<kBlock>(Vb, n, n, K, w.taub, w.x, w.tb);
+  }
+  core_product(Va, m, Vb, n, K, w.g);
+  __syncthreads();
+  qr_finish<T>(Va, m, m, Vb, n, n, K, w, eps, out, overflow, flag, stage);
 }
 
 // ---------------------------------------------------------------------------
@@ -1096,13 +1482,14 @@ __device__ void qr_finish(const double* Va, int lda, int m, const double* Vb, in
 // about 1e-16 / 1e-13 = 1e-3, so the truncated product stays within eps.
 // ---------------------------------------------------------------------------
 constexpr int kGramMaxK = 32;
+static_assert(kGramMaxK <= kCoreMax, "the core SVD takes the whole core");
 constexpr double kGramTol = 1e-13;
 constexpr double kGramJacobiTol2 = 1e-16;
 
 // Pivoted Cholesky of G (K x K, ld K, symmetric, K <= 64) by one wavefront:
 // returns the rank r; rows 0..r-1 of the upper triangle hold R in the pivoted
 // column order, piv[0..K) the order.
-__device__ inline int wave_pchol(double* G, int K, int* piv) {
+__device__ inline int wave_pchol(lptr<double> G, int K, lptr<int> piv) {
   const int lane = threadIdx.x & (kWave - 1);
   if (lane < K) piv[lane] = lane;
   const double dmax = wave_argmax(ArgMax{lane < K ? G[lane + (size_t)lane * K] : -1.0, lane < K ? lane : -1}).v;
@@ -1153,30 +1540,28 @@ __device__ inline int wave_pchol(double* G, int K, int* piv) {
 __device__ inline int gram_lds(int K) { return 6 * K * K + 4 * K + xty_part(K, K); }
 
 template <typename T>
-__device__ void gram_recompress(const FTask& t, int kt, int K, double* gws, double* sh, double eps,
+__device__ void gram_recompress(const FTask& t, int kt, int K, double* gws, lptr<double> sh, double eps,
                                 int* overflow, int* flag) {
   __shared__ int ranks[2];
   const RkRef tg = t.tgt;
   const int m = tg.m, n = tg.n;
-  double* Va = gws;
-  double* Vb = gws + (size_t)m * K;
+  const auto Va = (gptr<double>)gws;
+  const auto Vb = Va + (size_t)m * K;
   concat_side<T>(Va, m, m, false, t, kt);
   concat_side<T>(Vb, n, n, true, t, kt);
   __syncthreads();
   const int K2 = K * K;
-  double* Ga = sh;
-  double* Gb = Ga + K2;
-  double* Cm = Gb + K2;
-  double* Cin = Cm + K2;
-  double* Ma = Cin + K2;
-  double* Mb = Ma + K2;
-  double* sig = Mb + K2;
-  int* order = (int*)(sig + K);
-  int* pa = order + K;
-  int* pb = pa + K;
-  double* part = sig + 4 * K;
-  wg_xty_any<double>(Va, m, K, Va, m, K, m, Ga, K, false, part);
-  wg_xty_any<double>(Vb, n, K, Vb, n, K, n, Gb, K, false, part);
+  const lptr<double> Ga = sh;
+  const lptr<double> Gb = Ga + K2;
+  const lptr<double> Cm = Gb + K2;
+  const lptr<double> Cin = Cm + K2;
+  const lptr<double> Ma = Cin + K2;
+  const lptr<double> Mb = Ma + K2;
+  const lptr<double> sig = Mb + K2;
+  const lptr<int> order = (lptr<int>)(sig + K), pa = order + K, pb = pa + K;
+  const lptr<double> part = sig + 4 * K;
+  wg_xty_any(Va, m, K, Va, m, K, m, Ga, K, false, part);
+  wg_xty_any(Vb, n, K, Vb, n, K, n, Gb, K, false, part);
   const int wid = threadIdx.x / kWave, lane = threadIdx.x & (kWave - 1);
   if (wid == 0) {
     const int r = wave_pchol(Ga, K, pa);
@@ -1214,14 +1599,14 @@ __device__ void gram_recompress(const FTask& t, int kt, int K, double* gws, doub
   __syncthreads();
   // columns orthogonal to 1e-8 of their norms: far below the FP32 data's
   // rounding once scaled by the eps cut
-  if (rb <= kWaveJacobiMax) {
-    if (wid == 0) wave_jacobi_svd(Cm, ra, ra, rb, nullptr, 0, 40, kGramJacobiTol2);
-    __syncthreads();
-  } else {
-    jacobi_svd(Cm, ra, ra, rb, nullptr, 0, flag, 40, kGramJacobiTol2);
+  if (wid == 0) {
+    const int c = wave_core_svd(Cm, ra, ra, rb, kGramJacobiTol2, fmax(1e-30, 1e-16 * eps * eps));
+    if (lane == 0) ranks[0] = c;
   }
-  sorted_norms(Cm, ra, ra, rb, sig, order);
-  int nk = find_k(sig, order, rb, eps);
+  __syncthreads();
+  const int rc = ranks[0];
+  sorted_norms(Cm, ra, ra, rc, sig, order);
+  int nk = find_k(sig, order, rc, eps);
   if (nk > tg.cap) {
     if (threadIdx.x == 0) atomicOr(overflow, 1);
     nk = tg.cap;
@@ -1244,8 +1629,7 @@ __device__ void gram_recompress(const FTask& t, int kt, int K, double* gws, doub
     const bool bside = threadIdx.x >= half;
     const int c = bside ? threadIdx.x - half : threadIdx.x;
     const int r = bside ? rb : ra;
-    const double* R = bside ? Gb : Ga;
-    double* X = bside ? Mb : Ma;
+    const lptr<double> R = bside ? Gb : Ga, X = bside ? Mb : Ma;
     if (c < nk)
       for (int x = r - 1; x >= 0; --x) {
         double v = X[x + (size_t)c * K];
@@ -1262,8 +1646,8 @@ __device__ void gram_recompress(const FTask& t, int kt, int K, double* gws, doub
   for (int e = threadIdx.x; e < rb * nk; e += kBlock)
     Cin[pb[e % rb] + (size_t)(e / rb) * K] = Mb[e % rb + (size_t)(e / rb) * K];
   __syncthreads();
-  rows_times_small<double, T>(Va, m, m, K, Cm, K, nk, (T*)tg.a, tg.la);
-  rows_times_small<double, T>(Vb, n, n, K, Cin, K, nk, (T*)tg.b, tg.lb);
+  rows_times_small<T>(Va, m, m, K, Cm, K, nk, (gptr<T>)tg.a, tg.la);
+  rows_times_small<T>(Vb, n, n, K, Cin, K, nk, (gptr<T>)tg.b, tg.lb);
   if (threadIdx.x == 0) *tg.rank = nk;
 }
 
@@ -1347,13 +1731,13 @@ __global__ void __launch_bounds__(kBlock) k_fadd(const FTask* tasks, double* wsb
     }
     __syncthreads();
     double* V = G + (size_t)m * n;
-    dense_to_rk<T>(G, gr, gc, tr, V, V + (size_t)gc * gc, (int*)(V + (size_t)gc * gc + gc),
+    dense_to_rk<T>(G, G == sh, gr, gc, tr, V, V + (size_t)gc * gc, (int*)(V + (size_t)gc * gc + gc),
                    fabs(t.eps), tg, overflow, &flag);
     return;
   }
   if constexpr (sizeof(T) == 4) {
     if (K <= kGramMaxK) {
-      gram_recompress<T>(t, kt, K, gws, sh, fabs(t.eps), overflow, &flag);
+      gram_recompress<T>(t, kt, K, gws, (lptr<double>)sh, fabs(t.eps), overflow, &flag);
       return;
     }
   }
@@ -1368,56 +1752,41 @@ __global__ void __launch_bounds__(kBlock) k_fadd(const FTask* tasks, double* wsb
   // the banks.
   const int64_t core = qr_core(K);
   const int ldAf = m | 1, ldBf = n | 1, ldM = (m > n ? m : n) | 1;
-  int mode;
-  double *Va, *Vb, *cr;
-  int lda, ldb;
+  const double eps = fabs(t.eps);
+  const auto s3 = (lptr<double>)sh;
+  const auto Va = (gptr<double>)gws;
+  const auto Vb = Va + (size_t)m * K;
   if ((int64_t)(ldAf + ldBf) * K + core <= kShDoubles) {
-    mode = 5;
-    Va = sh;
-    lda = ldAf;
-    Vb = sh + (size_t)ldAf * K;
-    ldb = ldBf;
-    cr = Vb + (size_t)ldBf * K;
-  } else if ((int64_t)ldM * K + core <= kShDoubles) {
-    mode = 6;
-    Va = gws;
-    lda = m;
-    Vb = gws + (size_t)m * K;
-    ldb = n;
-    cr = sh + (size_t)ldM * K;
-  } else {
-    Va = gws;
-    lda = m;
-    Vb = gws + (size_t)m * K;
-    ldb = n;
-    cr = core <= kShDoubles ? sh : gws + (size_t)(m + n) * K;
-    mode = cr == sh ? 3 : 4;
-  }
-  const QrScratch w = carve_qr(cr, K);
-  if (mode == 5) {
-    concat_side<T>(Va, lda, m, false, t, kt);
-    concat_side<T>(Vb, ldb, n, true, t, kt);
+    const lptr<double> Pa = s3, Pb = Pa + ldAf * K;
+    const auto w = carve_qr<LdsScratch>(Pb + ldBf * K, K);
+    concat_side<T>(Pa, ldAf, m, false, t, kt);
+    concat_side<T>(Pb, ldBf, n, true, t, kt);
     __syncthreads();
     const int wid = threadIdx.x / kWave;
     if (wid == 0) {
-      wave_house_qr(Va, lda, m, K, w.taua);
-      team_larft<kWave>(Va, lda, m, K, w.taua, w.x, w.ta);
+      wave_house_qr(Pa, ldAf, m, K, w.taua);
+      team_larft<kWave>(Pa, ldAf, m, K, w.taua, w.x, w.ta);
     } else if (wid == 1) {
-      wave_house_qr(Vb, ldb, n, K, w.taub);
-      team_larft<kWave>(Vb, ldb, n, K, w.taub, w.w, w.tb);
+      wave_house_qr(Pb, ldBf, n, K, w.taub);
+      team_larft<kWave>(Pb, ldBf, n, K, w.taub, w.w, w.tb);
     }
     __syncthreads();
-    core_product(Va, lda, Vb, ldb, K, w.g);
-  } else if (mode == 6) {
-    double* P = sh;
+    core_product(Pa, ldAf, Pb, ldBf, K, w.g);
+    __syncthreads();
+    qr_finish<T>(Pa, ldAf, m, Pb, ldBf, n, K, w, eps, tg, overflow, &flag, lptr<double>(nullptr));
+    return;
+  }
+  if ((int64_t)ldM * K + core <= kShDoubles) {
+    const lptr<double> P = s3;
+    const auto w = carve_qr<LdsScratch>(P + ldM * K, K);
     concat_side<T>(P, ldM, m, false, t, kt);
     __syncthreads();
     house_qr(P, ldM, m, K, w.taua);
     team_larft<kBlock>(P, ldM, m, K, w.taua, w.x, w.ta);
     for (int e = threadIdx.x; e < m * K; e += kBlock) {
       const int i = e % m, c = e / m;
-      Va[i + (size_t)c * lda] = P[i + (size_t)c * ldM];
-      if (i < K) w.w[i + (size_t)c * K] = P[i + (size_t)c * ldM];  // Ra
+      Va[i + (size_t)c * m] = P[i + c * ldM];
+      if (i < K) w.w[i + c * K] = P[i + c * ldM];  // Ra
     }
     __syncthreads();
     concat_side<T>(P, ldM, n, true, t, kt);
@@ -1426,44 +1795,22 @@ __global__ void __launch_bounds__(kBlock) k_fadd(const FTask* tasks, double* wsb
     team_larft<kBlock>(P, ldM, n, K, w.taub, w.x, w.tb);
     for (int e = threadIdx.x; e < n * K; e += kBlock) {
       const int i = e % n, c = e / n;
-      Vb[i + (size_t)c * ldb] = P[i + (size_t)c * ldM];
+      Vb[i + (size_t)c * n] = P[i + c * ldM];
     }
     core_product(w.w, K, P, ldM, K, w.g);
-  } else {
-    concat_side<T>(Va, lda, m, false, t, kt);
-    concat_side<T>(Vb, ldb, n, true, t, kt);
     __syncthreads();
-    // V^T V of the global panels on the matrix cores when its LDS staging fits
-    double* part = cr == sh ? sh + core : sh;
-    const bool mfma_gram = K <= 64 && (part - sh) + gram_part(K) <= kShDoubles;
-    // both panels at once, one per half of the workgroup, when each has at
-    // most 16 rows per thread
-    const bool pair = m <= 16 * (kBlock / 2) && n <= 16 * (kBlock / 2);
-    if (pair)
-      house_qr_pair(Va, lda, m, w.taua, Vb, ldb, n, w.taub, K);
-    else
-      house_qr(Va, lda, m, K, w.taua);
-    if (mfma_gram) {
-      wg_reflector_gram_any(Va, lda, m, K, w.x, part);
-      larft_recurrence<kBlock>(K, w.taua, w.x, w.ta);
-    } else {
-      team_larft<kBlock>(Va, lda, m, K, w.taua, w.x, w.ta);
-    }
-    if (!pair) house_qr(Vb, ldb, n, K, w.taub);
-    if (mfma_gram) {
-      wg_reflector_gram_any(Vb, ldb, n, K, w.x, part);
-      larft_recurrence<kBlock>(K, w.taub, w.x, w.tb);
-    } else {
-      team_larft<kBlock>(Vb, ldb, n, K, w.taub, w.x, w.tb);
-    }
-    core_product(Va, lda, Vb, ldb, K, w.g);
+    qr_finish<T>(Va, m, m, Vb, n, n, K, w, eps, tg, overflow, &flag, lptr<double>(nullptr));
+    return;
   }
+  concat_side<T>(Va, m, m, false, t, kt);
+  concat_side<T>(Vb, n, n, true, t, kt);
   __syncthreads();
-  int sweeps = 0;
-  // the core SVD runs on one wavefront when its scratch is in LDS
-  const bool core_lds = mode == 5 || mode == 6 || cr == sh;
-  qr_finish<T>(Va, lda, m, Vb, ldb, n, K, w, core_lds && K <= kWaveJacobiMax, fabs(t.eps), tg, overflow, &flag,
-               &sweeps, core_lds ? nullptr : sh);
+  if (core <= kShDoubles)
+    qr_global<T>(Va, m, Vb, n, K, carve_qr<LdsScratch>(s3, K), s3 + core, kShDoubles - core, eps, tg, overflow,
+                 &flag, lptr<double>(nullptr));
+  else
+    qr_global<T>(Va, m, Vb, n, K, carve_qr<GlobalScratch>(Va + (size_t)(m + n) * K, K), s3, kShDoubles, eps, tg,
+                 overflow, &flag, s3);
 }
 
 // FADD_DENSE: RkMatrix::formattedAddParts with a full part (rk_matrix.cpp:984-1010)
@@ -1498,7 +1845,7 @@ __global__ void __launch_bounds__(kBlock) k_fadd_dense(const FTask* tasks, doubl
   }
   __syncthreads();
   double* V = G + (size_t)m * n;
-  dense_to_rk<T>(G, gr, gc, tr, V, V + (size_t)gc * gc, (int*)(V + (size_t)gc * gc + gc), t.eps, tg,
+  dense_to_rk<T>(G, G == sh, gr, gc, tr, V, V + (size_t)gc * gc, (int*)(V + (size_t)gc * gc + gc), t.eps, tg,
                  overflow, &flag);
 }
 
@@ -1507,40 +1854,26 @@ __global__ void __launch_bounds__(kBlock) k_fadd_dense(const FTask* tasks, doubl
 //   parts[0] = (A1, B1) op-applied left factor, parts[1] = (A2, B2) right factor
 //   tmp = B1^T A2, truncated SVD, newA = A1 U sqrt(S), newB = B2 V sqrt(S)
 // ---------------------------------------------------------------------------
-template <typename T>
-__global__ void __launch_bounds__(kBlock) k_rkrk(const FTask* tasks, double* wsbase, int* overflow) {
-  __shared__ double sh[kShDoubles];
-  __shared__ int flag;
-  if (overflow[1]) return;
-  const FTask& t = tasks[blockIdx.x];
-  const RkRef r1 = t.parts[0].rk, r2 = t.parts[1].rk;
-  RkRef out = t.tgt;
-  const int k1 = rank_of(r1), k2 = rank_of(r2);
-  if (k1 == 0 || k2 == 0) {
-    if (threadIdx.x == 0) *out.rank = 0;
-    return;
-  }
+// ws: the scratch (LDS or global); part: free LDS (part_size doubles), which may
+// be where the output factors go afterwards.
+template <typename T, typename P, typename PI>
+__device__ void rkrk_body(const FTask& t, int k1, int k2, P ws, lptr<double> part, int64_t part_size, int* overflow,
+                          int* flag) {
+  const RkRef r1 = t.parts[0].rk, r2 = t.parts[1].rk, out = t.tgt;
   const int p = r1.n;  // common dimension (rows of B1 == rows of A2)
   const bool tr = k1 < k2;
   const int gr = tr ? k2 : k1, gc = tr ? k1 : k2;
-  const int64_t need = (int64_t)gr * gc + (int64_t)gc * gc + 2 * gc;
-  // SVD scratch, then the output factors (at most (gr + gc) x gc)
-  const int64_t need_full = need + 1 + (int64_t)(gr + gc) * gc;
-  double* ws = need_full <= kShDoubles ? sh : wsbase + t.ws;
-  double* G = ws; ws += (size_t)gr * gc;
-  double* V = ws; ws += (size_t)gc * gc;
-  double* sig = ws; ws += gc;
-  int* order = (int*)ws;
-  const T* A1 = (const T*)r1.a;
-  const T* B1 = (const T*)r1.b;
-  const T* A2 = (const T*)r2.a;
-  const T* B2 = (const T*)r2.b;
+  const P G = ws, V = G + (size_t)gr * gc, sig = V + (size_t)gc * gc;
+  const PI order = (PI)(sig + gc);
+  const auto A1 = (cgptr<T>)r1.a;
+  const auto B1 = (cgptr<T>)r1.b;
+  const auto A2 = (cgptr<T>)r2.a;
+  const auto B2 = (cgptr<T>)r2.b;
   // core B1^T A2 (k1 x k2; stored transposed when tr): on the matrix cores
   // when both ranks are <= 32 and the LDS staging fits, else a wavefront per
   // entry
-  double* part = G == sh ? sh + need + 1 : sh;  // reused by the output factors afterwards
-  const bool mfma = k1 <= 32 && k2 <= 32 && (part - sh) + xty_part(k1, k2) <= kShDoubles &&
-                    wg_xty_any<T>(B1, r1.lb, k1, A2, r2.la, k2, p, G, gr, tr, part);
+  const bool mfma = k1 <= 32 && k2 <= 32 && xty_part(k1, k2) <= part_size &&
+                    wg_xty_any(B1, r1.lb, k1, A2, r2.la, k2, p, G, gr, tr, part);
   if (!mfma) {
     const int lane = threadIdx.x & (kWave - 1), w = threadIdx.x / kWave;
     for (int e = w; e < k1 * k2; e += kWaves) {
@@ -1548,23 +1881,39 @@ __global__ void __launch_bounds__(kBlock) k_rkrk(const FTask* tasks, double* wsb
       double s = 0.0;
       for (int r = lane; r < p; r += kWave) s += (double)B1[r + (size_t)i * r1.lb] * (double)A2[r + (size_t)j * r2.la];
       s = wave_sum(s);
-      if (lane == 0) {
-        if (tr)
-          G[j + (size_t)i * gr] = s;
-        else
-          G[i + (size_t)j * gr] = s;
-      }
+      if (lane == 0) G[tr ? j + (size_t)i * gr : i + (size_t)j * gr] = s;
     }
     __syncthreads();
   }
-  if (G == sh && gc <= kWaveJacobiMax) {
-    if (threadIdx.x < kWave) wave_jacobi_svd(G, gr, gr, gc, V, gc);
-    __syncthreads();
-  } else {
-    jacobi_svd(G, gr, gr, gc, V, gc, &flag);
+  int r = gc;
+  bool done = false;
+  if constexpr (std::is_same_v<P, lptr<double>>)
+    if (gr <= kCoreMax) {
+      // V (gc x r) = G_in^T U with the copy of G kept behind the output factors
+      const P Gin = sig + gc + gc + (gc & 1) + (size_t)(gr + gc) * gc;
+      for (int e = threadIdx.x; e < gr * gc; e += kBlock) Gin[e] = G[e];
+      __syncthreads();
+      if (threadIdx.x < kWave) {
+        const int c = wave_core_svd(G, gr, gr, gc, 1e-26, fmax(1e-30, 1e-16 * t.eps * t.eps));
+        if (threadIdx.x == 0) *flag = c;
+      }
+      __syncthreads();
+      r = *flag;
+      sorted_norms(G, gr, gr, r, sig, order);
+      for (int e = threadIdx.x; e < gc * r; e += kBlock) {
+        const int i = e % gc, j = e / gc;
+        double s = 0.0;
+        for (int l = 0; l < gr; ++l) s += Gin[l + i * gr] * G[l + j * gr];
+        V[i + (size_t)j * gc] = sig[j] > 0.0 ? s / (sig[j] * sig[j]) : 0.0;
+      }
+      __syncthreads();
+      done = true;
+    }
+  if (!done) {
+    jacobi_svd(G, gr, gr, gc, V, gc, flag);
+    sorted_norms(G, gr, gr, gc, sig, order);
   }
-  sorted_norms(G, gr, gr, gc, sig, order);
-  int nk = find_k(sig, order, gc, t.eps);
+  int nk = find_k(sig, order, r, t.eps);
   if (nk > out.cap) {
     if (threadIdx.x == 0) atomicOr(overflow, 1);
     nk = out.cap;
@@ -1573,8 +1922,7 @@ __global__ void __launch_bounds__(kBlock) k_rkrk(const FTask* tasks, double* wsb
   // The small factors Uc (k1 x nk) = U sqrt(S) and Vc (k2 x nk) = V sqrt(S)
   // go after the SVD scratch, then the outputs stream A1 and B2 once per
   // eight columns.
-  double* Uc = (double*)(order + gc + (gc & 1));
-  double* Vc = Uc + (size_t)k1 * nk;
+  const P Uc = sig + gc + gc + (gc & 1), Vc = Uc + (size_t)k1 * nk;
   for (int e = threadIdx.x; e < k1 * nk; e += kBlock) {
     const int l = e % k1, c = e / k1, j = order[c];
     const double sq = sqrt(sig[j]);
@@ -1587,39 +1935,158 @@ __global__ void __launch_bounds__(kBlock) k_rkrk(const FTask* tasks, double* wsb
   }
   __syncthreads();
   const int m = r1.m, n = r2.n;
-  rows_times_small<T>(A1, r1.la, m, k1, Uc, k1, nk, (T*)out.a, out.la);
-  rows_times_small<T>(B2, r2.lb, n, k2, Vc, k2, nk, (T*)out.b, out.lb);
+  rows_times_small<T>(A1, r1.la, m, k1, Uc, k1, nk, (gptr<T>)out.a, out.la);
+  rows_times_small<T>(B2, r2.lb, n, k2, Vc, k2, nk, (gptr<T>)out.b, out.lb);
   if (threadIdx.x == 0) *out.rank = nk;
+}
+
+template <typename T>
+__global__ void __launch_bounds__(kBlock) k_rkrk(const FTask* tasks, double* wsbase, int* overflow) {
+  __shared__ double sh[kShDoubles];
+  __shared__ int flag;
+  if (overflow[1]) return;
+  const FTask& t = tasks[blockIdx.x];
+  const int k1 = rank_of(t.parts[0].rk), k2 = rank_of(t.parts[1].rk);
+  if (k1 == 0 || k2 == 0) {
+    if (threadIdx.x == 0) *t.tgt.rank = 0;
+    return;
+  }
+  const int gr = k1 > k2 ? k1 : k2, gc = k1 < k2 ? k1 : k2;
+  const int64_t need = (int64_t)gr * gc + (int64_t)gc * gc + 2 * gc + 1;
+  // SVD scratch, then the output factors (at most (gr + gc) x gc)
+  const auto s3 = (lptr<double>)sh;
+  if (need + (int64_t)(gr + gc) * gc + (int64_t)gr * gc <= kShDoubles)
+    rkrk_body<T, lptr<double>, lptr<int>>(t, k1, k2, s3, s3 + need, kShDoubles - need, overflow, &flag);
+  else
+    rkrk_body<T, gptr<double>, gptr<int>>(t, k1, k2, (gptr<double>)(wsbase + t.ws), s3, kShDoubles, overflow, &flag);
 }
 
 // ---------------------------------------------------------------------------
 // ACAFULL: acaFull (compression.cpp:270-355) on a dense temp (modified)
 constexpr int kAcaLds = 16384;  // entries of the LDS copy (a 128 x 128 leaf product)
 // ---------------------------------------------------------------------------
+// acaFull's stopping estimate after term nu (the reference sums l < nu - 1):
+// est += 2 sum_l (a_nu . a_l)(b_nu . b_l) + |a_nu|^2 |b_nu|^2; true when the new
+// term is below eps of it.  Each wavefront takes the terms l = w, w + 4, ...
+// with wavefront sums, then one workgroup sum.
 template <typename T>
-__global__ void __launch_bounds__(kBlock) k_acafull(const FTask* tasks, const int* fail) {
+__device__ inline bool acafull_converged(const RkRef& out, int m, int n, int nu, double eps, double& est) {
+  __shared__ double red[3][kWaves];
+  const int lane = threadIdx.x & (kWave - 1), wv = threadIdx.x / kWave;
+  const auto OA = (gptr<T>)out.a;
+  const auto OB = (gptr<T>)out.b;
+  const auto va = OA + (size_t)nu * out.la;
+  const auto vb = OB + (size_t)nu * out.lb;
+  double part = 0.0, an = 0.0, bn = 0.0;
+  for (int l = wv; l + 1 < nu; l += kWaves) {
+    double da = 0.0, db = 0.0;
+    for (int r = lane; r < m; r += kWave) da += (double)va[r] * (double)OA[r + (size_t)l * out.la];
+    for (int c = lane; c < n; c += kWave) db += (double)vb[c] * (double)OB[c + (size_t)l * out.lb];
+    part += wave_sum(da) * wave_sum(db);
+  }
+  for (int r = threadIdx.x; r < m; r += kBlock) an += (double)va[r] * (double)va[r];
+  for (int c = threadIdx.x; c < n; c += kBlock) bn += (double)vb[c] * (double)vb[c];
+  an = wave_sum(an);
+  bn = wave_sum(bn);
+  __syncthreads();
+  if (lane == 0) {
+    red[0][wv] = part;
+    red[1][wv] = an;
+    red[2][wv] = bn;
+  }
+  __syncthreads();
+  double v[3] = {0.0, 0.0, 0.0};
+#pragma unroll
+  for (int q = 0; q < 3; ++q)
+#pragma unroll
+    for (int i = 0; i < kWaves; ++i) v[q] += red[q][i];
+  const double ab = v[1] * v[2];
+  est += 2.0 * v[0] + ab;
+  return ab < eps * eps * est;
+}
+
+// Blocks of at most 128 x 128: threads 2 c and 2 c + 1 hold the halves of column
+// c in registers (storage precision), so a step is one pass over them for the
+// update and the next maximum; the pivot column goes through LDS, the pivot
+// row's entry of a column is picked by its own thread.  Bound: those passes
+// (64 entries per thread).  125 x 125 blocks, ten terms: 170 us in LDS with an index
+// division per entry, 56 (FP32) to 71 us (FP64) now.
+constexpr int kAcaRows = 64;  // rows per thread
+template <typename T>
+__device__ void acafull_regs(const FTask& t) {
+  __shared__ T col[2 * kAcaRows];
   __shared__ double rv[kWaves];
   __shared__ int ri[kWaves];
-  __shared__ double red[kWaves];
-  if (*fail) return;
-  const FTask& t = tasks[blockIdx.x];
-  RkRef out = t.tgt;
+  const RkRef out = t.tgt;
   const int m = t.m.s, n = t.n.s;
-  // the dense block is a temporary: work on an LDS copy (in the storage
-  // precision) when it fits, on the block itself otherwise
-  __shared__ T dl[kAcaLds];
-  T* D = (T*)t.A;
-  int ld = t.lda;
-  if ((int64_t)m * n <= kAcaLds) {
-    stage_in(dl, m, (const T*)t.A, 1L, (long)t.lda, m, n);
-    __syncthreads();
-    D = dl;
-    ld = m;
+  const auto D = (cgptr<T>)t.A;
+  const int c = threadIdx.x >> 1, h = threadIdx.x & 1, r0 = h * kAcaRows;
+  const bool live = c < n;
+  T g[kAcaRows];
+#pragma unroll
+  for (int r = 0; r < kAcaRows; ++r) {
+    const int i = r0 + r < m ? r0 + r : m - 1;
+    const T v = D[i + (size_t)(live ? c : n - 1) * t.lda];
+    g[r] = (live && r0 + r < m) ? v : (T)0;
   }
   int maxk = m < n ? m : n;
   if (maxk > out.cap) maxk = out.cap;
-  T* OA = (T*)out.a;
-  T* OB = (T*)out.b;
+  double est = 0.0;
+  int nu = 0;
+  for (; nu < maxk; ++nu) {
+    // the largest |entry|, the first of equals in column-major order (NaNs lose)
+    T best = (T)-1;
+    int at = -1;
+#pragma unroll
+    for (int r = 0; r < kAcaRows; ++r) {
+      const T v = g[r] < (T)0 ? -g[r] : g[r];
+      if (v > best && live && r0 + r < m) {
+        best = v;
+        at = r;
+      }
+    }
+    ArgMax a{(double)best, at < 0 ? -1 : r0 + at + c * m};
+    a = block_argmax(a, rv, ri);
+    if (a.i < 0) break;  // all-NaN block
+    const int i = a.i % m, j = a.i / m;
+    const auto va = (gptr<T>)out.a + (size_t)nu * out.la;
+    const auto vb = (gptr<T>)out.b + (size_t)nu * out.lb;
+    if (c == j) {
+#pragma unroll
+      for (int r = 0; r < kAcaRows; ++r) col[r0 + r] = g[r];
+    }
+    // the entry of row i in this column (held by one half)
+    T x = (T)0;
+    const int ir = i - r0;
+#pragma unroll
+    for (int r = 0; r < kAcaRows; ++r) x = r == ir ? g[r] : x;
+    const T y = dpp_swap<0xB1>(x);
+    x = (ir >= 0 && ir < kAcaRows) ? x : y;
+    __syncthreads();
+    const double delta = (double)col[i];
+    if (delta == 0.0) break;
+    const T b = (T)((double)x / delta);
+    if (live && h == 0) vb[c] = b;
+    if ((int)threadIdx.x < m) va[threadIdx.x] = col[threadIdx.x];
+#pragma unroll
+    for (int r = 0; r < kAcaRows; ++r) g[r] -= col[r0 + r] * b;
+    __syncthreads();
+    if (acafull_converged<T>(out, m, n, nu, t.eps, est)) break;
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) *out.rank = nu;
+}
+
+// Other shapes: the dense block is a temporary, so the steps work on it (or on
+// its LDS copy) in place.
+template <typename T, typename PD>
+__device__ void acafull_body(const FTask& t, PD D, int ld) {
+  __shared__ double rv[kWaves];
+  __shared__ int ri[kWaves];
+  const RkRef out = t.tgt;
+  const int m = t.m.s, n = t.n.s;
+  int maxk = m < n ? m : n;
+  if (maxk > out.cap) maxk = out.cap;
   double est = 0.0;
   int nu = 0;
   for (; nu < maxk; ++nu) {
@@ -1631,8 +2098,8 @@ __global__ void __launch_bounds__(kBlock) k_acafull(const FTask* tasks, const in
     const int i = a.i % m, j = a.i / m;
     const double delta = (double)D[i + (size_t)j * ld];
     if (delta == 0.0) break;
-    T* va = OA + (size_t)nu * out.la;
-    T* vb = OB + (size_t)nu * out.lb;
+    const auto va = (gptr<T>)out.a + (size_t)nu * out.la;
+    const auto vb = (gptr<T>)out.b + (size_t)nu * out.lb;
     for (int r = threadIdx.x; r < m; r += kBlock) va[r] = D[r + (size_t)j * ld];
     for (int c = threadIdx.x; c < n; c += kBlock) vb[c] = (T)((double)D[i + (size_t)c * ld] / delta);
     __syncthreads();
@@ -1640,30 +2107,27 @@ __global__ void __launch_bounds__(kBlock) k_acafull(const FTask* tasks, const in
       const int r = e % m, c = e / m;
       D[r + (size_t)c * ld] -= va[r] * vb[c];
     }
-    // estimate (the reference sums l < nu - 1): each wavefront takes the terms
-    // l = w, w + 4, ... with wavefront sums, then one workgroup sum
-    double cross = 0.0;
-    {
-      const int lane = threadIdx.x & (kWave - 1), wv = threadIdx.x / kWave;
-      double part = 0.0;
-      for (int l = wv; l + 1 < nu; l += kWaves) {
-        double da = 0.0, db = 0.0;
-        for (int r = lane; r < m; r += kWave) da += (double)va[r] * (double)OA[r + (size_t)l * out.la];
-        for (int c = lane; c < n; c += kWave) db += (double)vb[c] * (double)OB[c + (size_t)l * out.lb];
-        part += wave_sum(da) * wave_sum(db);
-      }
-      cross = block_sum(lane == 0 ? part : 0.0, red);
-    }
-    double an = 0.0, bn = 0.0;
-    for (int r = threadIdx.x; r < m; r += kBlock) an += (double)va[r] * (double)va[r];
-    for (int c = threadIdx.x; c < n; c += kBlock) bn += (double)vb[c] * (double)vb[c];
-    an = block_sum(an, red);
-    bn = block_sum(bn, red);
-    est += 2.0 * cross + an * bn;
-    if (an * bn < t.eps * t.eps * est) break;
+    if (acafull_converged<T>(out, m, n, nu, t.eps, est)) break;
   }
   __syncthreads();
   if (threadIdx.x == 0) *out.rank = nu;
+}
+
+template <typename T>
+__global__ void __launch_bounds__(kBlock) k_acafull(const FTask* tasks, const int* fail) {
+  __shared__ T dl[kAcaLds];
+  if (*fail) return;
+  const FTask& t = tasks[blockIdx.x];
+  const int m = t.m.s, n = t.n.s;
+  if (m <= 2 * kAcaRows && n <= kBlock / 2) {
+    acafull_regs<T>(t);
+  } else if ((int64_t)m * n <= kAcaLds) {
+    stage_in((lptr<T>)dl, m, (cgptr<T>)t.A, 1L, (long)t.lda, m, n);
+    __syncthreads();
+    acafull_body<T>(t, (lptr<T>)dl, m);
+  } else {
+    acafull_body<T>(t, (gptr<T>)t.A, t.lda);
+  }
 }
 
 }  // namespace
