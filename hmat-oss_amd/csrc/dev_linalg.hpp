@@ -927,4 +927,28 @@ __device__ inline int find_k(PS sig, PI order, int n, double eps) {
   return k;
 }
 
+// sorted_norms and find_k of at most kCoreMax columns by one wavefront: a lane
+// per column, the order by counting.  Returns find_k's number.
+__device__ inline int wave_sorted_cut(lptr<double> G, int ldg, int rows, int cols, lptr<double> sig,
+                                      lptr<int> order, double eps) {
+  const int lane = threadIdx.x & (kWave - 1);
+  const lptr<double> g = G + (lane < cols ? lane : 0) * ldg;
+  double s = 0.0;
+  for (int i = 0; i < rows; ++i) s += g[i] * g[i];
+  s = (s >= 0.0 && s <= 1.79e308) ? sqrt(s) : 0.0;
+  int pos = 0;
+  double top = 0.0;
+  for (int i = 0; i < cols; ++i) {
+    const double si = lane_read(s, i);
+    pos += (si > s) || (si == s && i < lane);
+    top = fmax(top, si);
+  }
+  if (lane < cols) {
+    sig[lane] = s;
+    order[pos] = lane;
+  }
+  __builtin_amdgcn_wave_barrier();
+  return __popcll(__ballot(lane < cols && !(s <= top * eps)));
+}
+
 }  // namespace hmx

@@ -167,6 +167,69 @@ __device__ inline bool wg_xty_any(PX X, int ldx, int kx, PX Y, int ldy, int ky, 
   return true;
 }
 
+// G = X^T X (k x k, ld ldg, both triangles) for X (p x k, ld ldx, k <= 16 kNb <= 48):
+// wg_xty for one panel, each entry loaded once and the tiles on and above the
+// diagonal only; kU slabs' loads in flight per wavefront.
+template <int kNb, int kU, typename PX>
+__device__ void wg_gram(PX X, int ldx, int k, int p, lptr<double> G, int ldg, lptr<double> part) {
+  constexpr int kTiles = kNb * (kNb + 1) / 2;
+  const int lane = threadIdx.x & (kWave - 1), w = threadIdx.x / kWave;
+  const int kk = lane >> 4, ii = lane & 15;
+  hmx_double4 acc[kTiles];
+#pragma unroll
+  for (int t = 0; t < kTiles; ++t) acc[t] = hmx_double4{0.0, 0.0, 0.0, 0.0};
+  PX col[kNb];
+  bool in[kNb];
+#pragma unroll
+  for (int b = 0; b < kNb; ++b) {
+    in[b] = 16 * b + ii < k;
+    col[b] = X + (size_t)(in[b] ? 16 * b + ii : k - 1) * ldx;
+  }
+  for (int r0 = 4 * w; r0 < p; r0 += 16 * kU) {
+    double x[kU][kNb];
+#pragma unroll
+    for (int u = 0; u < kU; ++u) {
+      const int r = r0 + 16 * u + kk, rc = r < p ? r : p - 1;
+#pragma unroll
+      for (int b = 0; b < kNb; ++b) x[u][b] = col[b][rc];
+    }
+#pragma unroll
+    for (int u = 0; u < kU; ++u) {
+      const bool live = r0 + 16 * u + kk < p;
+#pragma unroll
+      for (int b = 0; b < kNb; ++b) x[u][b] = live && in[b] ? x[u][b] : 0.0;
+      int t = 0;
+#pragma unroll
+      for (int a = 0; a < kNb; ++a)
+#pragma unroll
+        for (int b = a; b < kNb; ++b, ++t)
+          acc[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(x[u][a], x[u][b], acc[t], 0, 0, 0);
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int t = 0; t < kTiles; ++t)
+#pragma unroll
+    for (int v = 0; v < 4; ++v) part[(w * kTiles + t) * 256 + v * kWave + lane] = acc[t][v];
+  __syncthreads();
+  // thread q of a tile holds entry (4 (q / 64) + (q mod 64) / 16, q mod 16)
+#pragma unroll
+  for (int t = 0; t < kTiles; ++t) {
+    // tile t is (a, b), a <= b, row by row
+    const int a = t < kNb ? 0 : (t < 2 * kNb - 1 ? 1 : 2), b = a == 0 ? t : (a == 1 ? t - kNb + 1 : 2);
+    const int q = threadIdx.x;
+    double s = 0.0;
+#pragma unroll
+    for (int v = 0; v < kWaves; ++v) s += part[(v * kTiles + t) * 256 + q];
+    const int i = 16 * a + 4 * (q / kWave) + (q & (kWave - 1)) / 16, j = 16 * b + (q & 15);
+    if (i < k && j < k) {
+      G[i + j * ldg] = s;
+      if (a != b) G[j + i * ldg] = s;
+    }
+  }
+  __syncthreads();
+}
+
 // out (rows x nk, ld ldo) = M (rows x k, ld ldm) C (k x nk, ld ldc; LDS or
 // global): each thread owns rows and streams a row of M once per eight
 // output columns.

@@ -66,6 +66,8 @@ struct Part {
   double alpha;
 };
 
+constexpr int kMaxParts = 4;
+
 struct FTask {
   int type;
   int mode;          // trsm mode, gemm beta (0/1)
@@ -80,7 +82,7 @@ struct FTask {
   int nparts;
   int pad;
   RkRef tgt;         // FADD / FADD_DENSE / RKRK / ACAFULL output
-  Part parts[4];     // FADD inputs; RKRK uses parts[0] (A1 B1^T) and parts[1] (A2 B2^T)
+  Part parts[kMaxParts];  // FADD inputs; RKRK uses parts[0] (A1 B1^T) and parts[1] (A2 B2^T)
   int64_t ws;        // workspace offset (doubles)
 };
 

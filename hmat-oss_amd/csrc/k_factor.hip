@@ -1260,6 +1260,87 @@ __device__ void concat_side(PD dst, int ld, int rows, bool bside, const FTask& t
   }
 }
 
+// Both sides at once for K <= kColsMax: a lane builds each column's descriptor,
+// then every wavefront copies four columns at a time, their loads in flight
+// together and no index divided.
+constexpr int kColsMax = 40;
+constexpr int kColDoubles = 6 * kColsMax;  // LDS for the descriptors (2 K of three doubles)
+
+template <typename T, typename PD>
+__device__ void concat_both(PD da, int lda, PD db, int ldb, int K, const FTask& t, int kt, lptr<double> desc) {
+  const int lane = threadIdx.x & (kWave - 1), w = threadIdx.x / kWave;
+  const RkRef& tg = t.tgt;
+  const auto base = (lptr<long>)desc;            // address of the column's row 0
+  const auto span = (lptr<int>)(desc + 2 * K);   // offset and rows
+  const auto scale = desc + 4 * K;
+  const int c = threadIdx.x;
+  if (c < 2 * K) {
+    const bool bside = c >= K;
+    int cc = bside ? c - K : c;
+    const T* p = (const T*)(bside ? tg.b : tg.a);
+    int ld = bside ? tg.lb : tg.la, o = 0, pr = bside ? tg.n : tg.m;
+    double f = 1.0;
+    if (cc >= kt) {
+      cc -= kt;
+      for (int q = 0; q < t.nparts; ++q) {
+        const Part& x = t.parts[q];
+        const int kq = rank_of(x.rk);
+        if (!(kq > 0 && x.alpha != 0.0 && x.rk.m > 0 && x.rk.n > 0)) continue;
+        if (cc < kq) {
+          p = (const T*)(bside ? x.rk.b : x.rk.a);
+          ld = bside ? x.rk.lb : x.rk.la;
+          o = bside ? x.coff : x.roff;
+          pr = bside ? x.rk.n : x.rk.m;
+          f = bside ? 1.0 : x.alpha;
+          break;
+        }
+        cc -= kq;
+      }
+    }
+    base[c] = (long)(p + (size_t)cc * ld);
+    span[2 * c] = o;
+    span[2 * c + 1] = pr;
+    scale[c] = f;
+  }
+  __syncthreads();
+  constexpr int kC = 4, kR = 2;
+  for (int c0 = kC * w; c0 < 2 * K; c0 += kC * kWaves) {
+    cgptr<T> p[kC];
+    int o[kC], pr[kC], len[kC], most = 0;
+    double f[kC];
+    PD dst[kC];
+#pragma unroll
+    for (int b = 0; b < kC; ++b) {
+      const int cb = c0 + b < 2 * K ? c0 + b : 2 * K - 1;
+      p[b] = (cgptr<T>)base[cb];
+      o[b] = span[2 * cb];
+      pr[b] = span[2 * cb + 1];
+      f[b] = scale[cb];
+      len[b] = c0 + b >= 2 * K ? 0 : (cb < K ? tg.m : tg.n);
+      dst[b] = cb < K ? da + (size_t)cb * lda : db + (size_t)(cb - K) * ldb;
+      most = len[b] > most ? len[b] : most;
+    }
+    for (int r0 = lane; r0 < most; r0 += kR * kWave) {
+      T x[kR][kC];
+#pragma unroll
+      for (int u = 0; u < kR; ++u)
+#pragma unroll
+        for (int b = 0; b < kC; ++b) {
+          const int r = r0 + u * kWave - o[b];
+          x[u][b] = p[b][r < 0 ? 0 : (r < pr[b] ? r : pr[b] - 1)];
+        }
+#pragma unroll
+      for (int u = 0; u < kR; ++u)
+#pragma unroll
+        for (int b = 0; b < kC; ++b) {
+          const int r = r0 + u * kWave;
+          if (r < len[b]) dst[b][r] = (r >= o[b] && r < o[b] + pr[b]) ? f[b] * (double)x[u][b] : 0.0;
+        }
+    }
+  }
+  __syncthreads();
+}
+
 // G (K x K) = Ra Rb^T with Ra, Rb the upper triangles of two panels.
 template <typename PA, typename PB, typename PG>
 __device__ inline void core_product(PA Ra, int lra, PB Rb, int lrb, int K, PG G) {
@@ -1370,7 +1451,7 @@ template <typename T, typename PV, typename P, typename PI>
 __device__ void qr_finish(PV Va, int lda, int m, PV Vb, int ldb, int n, int K, const QrScratch<P, PI>& w,
                           double eps, RkRef out, int* overflow, int* flag, lptr<double> stage) {
   constexpr bool kInLds = std::is_same_v<P, lptr<double>>;
-  __shared__ int core_rank;
+  __shared__ int core_rank, core_cut;
   int r = K;  // columns of the rotated core
   // one-sided Jacobi on G without V: G_in (kept in w.v) gives the right side
   // afterwards as G_in^T U, so the rounds only rotate G
@@ -1388,6 +1469,10 @@ __device__ void qr_finish(PV Va, int lda, int m, PV Vb, int ldb, int n, int K, c
     }
     if (threadIdx.x < kWave) {
       const int c = wave_core_svd(g, K, K, K, 1e-26, fmax(1e-30, 1e-16 * eps * eps));
+      if constexpr (kInLds) {
+        const int k = wave_sorted_cut(g, K, K, c, w.sig, w.order, eps);
+        if (threadIdx.x == 0) core_cut = k;
+      }
       if (threadIdx.x == 0) core_rank = c;
     }
     __syncthreads();
@@ -1409,8 +1494,13 @@ __device__ void qr_finish(PV Va, int lda, int m, PV Vb, int ldb, int n, int K, c
     jacobi_svd(w.g, K, K, K, P(nullptr), K, flag);
     __syncthreads();
   }
-  sorted_norms(w.g, K, K, r, w.sig, w.order);
-  int nk = find_k(w.sig, w.order, r, eps);
+  int nk;
+  if (kInLds && K <= kCoreMax) {
+    nk = core_cut;
+  } else {
+    sorted_norms(w.g, K, K, r, w.sig, w.order);
+    nk = find_k(w.sig, w.order, r, eps);
+  }
   if (nk > out.cap) {
     if (threadIdx.x == 0) atomicOr(overflow, 1);
     nk = out.cap;
@@ -1481,94 +1571,129 @@ __device__ void qr_global(gptr<double> Va, int m, gptr<double> Vb, int n, int K,
 // A' = A P1 R11^-1 U sqrt(S), B' = B P1 R11^-1 V sqrt(S).  Q is orthonormal to
 // about 1e-16 / 1e-13 = 1e-3, so the truncated product stays within eps.
 // ---------------------------------------------------------------------------
-constexpr int kGramMaxK = 32;
-static_assert(kGramMaxK <= kCoreMax, "the core SVD takes the whole core");
+// Widest sum in this form: its small matrices fit in LDS (K = 40: 130 KB).  33 to
+// 38 columns took 1.0 to 1.4 ms as Householder QR with a workgroup's Jacobi.
+constexpr int kGramMaxK = kColsMax;
 constexpr double kGramTol = 1e-13;
 constexpr double kGramJacobiTol2 = 1e-16;
 
-// Pivoted Cholesky of G (K x K, ld K, symmetric, K <= 64) by one wavefront:
-// returns the rank r; rows 0..r-1 of the upper triangle hold R in the pivoted
-// column order, piv[0..K) the order.
-__device__ inline int wave_pchol(lptr<double> G, int K, lptr<int> piv) {
-  const int lane = threadIdx.x & (kWave - 1);
-  if (lane < K) piv[lane] = lane;
-  const double dmax = wave_argmax(ArgMax{lane < K ? G[lane + (size_t)lane * K] : -1.0, lane < K ? lane : -1}).v;
-  const double tol = kGramTol * dmax;
-  __builtin_amdgcn_wave_barrier();
+// Pivoted Cholesky of G (K x K, ld K, symmetric, K <= kN) by one wavefront, lane
+// c holding column c of the factor in registers (left-looking: row j is G's row
+// of the pivot less the rows above, the pivot's entries by readlane): G = R^T R
+// with R (rank x K, ld K, columns in G's order, zeros in columns already
+// pivoted), piv[j] the pivot of row j, rinv[j] = 1 / R[j, piv[j]].  Returns the
+// rank.  Bound: its K^2 / 2 steps of two readlanes and an FMA.
+template <int kN>
+__device__ inline int wave_pchol(lptr<double> G, int K, lptr<double> R, lptr<int> piv, lptr<double> rinv) {
+  const int lane = threadIdx.x & (kWave - 1), lc = lane < K ? lane : K - 1;
+  double d = lane < K ? G[lc + lc * K] : -1.0;
+  const double tol = kGramTol * wave_max(d);
+  double row[kN];
   int r = 0;
-  for (int j = 0; j < K; ++j) {
-    const bool in = lane >= j && lane < K;
-    const ArgMax a = wave_argmax(ArgMax{in ? G[lane + (size_t)lane * K] : -1.0, in ? lane : -1});
-    if (!(a.v > tol)) break;  // also on NaN
-    const int p = a.i;
-    if (p != j) {
-      if (lane < K) {
-        const double x = G[j + (size_t)lane * K];
-        G[j + (size_t)lane * K] = G[p + (size_t)lane * K];
-        G[p + (size_t)lane * K] = x;
+  bool go = true;
+  static_for<0, kN>([&](auto jc) __attribute__((always_inline)) {
+    constexpr int j = decltype(jc)::value;
+    if (go && j < K) {
+      const double m = wave_max(d);
+      if (m > tol) {
+        const int p = __builtin_ctzll(__ballot(d == m));
+        double v = G[lc + p * K];
+        static_for<0, j>([&](auto ic) __attribute__((always_inline)) {
+          constexpr int i = decltype(ic)::value;
+          v -= lane_read(row[i], p) * row[i];
+        });
+        const double root = chain_sqrt(m), inv = chain_rcp(root);
+        const bool done = !(d >= 0.0) && lane != p;  // pivoted before (or past K)
+        const double x = lane == p ? root : (done ? 0.0 : v * inv);
+        row[j] = x;
+        d = lane == p || done ? -1.0 : fmax(d - x * x, 0.0);
+        if (lane < K) R[j + lane * K] = x;
+        if (lane == 0) {
+          piv[j] = p;
+          rinv[j] = inv;
+        }
+        r = j + 1;
+      } else {
+        go = false;
       }
-      __builtin_amdgcn_wave_barrier();
-      if (lane < K) {
-        const double x = G[lane + (size_t)j * K];
-        G[lane + (size_t)j * K] = G[lane + (size_t)p * K];
-        G[lane + (size_t)p * K] = x;
-      }
-      if (lane == 0) {
-        const int q = piv[j];
-        piv[j] = piv[p];
-        piv[p] = q;
-      }
-      __builtin_amdgcn_wave_barrier();
     }
-    const double d = sqrt(G[j + (size_t)j * K]);
-    __builtin_amdgcn_wave_barrier();
-    if (lane > j && lane < K) G[j + (size_t)lane * K] /= d;
-    if (lane == j) G[j + (size_t)j * K] = d;
-    __builtin_amdgcn_wave_barrier();
-    const int tr = K - j - 1;
-    for (int e = lane; e < tr * tr; e += kWave) {
-      const int i = j + 1 + e % tr, l = j + 1 + e / tr;
-      G[i + (size_t)l * K] -= G[j + (size_t)i * K] * G[j + (size_t)l * K];
-    }
-    __builtin_amdgcn_wave_barrier();
-    r = j + 1;
-  }
+  });
+  __builtin_amdgcn_wave_barrier();
   return r;
 }
 
-// LDS doubles of gram_recompress for K columns
-__device__ inline int gram_lds(int K) { return 6 * K * K + 4 * K + xty_part(K, K); }
+// out (K, rows piv[i] = solution, zero elsewhere) = P1 R11^-1 x for one column x
+// (r entries) on this thread: R as wave_pchol leaves it.  Column-oriented, x in
+// registers, so that a step's products are independent.
+template <int kN>
+__device__ inline void pchol_solve(lptr<double> R, int K, lptr<int> piv, lptr<double> rinv, int r, lptr<double> x,
+                                   lptr<double> out) {
+  double v[kN];
+#pragma unroll
+  for (int i = 0; i < kN; ++i) v[i] = i < r ? x[i] : 0.0;
+  for (int i = 0; i < K; ++i) out[i] = 0.0;
+  static_for<0, kN>([&](auto ic) __attribute__((always_inline)) {
+    constexpr int i = kN - 1 - decltype(ic)::value;
+    if (i < r) {
+      const int p = piv[i];
+      const lptr<double> col = R + p * K;
+      const double y = v[i] * rinv[i];
+      out[p] = y;
+#pragma unroll
+      for (int l = 0; l < i; ++l) v[l] -= col[l] * y;
+    }
+  });
+}
 
-template <typename T>
-__device__ void gram_recompress(const FTask& t, int kt, int K, double* gws, lptr<double> sh, double eps,
-                                int* overflow, int* flag) {
-  __shared__ int ranks[2];
+// LDS doubles of gram_recompress for K columns, beside the panels
+__device__ inline int gram_lds(int K) {
+  const int nb = (K + 15) / 16;
+  const int part = 512 * nb * (nb + 1);
+  return 6 * K * K + 6 * K + (part > kColDoubles ? part : kColDoubles);
+}
+
+// The panels Va (m x K, ld lda) and Vb in LDS or global memory (PV).  With an
+// index division per entry, both panels in global memory and the Cholesky, the
+// sort and the triangular solve through LDS, a block of up to 256 rows took 55 us
+// (19 of them the core SVD) and an average launch of FADD 147 us (40,000 points)
+// and 159 us (8,000 points); now 104 and 120 us.  Bound: the serial steps of the
+// core SVD, in long panels the reads of the Gram products.
+template <typename T, typename PV>
+__device__ void gram_recompress(PV Va, int lda, PV Vb, int ldb, const FTask& t, int kt, int K, lptr<double> sh,
+                                double eps, int* overflow) {
+  __shared__ int ranks[3];
   const RkRef tg = t.tgt;
   const int m = tg.m, n = tg.n;
-  const auto Va = (gptr<double>)gws;
-  const auto Vb = Va + (size_t)m * K;
-  concat_side<T>(Va, m, m, false, t, kt);
-  concat_side<T>(Vb, n, n, true, t, kt);
-  __syncthreads();
   const int K2 = K * K;
   const lptr<double> Ga = sh;
   const lptr<double> Gb = Ga + K2;
   const lptr<double> Cm = Gb + K2;
   const lptr<double> Cin = Cm + K2;
-  const lptr<double> Ma = Cin + K2;
-  const lptr<double> Mb = Ma + K2;
-  const lptr<double> sig = Mb + K2;
-  const lptr<int> order = (lptr<int>)(sig + K), pa = order + K, pb = pa + K;
-  const lptr<double> part = sig + 4 * K;
-  wg_xty_any(Va, m, K, Va, m, K, m, Ga, K, false, part);
-  wg_xty_any(Vb, n, K, Vb, n, K, n, Gb, K, false, part);
+  const lptr<double> Ra = Cin + K2;
+  const lptr<double> Rb = Ra + K2;
+  const lptr<double> sig = Rb + K2;
+  const lptr<double> scale = sig + K, ia = scale + K, ib = ia + K;
+  const lptr<int> order = (lptr<int>)(ib + K), pa = order + K, pb = pa + K;
+  const lptr<double> part = sig + 6 * K;
+  concat_both<T>(Va, lda, Vb, ldb, K, t, kt, part);
+  constexpr bool kInLds = std::is_same_v<PV, lptr<double>>;
+  constexpr int kU = kInLds ? 4 : 8;
+  if (K <= 16) {
+    wg_gram<1, kU>(Va, lda, K, m, Ga, K, part);
+    wg_gram<1, kU>(Vb, ldb, K, n, Gb, K, part);
+  } else if (K <= 32) {
+    wg_gram<2, kU / 2>(Va, lda, K, m, Ga, K, part);
+    wg_gram<2, kU / 2>(Vb, ldb, K, n, Gb, K, part);
+  } else {
+    wg_gram<3, 2>(Va, lda, K, m, Ga, K, part);
+    wg_gram<3, 2>(Vb, ldb, K, n, Gb, K, part);
+  }
   const int wid = threadIdx.x / kWave, lane = threadIdx.x & (kWave - 1);
-  if (wid == 0) {
-    const int r = wave_pchol(Ga, K, pa);
-    if (lane == 0) ranks[0] = r;
-  } else if (wid == 1) {
-    const int r = wave_pchol(Gb, K, pb);
-    if (lane == 0) ranks[1] = r;
+  if (wid < 2) {
+    const lptr<double> G = wid ? Gb : Ga, R = wid ? Rb : Ra, inv = wid ? ib : ia;
+    const lptr<int> piv = wid ? pb : pa;
+    const int r = K <= 16 ? wave_pchol<16>(G, K, R, piv, inv) : wave_pchol<kGramMaxK>(G, K, R, piv, inv);
+    if (lane == 0) ranks[wid] = r;
   }
   __syncthreads();
   const int ra = ranks[0], rb = ranks[1];
@@ -1576,78 +1701,63 @@ __device__ void gram_recompress(const FTask& t, int kt, int K, double* gws, lptr
     if (threadIdx.x == 0) *tg.rank = 0;
     return;
   }
-  // R~a (ra x K) and R~b (rb x K), ld K, columns in panel order
-  for (int e = threadIdx.x; e < K2; e += kBlock) Ma[e] = Mb[e] = 0.0;
-  __syncthreads();
-  for (int e = threadIdx.x; e < ra * K; e += kBlock) {
-    const int x = e % ra, i = e / ra;
-    if (i >= x) Ma[x + (size_t)pa[i] * K] = Ga[x + (size_t)i * K];
-  }
-  for (int e = threadIdx.x; e < rb * K; e += kBlock) {
-    const int y = e % rb, i = e / rb;
-    if (i >= y) Mb[y + (size_t)pb[i] * K] = Gb[y + (size_t)i * K];
-  }
-  __syncthreads();
-  // core (ra x rb, ld ra) = R~a R~b^T, kept in Cin for the right side
+  // core (ra x rb, ld ra) = Ra Rb^T, kept in Cin for the right side
   for (int e = threadIdx.x; e < ra * rb; e += kBlock) {
     const int x = e % ra, y = e / ra;
     double s = 0.0;
-    for (int c = 0; c < K; ++c) s += Ma[x + (size_t)c * K] * Mb[y + (size_t)c * K];
+    for (int c = 0; c < K; ++c) s += Ra[x + c * K] * Rb[y + c * K];
     Cm[e] = s;
     Cin[e] = s;
   }
   __syncthreads();
   // columns orthogonal to 1e-8 of their norms: far below the FP32 data's
   // rounding once scaled by the eps cut
-  if (wid == 0) {
-    const int c = wave_core_svd(Cm, ra, ra, rb, kGramJacobiTol2, fmax(1e-30, 1e-16 * eps * eps));
-    if (lane == 0) ranks[0] = c;
+  if (ra <= kCoreMax && rb <= kCoreMax) {
+    if (wid == 0) {
+      const int c = wave_core_svd(Cm, ra, ra, rb, kGramJacobiTol2, fmax(1e-30, 1e-16 * eps * eps));
+      const int k = wave_sorted_cut(Cm, ra, ra, c, sig, order, eps);
+      if (lane < c) scale[lane] = 1.0 / sqrt(sig[lane]);
+      if (lane == 0) ranks[2] = k;
+    }
+  } else {
+    jacobi_svd(Cm, ra, ra, rb, lptr<double>(nullptr), rb, nullptr, 40, kGramJacobiTol2);
+    sorted_norms(Cm, ra, ra, rb, sig, order);
+    if (threadIdx.x < rb) scale[threadIdx.x] = 1.0 / sqrt(sig[threadIdx.x]);
+    if (threadIdx.x == 0) ranks[2] = find_k(sig, order, rb, eps);
   }
   __syncthreads();
-  const int rc = ranks[0];
-  sorted_norms(Cm, ra, ra, rc, sig, order);
-  int nk = find_k(sig, order, rc, eps);
+  int nk = ranks[2];
   if (nk > tg.cap) {
     if (threadIdx.x == 0) atomicOr(overflow, 1);
     nk = tg.cap;
   }
-  // left U sqrt(S) (ra x nk) and right V sqrt(S) = Cin^T U / sqrt(S) (rb x nk), ld K
+  // left U sqrt(S) (ra x nk, into Ga) and right V sqrt(S) = Cin^T U / sqrt(S)
+  // (rb x nk, into Gb), ld K
   for (int e = threadIdx.x; e < ra * nk; e += kBlock) {
-    const int x = e % ra, oc = order[e / ra];
-    Ma[x + (size_t)(e / ra) * K] = Cm[x + (size_t)oc * ra] / sqrt(sig[oc]);
+    const int x = e % ra, c = e / ra, oc = order[c];
+    Ga[x + c * K] = Cm[x + oc * ra] * scale[oc];
   }
   for (int e = threadIdx.x; e < rb * nk; e += kBlock) {
-    const int y = e % rb, oc = order[e / rb];
+    const int y = e % rb, c = e / rb, oc = order[c];
     double s = 0.0;
-    for (int x = 0; x < ra; ++x) s += Cin[x + (size_t)y * ra] * Cm[x + (size_t)oc * ra];
-    Mb[y + (size_t)(e / rb) * K] = s / (sig[oc] * sqrt(sig[oc]));
+    for (int x = 0; x < ra; ++x) s += Cin[x + y * ra] * Cm[x + oc * ra];
+    Gb[y + c * K] = s * scale[oc] / sig[oc];
   }
   __syncthreads();
-  // R11^-1 of each side, one column per thread (A: threads 0.., B: 128..)
-  const int half = kBlock / 2;
-  {
-    const bool bside = threadIdx.x >= half;
-    const int c = bside ? threadIdx.x - half : threadIdx.x;
-    const int r = bside ? rb : ra;
-    const lptr<double> R = bside ? Gb : Ga, X = bside ? Mb : Ma;
-    if (c < nk)
-      for (int x = r - 1; x >= 0; --x) {
-        double v = X[x + (size_t)c * K];
-        for (int i = x + 1; i < r; ++i) v -= R[x + (size_t)i * K] * X[i + (size_t)c * K];
-        X[x + (size_t)c * K] = v / R[x + (size_t)x * K];
-      }
+  // P1 R11^-1 of each side into Cm / Cin (K x nk, ld K), one column per thread
+  if (wid < 2 && lane < nk) {
+    const lptr<double> R = wid ? Rb : Ra, inv = wid ? ib : ia;
+    const lptr<double> x = (wid ? Gb : Ga) + lane * K, out = (wid ? Cin : Cm) + lane * K;
+    const lptr<int> piv = wid ? pb : pa;
+    const int r = wid ? rb : ra;
+    if (K <= 16)
+      pchol_solve<16>(R, K, piv, inv, r, x, out);
+    else
+      pchol_solve<kGramMaxK>(R, K, piv, inv, r, x, out);
   }
   __syncthreads();
-  // scatter to panel order (rows piv[i]) into Cm / Cin, K x nk, ld K
-  for (int e = threadIdx.x; e < K * nk; e += kBlock) Cm[e] = Cin[e] = 0.0;
-  __syncthreads();
-  for (int e = threadIdx.x; e < ra * nk; e += kBlock)
-    Cm[pa[e % ra] + (size_t)(e / ra) * K] = Ma[e % ra + (size_t)(e / ra) * K];
-  for (int e = threadIdx.x; e < rb * nk; e += kBlock)
-    Cin[pb[e % rb] + (size_t)(e / rb) * K] = Mb[e % rb + (size_t)(e / rb) * K];
-  __syncthreads();
-  rows_times_small<T>(Va, m, m, K, Cm, K, nk, (gptr<T>)tg.a, tg.la);
-  rows_times_small<T>(Vb, n, n, K, Cin, K, nk, (gptr<T>)tg.b, tg.lb);
+  rows_times_small<T>(Va, lda, m, K, Cm, K, nk, (gptr<T>)tg.a, tg.la);
+  rows_times_small<T>(Vb, ldb, n, K, Cin, K, nk, (gptr<T>)tg.b, tg.lb);
   if (threadIdx.x == 0) *tg.rank = nk;
 }
 
@@ -1664,8 +1774,13 @@ __global__ void __launch_bounds__(kBlock) k_fadd(const FTask* tasks, double* wsb
   const int m = tg.m, n = tg.n;
   const int kt = rank_of(tg);
   int K = kt, np = 0, last = -1;
-  for (int q = 0; q < t.nparts; ++q) {
-    const int kq = rank_of(t.parts[q].rk);
+  // the ranks' loads in flight together
+  int kqs[kMaxParts];
+#pragma unroll
+  for (int q = 0; q < kMaxParts; ++q) kqs[q] = q < t.nparts ? rank_of(t.parts[q].rk) : 0;
+#pragma unroll
+  for (int q = 0; q < kMaxParts; ++q) {
+    const int kq = kqs[q];
     if (kq > 0 && t.parts[q].alpha != 0.0 && t.parts[q].rk.m > 0 && t.parts[q].rk.n > 0) {
       K += kq;
       ++np;
@@ -1737,7 +1852,17 @@ __global__ void __launch_bounds__(kBlock) k_fadd(const FTask* tasks, double* wsb
   }
   if constexpr (sizeof(T) == 4) {
     if (K <= kGramMaxK) {
-      gram_recompress<T>(t, kt, K, gws, (lptr<double>)sh, fabs(t.eps), overflow, &flag);
+      // panels in LDS (odd ld: strided lane accesses spread over the banks) when
+      // they fit beside the small matrices, else in the workspace
+      const int64_t small = gram_lds(K);
+      const auto s3 = (lptr<double>)sh;
+      if (small + (int64_t)((m | 1) + (n | 1)) * K <= kShDoubles) {
+        const lptr<double> Pa = s3 + small, Pb = Pa + (m | 1) * K;
+        gram_recompress<T>(Pa, m | 1, Pb, n | 1, t, kt, K, s3, fabs(t.eps), overflow);
+      } else {
+        const auto Pa = (gptr<double>)gws;
+        gram_recompress<T>(Pa, m, Pa + (size_t)m * K, n, t, kt, K, s3, fabs(t.eps), overflow);
+      }
       return;
     }
   }
@@ -1895,11 +2020,14 @@ __device__ void rkrk_body(const FTask& t, int k1, int k2, P ws, lptr<double> par
       __syncthreads();
       if (threadIdx.x < kWave) {
         const int c = wave_core_svd(G, gr, gr, gc, 1e-26, fmax(1e-30, 1e-16 * t.eps * t.eps));
-        if (threadIdx.x == 0) *flag = c;
+        const int k = wave_sorted_cut(G, gr, gr, c, sig, order, t.eps);
+        if (threadIdx.x == 0) {
+          flag[0] = c;
+          flag[1] = k;
+        }
       }
       __syncthreads();
-      r = *flag;
-      sorted_norms(G, gr, gr, r, sig, order);
+      r = flag[0];
       for (int e = threadIdx.x; e < gc * r; e += kBlock) {
         const int i = e % gc, j = e / gc;
         double s = 0.0;
@@ -1913,7 +2041,7 @@ __device__ void rkrk_body(const FTask& t, int k1, int k2, P ws, lptr<double> par
     jacobi_svd(G, gr, gr, gc, V, gc, flag);
     sorted_norms(G, gr, gr, gc, sig, order);
   }
-  int nk = find_k(sig, order, r, t.eps);
+  int nk = done ? flag[1] : find_k(sig, order, r, t.eps);
   if (nk > out.cap) {
     if (threadIdx.x == 0) atomicOr(overflow, 1);
     nk = out.cap;
@@ -1943,7 +2071,7 @@ __device__ void rkrk_body(const FTask& t, int k1, int k2, P ws, lptr<double> par
 template <typename T>
 __global__ void __launch_bounds__(kBlock) k_rkrk(const FTask* tasks, double* wsbase, int* overflow) {
   __shared__ double sh[kShDoubles];
-  __shared__ int flag;
+  __shared__ int flag[2];
   if (overflow[1]) return;
   const FTask& t = tasks[blockIdx.x];
   const int k1 = rank_of(t.parts[0].rk), k2 = rank_of(t.parts[1].rk);
@@ -1956,9 +2084,9 @@ __global__ void __launch_bounds__(kBlock) k_rkrk(const FTask* tasks, double* wsb
   // SVD scratch, then the output factors (at most (gr + gc) x gc)
   const auto s3 = (lptr<double>)sh;
   if (need + (int64_t)(gr + gc) * gc + (int64_t)gr * gc <= kShDoubles)
-    rkrk_body<T, lptr<double>, lptr<int>>(t, k1, k2, s3, s3 + need, kShDoubles - need, overflow, &flag);
+    rkrk_body<T, lptr<double>, lptr<int>>(t, k1, k2, s3, s3 + need, kShDoubles - need, overflow, flag);
   else
-    rkrk_body<T, gptr<double>, gptr<int>>(t, k1, k2, (gptr<double>)(wsbase + t.ws), s3, kShDoubles, overflow, &flag);
+    rkrk_body<T, gptr<double>, gptr<int>>(t, k1, k2, (gptr<double>)(wsbase + t.ws), s3, kShDoubles, overflow, flag);
 }
 
 // ---------------------------------------------------------------------------

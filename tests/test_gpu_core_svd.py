@@ -1,5 +1,6 @@
 """Core SVD of the recompressions on one wavefront (FADD and RKRK) at the edges
-of its register forms (16, 24 and 32 columns) and just above, with cores that
+of its register forms (16, 24 and 32 columns) and above (FADD of 40 and 41
+columns, where the FP32 Gram form ends), with cores that
 are rectangular, rank deficient, zero or of one column, against numpy's
 truncated SVD.  The singular values fall by 0.6 a step, so the cut at eps has a
 relative gap of 0.4 and the truncated matrix moves by a few K u / 0.4 of its
@@ -48,7 +49,7 @@ def test_fadd_core_sizes(fp32):
                                (99, 65, 8, 8, "full"), (99, 65, 8, 9, "full"), (99, 65, 12, 12, "full"),
                                (99, 65, 12, 13, "full"), (99, 65, 16, 15, "full"), (130, 140, 16, 16, "full"),
                                (130, 140, 16, 17, "full"), (130, 140, 20, 20, "full"), (700, 900, 9, 8, "full"),
-                               (700, 900, 16, 16, "full"), (70, 90, 6, 6, "same"), (700, 900, 14, 14, "same"),
+                               (700, 900, 16, 16, "full"), (900, 800, 18, 21, "full"), (130, 140, 20, 21, "full"), (70, 90, 6, 6, "same"), (700, 900, 14, 14, "same"),
                                (70, 90, 5, 5, "zero")]:
         ta, tb = _rk(rng, m, n, kt, fp32)
         pa, pb = _rk(rng, m, n, kp, fp32)
