@@ -52,7 +52,12 @@ __device__ __forceinline__ void static_for(F f) {
 }
 
 // ---------------------------------------------------------------------------
-// GEMM: C (m x n, ldc) = beta C + alpha op(A) op(B), 64 x 64 tiles.
+// GEMM: C (m x n, ldc) = beta C + alpha op(A) op(B), 64 x 64 tiles.  Bound in the
+// factorisation's launches (98-row leaves, some 200 tiles): latency, of the
+// flag, tile, task and operands and then of each k-step.  With C read entry by
+// entry after the products, its columns across the lanes, and transposed
+// operands gathered, a launch averaged 13.0 us (40,000 points, FP32) and 16.3 us
+// (8,000 points), now 10.8 and 12.4 us.
 // ---------------------------------------------------------------------------
 constexpr int TM = 64, TN = 64, TK = 32;
 
@@ -61,18 +66,18 @@ __global__ void __launch_bounds__(256) k_gemm(const FTask* tasks, const GemmTile
                                               const int* fail) {
   __shared__ T As[TK][TM + 1];
   __shared__ T Bs[TK][TN + 1];
-  if (*fail) return;
+  const int failed = *fail;  // in flight together with the tile and the task
   const GemmTile tl = tiles[blockIdx.x];
   const FTask& t = tasks[tl.task];
   const int M = eff(t.m), N = eff(t.n), P = eff(t.p);
   const int i0 = tl.tm * TM, j0 = tl.tn * TN;
-  if (i0 >= M || j0 >= N) return;
+  if ((failed != 0) | (i0 >= M) | (j0 >= N)) return;
   const auto A = (cgptr<T>)t.A;
   const auto B = (cgptr<T>)t.B;
   const auto C = (gptr<T>)t.C;
   // wavefront w computes the 32 x 32 quadrant (w & 1, w >> 1) of the tile as
-  // 2 x 2 matrix-core tiles of 16 x 16: A[i][k] comes from lane i + 16 k,
-  // B[k][j] from lane j + 16 k (inner dimension 4 per instruction)
+  // 2 x 2 matrix-core tiles of 16 x 16, transposed (op(B)^T is the A operand), so
+  // that 16 lanes hold 16 rows of a column of C
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const int li = lane & 15, lk = lane >> 4;
   const int qi = (w & 1) * 32, qj = (w >> 1) * 32;
@@ -84,33 +89,59 @@ __global__ void __launch_bounds__(256) k_gemm(const FTask* tasks, const GemmTile
     for (int b = 0; b < 2; ++b) acc[a][b] = Acc{0, 0, 0, 0};
   // As[kk][ii] = op(A)(i0 + ii, k0 + kk), Bs[kk][jj] = op(B)(k0 + kk, j0 + jj):
   // each thread loads 8 + 8 entries of a k-step into registers; the loads of
-  // step k0 + TK are in flight while step k0 is multiplied
+  // step k0 + TK are in flight while step k0 is multiplied (two steps ahead cost
+  // a wavefront per SIMD and made large launches 2.5 times slower).  Consecutive lanes
+  // take consecutive addresses: rows of the tile, or its k when the stored
+  // matrix is the transpose.  The loads read a clamped entry and select.
   constexpr int kPer = TM * TK / 256;
+  const int mi = M - i0 < TM ? M - i0 : TM, nj = N - j0 < TN ? N - j0 : TN;
+  const bool ka = t.ta, kb = !t.tb;  // k runs along the lanes
+  const int ia = ka ? threadIdx.x / TK : threadIdx.x % TM, ja = ka ? threadIdx.x % TK : threadIdx.x / TM;
+  const int ib = kb ? threadIdx.x / TK : threadIdx.x % TN, jb = kb ? threadIdx.x % TK : threadIdx.x / TN;
+  const int dia = ka ? 256 / TK : 0, dja = ka ? 0 : 256 / TM;
+  const int dib = kb ? 256 / TK : 0, djb = kb ? 0 : 256 / TN;
   const long la = t.lda, lb = t.ldb;
+  const long sia = ka ? la : 1, ska = ka ? 1 : la, sib = kb ? lb : 1, skb = kb ? 1 : lb;
+  const auto A0 = A + i0 * sia;
+  const auto B0 = B + j0 * sib;
   T ra[kPer], rb[kPer];
-  auto load_step = [&](int k0) {
+  auto load_step = [&](int k0) __attribute__((always_inline)) {
+    const int pk = P - k0 < TK ? P - k0 : TK;
+    const auto Ak = A0 + k0 * ska;
+    const auto Bk = B0 + k0 * skb;
 #pragma unroll
     for (int u = 0; u < kPer; ++u) {
-      const int e = threadIdx.x + 256 * u, i = e % TM, j = e / TM;
-      const bool ok = i < M - i0 && j < P - k0;
-      ra[u] = ok ? A[t.ta ? (size_t)(k0 + j) + (size_t)(i0 + i) * la : (size_t)(i0 + i) + (size_t)(k0 + j) * la]
-                 : (T)0;
+      const int i = ia + u * dia, j = ja + u * dja;
+      ra[u] = Ak[(i < mi ? i : mi - 1) * sia + (j < pk ? j : pk - 1) * ska];
     }
 #pragma unroll
     for (int u = 0; u < kPer; ++u) {
-      const int e = threadIdx.x + 256 * u, i = e % TN, j = e / TN;
-      const bool ok = i < N - j0 && j < P - k0;
-      rb[u] = ok ? B[t.tb ? (size_t)(j0 + i) + (size_t)(k0 + j) * lb : (size_t)(k0 + j) + (size_t)(j0 + i) * lb]
-                 : (T)0;
+      const int i = ib + u * dib, j = jb + u * djb;
+      rb[u] = Bk[(i < nj ? i : nj - 1) * sib + (j < pk ? j : pk - 1) * skb];
     }
   };
-  load_step(0);
+  if (P > 0) load_step(0);
+  // C is in flight during the products
+  const auto C0 = C + i0 + (size_t)j0 * t.ldc;
+  const bool add = t.mode != 0;
+  T old[2][2][4];
+  if (add) {
+#pragma unroll
+    for (int a = 0; a < 2; ++a)
+#pragma unroll
+      for (int b = 0; b < 2; ++b)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          const int i = qi + 16 * a + li, j = qj + 16 * b + MfmaAcc<T>::row(lane, v);
+          old[a][b][v] = C0[(i < mi ? i : mi - 1) + (size_t)(j < nj ? j : nj - 1) * t.ldc];
+        }
+  }
   for (int k0 = 0; k0 < P; k0 += TK) {
 #pragma unroll
     for (int u = 0; u < kPer; ++u) {
-      const int e = threadIdx.x + 256 * u;
-      As[e / TM][e % TM] = ra[u];
-      Bs[e / TN][e % TN] = rb[u];
+      const int i = ia + u * dia, j = ja + u * dja, ii = ib + u * dib, jj = jb + u * djb;
+      As[j][i] = i < mi && k0 + j < P ? ra[u] : (T)0;
+      Bs[jj][ii] = ii < nj && k0 + jj < P ? rb[u] : (T)0;
     }
     __syncthreads();
     if (k0 + TK < P) load_step(k0 + TK);
@@ -124,7 +155,7 @@ __global__ void __launch_bounds__(256) k_gemm(const FTask* tasks, const GemmTile
 #pragma unroll
       for (int a = 0; a < 2; ++a)
 #pragma unroll
-        for (int b = 0; b < 2; ++b) acc[a][b] = mfma16x16x4(fa[a], fb[b], acc[a][b]);
+        for (int b = 0; b < 2; ++b) acc[a][b] = mfma16x16x4(fb[b], fa[a], acc[a][b]);
     }
     __syncthreads();
   }
@@ -135,10 +166,9 @@ __global__ void __launch_bounds__(256) k_gemm(const FTask* tasks, const GemmTile
     for (int b = 0; b < 2; ++b)
 #pragma unroll
       for (int v = 0; v < 4; ++v) {
-        const int i = i0 + qi + 16 * a + MfmaAcc<T>::row(lane, v), j = j0 + qj + 16 * b + li;
-        if (i >= M || j >= N) continue;
-        const auto pc = C + i + (size_t)j * t.ldc;
-        *pc = t.mode ? *pc + alpha * acc[a][b][v] : alpha * acc[a][b][v];
+        const int i = qi + 16 * a + li, j = qj + 16 * b + MfmaAcc<T>::row(lane, v);
+        const T x = alpha * acc[a][b][v];
+        if (i < mi && j < nj) C0[i + (size_t)j * t.ldc] = add ? old[a][b][v] + x : x;
       }
 }
 
