@@ -1200,10 +1200,10 @@ int hmx_run_tasks(int precision, int type, const void* tasks, int count, int* fl
         need = hmx::hodlr_workspace(x.lda);
       }
       x.type = type;
-      hmx::append_tiles(x, i, tiles);
       x.ws = ws;
       ws += need;
     }
+    hmx::append_tiles(t.data(), count, tiles);
     hipStream_t s = nullptr;
     HMX_CHECK(hipStreamCreateWithFlags(&s, hipStreamNonBlocking));
     struct StreamGuard {

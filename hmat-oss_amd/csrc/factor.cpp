@@ -2402,10 +2402,10 @@ class Exec {
         t.ws = ws;
         ws += need;
         sorted[i] = t;
-        append_tiles(t, (int)i - L.first, tiles);
         ++L.count;
         ++i;
       }
+      append_tiles(sorted.data() + L.first, L.count, tiles);
       L.tcount = (int)tiles.size() - L.tfirst;
       // workspace after the other launches of the wave, so that they can run
       // side by side; a launch that would exceed the budget runs alone

@@ -22,12 +22,12 @@ int64_t hodlr_workspace(int cap);
 void launch_fill_int(int* p, size_t n, int v, hipStream_t s);
 
 // The work items of the types that cut a task into tiles, one workgroup each:
-// 64 x 64 tiles of C (GEMM), slabs of independent rows / columns (TRSM), runs
-// of entries (ZERO, AXPY, SUMK).  append_tiles adds those of a task (by its
-// static sizes; a tile past a dynamic size returns at once), task 'index' of
-// its launch.
+// tiles of C (GEMM: 64 x 64, or 32 x 32 where the launch leaves the chip idle),
+// slabs of independent rows / columns (TRSM), runs of entries (ZERO, AXPY, SUMK).
+// append_tiles adds those of a launch's tasks, all of one type (by their static
+// sizes; a tile past a dynamic size returns at once).
 bool task_has_tiles(int type);
-void append_tiles(const FTask& t, int index, std::vector<GemmTile>& tiles);
+void append_tiles(const FTask* tasks, int count, std::vector<GemmTile>& tiles);
 
 // One batched launch of 'count' tasks of 'type' ('ntiles' tiles where the
 // type has tiles).

@@ -88,7 +88,7 @@ struct FTask {
 
 struct GemmTile {
   int task;
-  int tm, tn;
+  int tm, tn;        // GEMM: tm = ~row of the tile for 32 x 32 tiles
 };
 
 }  // namespace hmx

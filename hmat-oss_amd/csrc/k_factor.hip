@@ -60,18 +60,139 @@ __device__ __forceinline__ void static_for(F f) {
 // (8,000 points), now 10.8 and 12.4 us.
 // ---------------------------------------------------------------------------
 constexpr int TM = 64, TN = 64, TK = 32;
+static_assert(TM == TN, "one tile side");
+
+// Products with a side of at most 32 (the right-hand sides of a solve, a rank) or
+// all of a leaf's size, in launches of few tiles, are bound by the latency of
+// their loads: a workgroup takes a 32 x 32 tile, its wavefronts a quarter of the
+// inner dimension each with 32 or 64 steps' operands in flight straight into the
+// matrix-core layout, and the four partial tiles meet in LDS.  Larger products
+// and launches share operands through LDS (k_gemm's 64 x 64 tiles).
+// Where the line lies, 64 x 64 tiles against these, by the launch's number of
+// 64 x 64 tiles: up to 16 9.8 against 5.3 us (6,000 points, FP64), 65 to 128
+// 10.2 against 6.9 us, 513 to 1,024 17.6 against 15.1 us, 1,025 to 2,048 24.4
+// against 27.6 us, above 4,096 71 against 142 us (40,000 points, FP32).
+constexpr int kThin = 32, kThinSide = 256, kThinLaunch = 1024;
+inline bool gemm_is_thin(const FTask& t) {
+  const int m = t.m.s, n = t.n.s;
+  return m <= kThin || n <= kThin || (m <= kThinSide && n <= kThinSide && t.p.s <= kThinSide);
+}
+
+// sh: 4096 entries
+template <typename T>
+__device__ __forceinline__ void gemm_thin(const FTask& t, int i0, int j0, int M, int N, int P, T* sh) {
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int li = lane & 15, lk = lane >> 4;
+  const long sia = t.ta ? (long)t.lda : 1L, ska = t.ta ? 1L : (long)t.lda;
+  const long sib = t.tb ? 1L : (long)t.ldb, skb = t.tb ? (long)t.ldb : 1L;
+  const int mi = M - i0 < kThin ? M - i0 : kThin, nj = N - j0 < kThin ? N - j0 : kThin;
+  const bool two_a = mi > 16, two_b = nj > 16;
+  cgptr<T> pa[2], pb[2];
+#pragma unroll
+  for (int a = 0; a < 2; ++a) {
+    const int i = 16 * a + li;
+    pa[a] = (cgptr<T>)t.A + (i0 + (i < mi ? i : mi - 1)) * sia;
+    pb[a] = (cgptr<T>)t.B + (j0 + (i < nj ? i : nj - 1)) * sib;
+  }
+  // thread (w, lane) finishes entry (16 a + li, 16 b + row(lane, w)) of each 16 x 16
+  // tile: C in flight during the products
+  const auto C0 = (gptr<T>)t.C + i0 + (size_t)j0 * t.ldc;
+  const bool add = t.mode != 0;
+  const int jr = MfmaAcc<T>::row(lane, w);
+  T old[2][2];
+  if (add) {
+#pragma unroll
+    for (int a = 0; a < 2; ++a)
+#pragma unroll
+      for (int b = 0; b < 2; ++b) {
+        const int i = 16 * a + li, j = 16 * b + jr;
+        old[a][b] = C0[(i < mi ? i : mi - 1) + (size_t)(j < nj ? j : nj - 1) * t.ldc];
+      }
+  }
+  using Acc = typename MfmaAcc<T>::type;
+  Acc acc[2][2];
+#pragma unroll
+  for (int a = 0; a < 2; ++a)
+#pragma unroll
+    for (int b = 0; b < 2; ++b) acc[a][b] = Acc{0, 0, 0, 0};
+  // lane group lk takes the inner indices 16 s + 4 lk + e, e = 0..3: a lane's four
+  // loads are neighbours where the inner index runs along memory
+  constexpr int kB = sizeof(T) == 4 ? 4 : 2;  // groups of 16 in flight
+  const int chunk = (P + 63) / 64 * 16;
+  const int lo = w * chunk, hi = lo + chunk < P ? lo + chunk : P;
+  for (int k0 = lo; k0 < hi; k0 += 16 * kB) {
+    T fa[2][4 * kB], fb[2][4 * kB];
+#pragma unroll
+    for (int q = 0; q < 4 * kB; ++q) {
+      const int k = k0 + 16 * (q / 4) + 4 * lk + q % 4, kc = k < hi ? k : hi - 1;
+      fa[0][q] = pa[0][kc * ska];
+      fb[0][q] = pb[0][kc * skb];
+    }
+    if (two_a) {
+#pragma unroll
+      for (int q = 0; q < 4 * kB; ++q) {
+        const int k = k0 + 16 * (q / 4) + 4 * lk + q % 4;
+        fa[1][q] = pa[1][(k < hi ? k : hi - 1) * ska];
+      }
+    }
+    if (two_b) {
+#pragma unroll
+      for (int q = 0; q < 4 * kB; ++q) {
+        const int k = k0 + 16 * (q / 4) + 4 * lk + q % 4;
+        fb[1][q] = pb[1][(k < hi ? k : hi - 1) * skb];
+      }
+    }
+#pragma unroll
+    for (int q = 0; q < 4 * kB; ++q) {
+      const bool in = k0 + 16 * (q / 4) + 4 * lk + q % 4 < hi;
+      const T a0 = in ? fa[0][q] : (T)0, b0 = in ? fb[0][q] : (T)0;
+      acc[0][0] = mfma16x16x4(b0, a0, acc[0][0]);
+      if (two_a) acc[1][0] = mfma16x16x4(b0, in ? fa[1][q] : (T)0, acc[1][0]);
+      if (two_b) {
+        const T b1 = in ? fb[1][q] : (T)0;
+        acc[0][1] = mfma16x16x4(b1, a0, acc[0][1]);
+        if (two_a) acc[1][1] = mfma16x16x4(b1, in ? fa[1][q] : (T)0, acc[1][1]);
+      }
+    }
+  }
+#pragma unroll
+  for (int a = 0; a < 2; ++a)
+#pragma unroll
+    for (int b = 0; b < 2; ++b)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) sh[((w * 2 + a) * 2 + b) * 256 + v * 64 + lane] = acc[a][b][v];
+  __syncthreads();
+  const T alpha = (T)t.alpha;
+#pragma unroll
+  for (int a = 0; a < 2; ++a)
+#pragma unroll
+    for (int b = 0; b < 2; ++b) {
+      T x = (T)0;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) x += sh[((q * 2 + a) * 2 + b) * 256 + threadIdx.x];
+      x *= alpha;
+      const int i = 16 * a + li, j = 16 * b + jr;
+      if (i < mi && j < nj) C0[i + (size_t)j * t.ldc] = add ? old[a][b] + x : x;
+    }
+}
 
 template <typename T>
 __global__ void __launch_bounds__(256) k_gemm(const FTask* tasks, const GemmTile* tiles,
                                               const int* fail) {
-  __shared__ T As[TK][TM + 1];
-  __shared__ T Bs[TK][TN + 1];
+  __shared__ T sh[2 * TK * (TM + 1)];
+  auto& As = *(T(*)[TK][TM + 1])sh;
+  auto& Bs = *(T(*)[TK][TN + 1])(sh + TK * (TM + 1));
   const int failed = *fail;  // in flight together with the tile and the task
   const GemmTile tl = tiles[blockIdx.x];
   const FTask& t = tasks[tl.task];
   const int M = eff(t.m), N = eff(t.n), P = eff(t.p);
-  const int i0 = tl.tm * TM, j0 = tl.tn * TN;
+  const bool thin = tl.tm < 0;
+  const int i0 = thin ? ~tl.tm * kThin : tl.tm * TM, j0 = tl.tn * (thin ? kThin : TN);
   if ((failed != 0) | (i0 >= M) | (j0 >= N)) return;
+  if (thin) {
+    gemm_thin<T>(t, i0, j0, M, N, P, sh);
+    return;
+  }
   const auto A = (cgptr<T>)t.A;
   const auto B = (cgptr<T>)t.B;
   const auto C = (gptr<T>)t.C;
@@ -2293,24 +2414,34 @@ __global__ void __launch_bounds__(kBlock) k_acafull(const FTask* tasks, const in
 bool task_has_tiles(int type) {
   return type == T_GEMM || type == T_TRSM || type == T_ZERO || type == T_AXPY || type == T_SUMK;
 }
-void append_tiles(const FTask& t, int index, std::vector<GemmTile>& tiles) {
-  switch (t.type) {
-    case T_GEMM:
-      for (int a = 0; a < (t.m.s + TM - 1) / TM; ++a)
-        for (int b = 0; b < (t.n.s + TN - 1) / TN; ++b) tiles.push_back(GemmTile{index, a, b});
-      break;
-    case T_TRSM:
-      for (int a = 0; a < (t.m.s + kTrsmCols - 1) / kTrsmCols; ++a) tiles.push_back(GemmTile{index, a, 0});
-      break;
-    case T_ZERO:
-    case T_AXPY:
-    case T_SUMK: {
-      const int64_t e = (int64_t)t.m.s * t.n.s;
-      for (int64_t a = 0; a * kElemsPerTile < e; ++a) tiles.push_back(GemmTile{index, (int)a, 0});
-      break;
+void append_tiles(const FTask* tasks, int count, std::vector<GemmTile>& tiles) {
+  if (count == 0 || !task_has_tiles(tasks[0].type)) return;
+  auto parts = [](int n, int side) { return (n + side - 1) / side; };
+  bool few = false;
+  if (tasks[0].type == T_GEMM) {
+    int64_t wide = 0;
+    for (int q = 0; q < count; ++q) wide += (int64_t)parts(tasks[q].m.s, TM) * parts(tasks[q].n.s, TN);
+    few = wide <= kThinLaunch;
+  }
+  for (int q = 0; q < count; ++q) {
+    const FTask& t = tasks[q];
+    switch (t.type) {
+      case T_GEMM: {
+        const bool thin = few && gemm_is_thin(t);
+        const int side = thin ? kThin : TM;
+        for (int a = 0; a < parts(t.m.s, side); ++a)
+          for (int b = 0; b < parts(t.n.s, side); ++b) tiles.push_back(GemmTile{q, thin ? ~a : a, b});
+        break;
+      }
+      case T_TRSM:
+        for (int a = 0; a < parts(t.m.s, kTrsmCols); ++a) tiles.push_back(GemmTile{q, a, 0});
+        break;
+      default: {  // T_ZERO, T_AXPY, T_SUMK
+        const int64_t e = (int64_t)t.m.s * t.n.s;
+        for (int64_t a = 0; a * kElemsPerTile < e; ++a) tiles.push_back(GemmTile{q, (int)a, 0});
+        break;
+      }
     }
-    default:
-      break;
   }
 }
 

@@ -225,7 +225,7 @@ void SweepSolver::ensure_inverse(const Store<T>& st, hipStream_t s) {
   }
   put(trsm_tasks_, tasks, s);
   std::vector<GemmTile> tiles;
-  for (int q = 0; q < nrows_; ++q) append_tiles(tasks[q], q, tiles);
+  append_tiles(tasks.data(), nrows_, tiles);
   put(trsm_tiles_, tiles, s);
   launch_task_kernel<T>(T_TRSM, trsm_tasks_.as<FTask>(), nrows_, trsm_tiles_.as<GemmTile>(),
                         (int)tiles.size(), nullptr, flags_.as<int>(), s);
