@@ -1031,6 +1031,10 @@ constexpr int kShDoubles = 18432;  // 144 KiB of LDS per workgroup, beside the c
 // of 125 rows, inverses of its 2,000-row diagonal blocks for the solve) went
 // from 138.9 to 24.4 ms with this, the tiles of the elementwise tasks and the
 // skipped zero half of the inverses.
+// With the masks and the conversion at the use and not at the load (which made
+// every load wait), the interchanges followed backwards and the diagonal's loads
+// together, an average launch went from 32.4 to 18.3 us (94 rows, FP64, with
+// interchanges), 29 to 20 us (125 rows, FP32) and 16 to 12.8 us (78 rows, FP32).
 constexpr int kTrsmBlocks = 8;              // blocks solved in registers at a time
 constexpr int kTrsmInvLd = kNb * kNb + 8;   // diagonal blocks in LDS: spread over the banks
 
@@ -1047,11 +1051,11 @@ __global__ void __launch_bounds__(kBlock) k_trsm(const FTask* tasks, const GemmT
   __shared__ double rdiag[kTrsmBlocks * kNb];
   __shared__ int perm[kTrsmBlocks * kNb];
   constexpr int NB = kTrsmBlocks;
-  if (*fail) return;
+  const int failed = *fail;  // in flight together with the tile and the task
   const GemmTile tl = tiles[blockIdx.x];
   const FTask& t = tasks[tl.task];
   const int other = eff(t.m), col0 = tl.tm * kTrsmCols, n = t.n.s;
-  if (col0 >= other || n <= 0) return;
+  if ((failed != 0) | (col0 >= other) | (n <= 0)) return;
   const int nb = (n + kNb - 1) / kNb;
   const int mode = t.mode & kTrsmBase;
   const bool transa = (t.mode & kTrsmTransA) != 0, unit = (t.mode & kTrsmUnit) != 0;
@@ -1070,37 +1074,27 @@ __global__ void __launch_bounds__(kBlock) k_trsm(const FTask* tasks, const GemmT
   const auto Xc = X + (mode == 0 ? (size_t)jc : (size_t)jc * t.ldc);
   const bool permuted = pivot && nb <= NB;
   if (permuted && w == 0) {
-    // the interchanges as one permutation, rows lane + 64 q in registers
+    // the interchanges as one permutation: the lane follows the content of rows
+    // lane + 64 q back through them (steps of two compares, no chain of exchanges)
     const auto piv = (cgptr<int>)t.B;
     constexpr int kQ = NB / 4;
-    int pr[kQ], pv[kQ];
+    int src[kQ], pv[kQ];
 #pragma unroll
     for (int q = 0; q < kQ; ++q) {
       const int r = lane + kWave * q;
-      pr[q] = r;
+      src[q] = r;
       const int p = piv[r < n ? r : n - 1];
       pv[q] = p < 0 ? 0 : (p >= n ? n - 1 : p);
     }
-    auto at = [](const int (&v)[kQ], int i) __attribute__((always_inline)) {
-      int x = 0;
 #pragma unroll
-      for (int q = 0; q < kQ; ++q) {
-        const int y = __builtin_amdgcn_readlane(v[q], i & (kWave - 1));
-        x = (i >> 6) == q ? y : x;
+    for (int h = kQ - 1; h >= 0; --h)
+      for (int i = (n - kWave * h < kWave ? n - kWave * h : kWave) - 1; i >= 0; --i) {
+        const int p = __builtin_amdgcn_readlane(pv[h], i), g = i + kWave * h;
+#pragma unroll
+        for (int q = 0; q < kQ; ++q) src[q] = src[q] == g ? p : (src[q] == p ? g : src[q]);
       }
-      return x;
-    };
-    for (int i = 0; i < n; ++i) {
-      const int p = at(pv, i);
-      const int a = at(pr, i), b = at(pr, p);
 #pragma unroll
-      for (int q = 0; q < kQ; ++q) {
-        const int r = lane + kWave * q;
-        pr[q] = r == i ? b : (r == p ? a : pr[q]);
-      }
-    }
-#pragma unroll
-    for (int q = 0; q < kQ; ++q) perm[lane + kWave * q] = pr[q];
+    for (int q = 0; q < kQ; ++q) perm[lane + kWave * q] = src[q];
   } else if (pivot && !permuted) {
     // wide leaves: each thread replays the interchanges on its own column
     const auto piv = (cgptr<int>)t.B;
@@ -1122,13 +1116,23 @@ __global__ void __launch_bounds__(kBlock) k_trsm(const FTask* tasks, const GemmT
     auto block_of = [&](int p) { return back ? nb - 1 - p : p; };
     __syncthreads();
     // the diagonal blocks (lower triangles) and the reciprocals of the diagonal
-    for (int e = threadIdx.x; e < np * kNb * kNb; e += kBlock) {
-      const int q = e / (kNb * kNb), r = e % kNb, l = e / kNb % kNb;
-      const int gr = block_of(p0 + q) * kNb + r, gl = gr - r + l;
-      const bool in = gr < n && l <= r;
-      const double v = (double)Lg[(gr < n ? gr : n - 1) * li + (gl < n ? gl : n - 1) * lk];
-      inv[q * kTrsmInvLd + r + l * kNb] = in ? v : 0.0;
-      if (r == l) rdiag[q * kNb + r] = (unit || !in) ? 1.0 : 1.0 / v;
+    {
+      static_assert(kNb * kNb == kBlock, "an entry of each block per thread");
+      const int r = threadIdx.x % kNb, l = threadIdx.x / kNb;
+      T v[NB];
+#pragma unroll
+      for (int q = 0; q < NB; ++q) {
+        const int gr = block_of(p0 + (q < np ? q : np - 1)) * kNb + r, gl = gr - r + l;
+        v[q] = Lg[(gr < n ? gr : n - 1) * li + (gl < n ? gl : n - 1) * lk];
+      }
+#pragma unroll
+      for (int q = 0; q < NB; ++q) {
+        if (q >= np) break;
+        const int gr = block_of(p0 + q) * kNb + r;
+        const bool in = gr < n && l <= r;
+        inv[q * kTrsmInvLd + r + l * kNb] = in ? (double)v[q] : 0.0;
+        if (r == l) rdiag[q * kNb + r] = (unit || !in) ? 1.0 : 1.0 / (double)v[q];
+      }
     }
     __syncthreads();
     // thread (q, c): column c of the inverse of block q by forward
@@ -1157,17 +1161,41 @@ __global__ void __launch_bounds__(kBlock) k_trsm(const FTask* tasks, const GemmT
     }
     __syncthreads();
     if (!mine) continue;
-    hmx_double4 x[NB];
+    // (all loads of X and of the operand blocks issue before anything waits for
+    // one: the conversion and the masks come at the use)
+    T xin[NB][4];
 #pragma unroll
     for (int p = 0; p < NB; ++p) {
-      if (p >= np) continue;
-      const int r0 = kNb * block_of(p0 + p);
+      const int r0 = kNb * block_of(p0 + (p < np ? p : np - 1));
 #pragma unroll
       for (int v = 0; v < 4; ++v) {
         const int r = r0 + kk + 4 * v, rc = r < n ? r : n - 1;
-        const double y = (double)Xc[(permuted ? perm[rc] : rc) * xr];
-        x[p][v] = r < n ? y : 0.0;
+        xin[p][v] = Xc[(permuted ? perm[rc] : rc) * xr];
       }
+    }
+    // operand blocks in the order in which they are used, (1, 0), (2, 0),
+    // (2, 1), ...: kAhead of them in flight.  Past the last row they repeat it: such
+    // inner indices meet zeros of x, and such rows of the sum are cleared.
+    constexpr int kAhead = 8, kPairs = NB * (NB - 1) / 2;
+    T a[kAhead][4];
+    auto load_block = [&](auto S) __attribute__((always_inline)) {
+      constexpr int s = decltype(S)::value, p = trsm_pair_row(s), c = s - p * (p - 1) / 2;
+      if (p >= np) return;
+      const int r = kNb * block_of(p0 + p) + ii, rc = r < n ? r : n - 1;
+      const int k0 = kNb * block_of(p0 + c) + kk;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int k = k0 + 4 * q, kc = k < n ? k : n - 1;
+        a[s % kAhead][q] = Lg[rc * ai + kc * ak];
+      }
+    };
+    static_for<0, kAhead < kPairs ? kAhead : kPairs>(load_block);
+    hmx_double4 x[NB];
+#pragma unroll
+    for (int p = 0; p < NB; ++p) {
+      const int r0 = kNb * block_of(p0 + p) + kk;
+#pragma unroll
+      for (int v = 0; v < 4; ++v) x[p][v] = p < np && r0 + 4 * v < n ? (double)xin[p][v] : 0.0;
     }
     // the blocks solved before these eight
     for (int c = 0; c < p0; ++c) {
@@ -1190,23 +1218,6 @@ __global__ void __launch_bounds__(kBlock) k_trsm(const FTask* tasks, const GemmT
 #pragma unroll
         for (int q = 0; q < 4; ++q) x[p] = __builtin_amdgcn_mfma_f64_16x16x4f64(as[p][q], xs[q], x[p], 0, 0, 0);
     }
-    // operand blocks in the order in which they are used, (1, 0), (2, 0),
-    // (2, 1), ...: kAhead of them in flight
-    constexpr int kAhead = 8, kPairs = NB * (NB - 1) / 2;
-    double a[kAhead][4];
-    auto load_block = [&](auto S) __attribute__((always_inline)) {
-      constexpr int s = decltype(S)::value, p = trsm_pair_row(s), c = s - p * (p - 1) / 2;
-      if (p >= np) return;
-      const int r = kNb * block_of(p0 + p) + ii, rc = r < n ? r : n - 1;
-      const int k0 = kNb * block_of(p0 + c) + kk;
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const int k = k0 + 4 * q, kc = k < n ? k : n - 1;
-        const double v = (double)Lg[rc * ai + kc * ak];
-        a[s % kAhead][q] = (r < n && k < n) ? v : 0.0;
-      }
-    };
-    static_for<0, kAhead < kPairs ? kAhead : kPairs>(load_block);
     static_for<0, NB>([&](auto P) __attribute__((always_inline)) {
       constexpr int p = decltype(P)::value;
       if (p >= np) return;
@@ -1217,18 +1228,18 @@ __global__ void __launch_bounds__(kBlock) k_trsm(const FTask* tasks, const GemmT
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
           if constexpr (c & 1)
-            s1 = __builtin_amdgcn_mfma_f64_16x16x4f64(a[s % kAhead][q], x[c][q], s1, 0, 0, 0);
+            s1 = __builtin_amdgcn_mfma_f64_16x16x4f64((double)a[s % kAhead][q], x[c][q], s1, 0, 0, 0);
           else
-            s0 = __builtin_amdgcn_mfma_f64_16x16x4f64(a[s % kAhead][q], x[c][q], s0, 0, 0, 0);
+            s0 = __builtin_amdgcn_mfma_f64_16x16x4f64((double)a[s % kAhead][q], x[c][q], s0, 0, 0, 0);
         }
         if constexpr (s + kAhead < kPairs) load_block(std::integral_constant<int, s + kAhead>{});
       });
+      const int r0 = kNb * block_of(p0 + p) + kk;
       const double* blk = inv + p * kTrsmInvLd;
       hmx_double4 y = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
       for (int q = 0; q < 4; ++q)
-        y = __builtin_amdgcn_mfma_f64_16x16x4f64(blk[q * kWave + lane], s0[q] + s1[q], y, 0, 0, 0);
-      const int r0 = kNb * block_of(p0 + p) + kk;
+        y = __builtin_amdgcn_mfma_f64_16x16x4f64(blk[q * kWave + lane], r0 + 4 * q < n ? s0[q] + s1[q] : 0.0, y, 0, 0, 0);
 #pragma unroll
       for (int v = 0; v < 4; ++v) {
         if (r0 + 4 * v < n && j < other) Xc[(r0 + 4 * v) * xr] = (T)y[v];
