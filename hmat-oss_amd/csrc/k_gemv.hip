@@ -295,10 +295,17 @@ __global__ void __launch_bounds__(kBlock) k_ypass1(const int* ranks, const T* ar
   for (int v = 0; v < kYv; ++v) {
     const int i = lane + kWave * v;
     row[v] = i < it.len ? i : it.len - 1;
-    const double t = (double)x[it.x0 + row[v]];
-    xi[v] = (it.mirrored && i < it.len) ? t : 0.0;
+    xi[v] = 0.0;
     acc[v] = 0.0;
   }
+  // x_I of mirrored leaves: the rows' numbering is x's in symmetric storage
+  // only (with other column trees it may reach past x)
+  if (it.mirrored)
+#pragma unroll
+    for (int v = 0; v < kYv; ++v) {
+      const double t = (double)x[it.x0 + row[v]];
+      xi[v] = lane + kWave * v < it.len ? t : 0.0;
+    }
   constexpr int kC = 8;  // columns in flight
   const int cnt = it.end - it.beg;
   for (int u0 = w; u0 < cnt; u0 += kWaves * kWave) {

@@ -50,3 +50,54 @@ def test_gemv_ranges(n, leaf, sym, vt, height):
         assert (np.abs(y.double().cpu().numpy().T - want) <= bound).all(), nrhs
     print(f"gemv ranges n={n} leaf={leaf}", flush=True)
     h.close()
+
+
+@pytest.mark.parametrize("rows,cols", [(1500, 200), (200, 1500), (130, 129), (700, 110)])
+def test_gemv_two_trees(rows, cols):
+    """Different row and column trees: x ends at the last column, whatever the
+    rows (a row's position is no position of x)."""
+    import ctypes as C
+    import torch
+    rng = np.random.default_rng(rows)
+    P, Q = rng.random((rows, 3)) * [1, 1, 6], rng.random((cols, 3)) * [1, 1, 6]
+    tr, tc = hmat_amd.ClusterTree(P, 100), hmat_amd.ClusterTree(Q, 100)
+
+    @hmat_amd.PREPARE_FUNC
+    def prepare(r0, rc, c0, cc, rows_h2c, rows_c2h, cols_h2c, cols_c2h, ctx, info):
+        blocks[len(blocks) + 1] = (np.array(rows_h2c[r0:r0 + rc]), np.array(cols_h2c[c0:c0 + cc]))
+        info[0].user_data = len(blocks)
+
+    @hmat_amd.COMPUTE_FUNC
+    def compute(data, r0, rc, c0, cc, out):
+        ri, ci = blocks[data]
+        d = P[ri[r0:r0 + rc]][:, None] - Q[ci[c0:c0 + cc]][None]
+        np.ctypeslib.as_array(C.cast(out, C.POINTER(C.c_double)), shape=(cc, rc))[:] = \
+            np.exp(-np.sqrt((d * d).sum(axis=2))).T
+
+    blocks = {}
+    h = hmat_amd.HMatrix(tr, lower_symmetric=False)
+    h.close()
+    lib = hmat_amd.load()
+    adm = lib.hmat_create_admissibility_standard(2.0)
+    h.handle = h.iface.create_empty_hmatrix_admissibility(tr.handle, tc.handle, 0, adm)
+    lib.hmat_delete_admissibility(adm)
+    h.iface.set_low_rank_epsilon(h.handle, 1e-4)
+    h.assemble_functions(block=compute, prepare=prepare)
+    A = np.zeros((rows, cols))
+    for m, n, r0, c0, kind, rank, a, b in h.leaves():
+        A[r0:r0 + m, c0:c0 + n] = a if kind == 0 else a @ b.T
+    print(f"gemv two trees {rows} x {cols}", flush=True)
+    for nrhs in (1, 2):
+        X, Y = rng.standard_normal((cols, nrhs)), rng.standard_normal((rows, nrhs))
+        want = 0.75 * (A @ X) - 0.5 * Y
+        bound = 4 * (rows + cols) * 2.0 ** -53 * (np.abs(A) @ np.abs(X) + np.abs(Y))
+        x, y = torch.tensor(X.T.copy(), device="cuda"), torch.tensor(Y.T.copy(), device="cuda")
+        torch.cuda.synchronize()
+        h.gemv_device(x.data_ptr(), y.data_ptr(), nrhs, alpha=0.75, beta=-0.5)
+        assert (np.abs(y.cpu().numpy().T - want) <= bound).all()
+        x, y = np.asfortranarray(X[np.argsort(tc.indices)]), np.asfortranarray(Y[np.argsort(tr.indices)])
+        al, be = C.c_double(0.75), C.c_double(-0.5)
+        assert h.iface.gemv(b"N", C.cast(C.byref(al), C.c_void_p), h.handle, x.ctypes.data,
+                            C.cast(C.byref(be), C.c_void_p), y.ctypes.data, nrhs) == 0
+        assert (np.abs(y[tr.indices] - want) <= bound).all()
+    h.close()
