@@ -6,126 +6,34 @@
 
 #include "factor_kernels.hpp"
 #include <chrono>
-#include <list>
-#include <mutex>
 #include <cstring>
 #include <functional>
 #include <stdexcept>
 
 namespace hmx {
 
-// ---- device buffers kept between objects --------------------------------------
-// A buffer given up by a DevBuf is kept for the next one of its size instead
-// of going back to the driver, which clears device memory before it hands it
-// out again: a program that builds, factorises and drops one matrix after the
-// other (a likelihood per hyperparameter, a batch of systems) spent most of
-// its time there (N = 50,000: assembly 12 ms of kernels, 474 ms a pass; an
-// 8,000-point likelihood and gradient 107 ms with clean memory at hand, 204 ms
-// without).  At most kept_limit() bytes are kept per process and device, the
-// oldest go first; all of them go back when an allocation fails and at
-// hmat_interface_t.finalize.
-//
-// release() waits for the device, as hipFree does, so that a kept buffer has
-// no work of any stream left on it; the lists are guarded by a mutex.
-namespace {
-struct KeptBuffer {
-  void* p;
-  size_t bytes;
-  int dev;
-};
-std::mutex kept_mutex;
-std::list<KeptBuffer>& kept_list() {  // oldest first; never destroyed (the runtime may end before it)
-  static auto* l = new std::list<KeptBuffer>;
-  return *l;
-}
-size_t kept_bytes = 0;
-
-// an eighth of the device's memory: 36 GB of 288
-size_t kept_limit() {
-  size_t freeb = 0, total = 0;
-  if (hipMemGetInfo(&freeb, &total) != hipSuccess) return 0;
-  return total / 8;
-}
-
-// sizes are rounded up to an eighth of their power of two, so that buffers of
-// similar objects fit each other
-size_t rounded_size(size_t n) {
-  size_t step = 256;
-  while (step * 16 <= n) step *= 2;
-  return (n + step - 1) / step * step;
-}
-}  // namespace
-
-void release_kept_memory() {
-  std::lock_guard<std::mutex> lock(kept_mutex);
-  for (const KeptBuffer& k : kept_list()) (void)hipFree(k.p);
-  kept_list().clear();
-  kept_bytes = 0;
-}
-
 size_t device_free_bytes() {
   size_t freeb = 0, total = 0;
   HMX_CHECK(hipMemGetInfo(&freeb, &total));
   int dev = 0;
   HMX_CHECK(hipGetDevice(&dev));
-  std::lock_guard<std::mutex> lock(kept_mutex);
-  for (const KeptBuffer& k : kept_list())
-    if (k.dev == dev) freeb += k.bytes;
-  return freeb;
+  return freeb + kept_memory(dev);
 }
 
 void DevBuf::release() {
-  if (p && hipDeviceSynchronize() == hipSuccess) {
-    static const size_t limit = kept_limit();
-    std::lock_guard<std::mutex> lock(kept_mutex);
-    if (bytes <= limit) {
-      auto& l = kept_list();
-      l.push_back(KeptBuffer{p, bytes, dev});
-      kept_bytes += bytes;
-      while (kept_bytes > limit) {
-        (void)hipFree(l.front().p);
-        kept_bytes -= l.front().bytes;
-        l.pop_front();
-      }
-      p = nullptr;
-    }
-  }
-  if (p) (void)hipFree(p);
+  give_buffer(TakenBuffer{p, bytes, dev});
   p = nullptr;
   bytes = 0;
 }
 
 void DevBuf::alloc(size_t nbytes) {
   release();
-  const size_t want = rounded_size(std::max<size_t>(nbytes, 1));
-  int d = 0;
-  HMX_CHECK(hipGetDevice(&d));
-  {
-    std::lock_guard<std::mutex> lock(kept_mutex);
-    auto& l = kept_list();
-    auto best = l.end();
-    for (auto it = l.begin(); it != l.end(); ++it)
-      if (it->dev == d && it->bytes >= want && it->bytes <= want + want / 4 &&
-          (best == l.end() || it->bytes < best->bytes))
-        best = it;
-    if (best != l.end()) {
-      p = best->p;
-      bytes = best->bytes;
-      dev = d;
-      kept_bytes -= bytes;
-      l.erase(best);
-      return;
-    }
-  }
-  hipError_t e = hipMalloc(&p, want);
-  if (e != hipSuccess) {
-    (void)hipGetLastError();
-    release_kept_memory();
-    p = nullptr;
-    HMX_CHECK(hipMalloc(&p, want));
-  }
-  bytes = want;
-  dev = d;
+  int error = 0;
+  const TakenBuffer b = take_buffer(nbytes, &error);
+  HMX_CHECK((hipError_t)error);
+  p = b.p;
+  bytes = b.bytes;
+  dev = b.dev;
 }
 
 void DevBuf::ensure(size_t nbytes) {

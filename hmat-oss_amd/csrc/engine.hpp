@@ -12,13 +12,14 @@
 #include <vector>
 
 #include "hmat/hmat.h"
+#include "kept_buffers.hpp"
 #include "kernels.hpp"
 #include "tree.hpp"
 
 namespace hmx {
 
 // Owning device allocation.  Buffers given up are kept for later ones, within
-// a bound (see engine.cpp); the content of a new one is undefined.
+// a bound (kept_buffers.hpp); the content of a new one is undefined.
 struct DevBuf {
   void* p = nullptr;
   size_t bytes = 0;
@@ -36,8 +37,6 @@ struct DevBuf {
 
 void upload(DevBuf& b, const void* src, size_t bytes, hipStream_t s);
 
-// Gives the kept buffers back to the driver.
-void release_kept_memory();
 // Free memory of the current device, the kept buffers included.
 size_t device_free_bytes();
 

@@ -4,6 +4,7 @@
   the other, in one thread and in four, reuse each other's buffers: every
   product equals that of the matrix's own leaves (4 N u |A| |x|), every solve
   leaves the compression's residual.
+* A matrix closed with products queued on the caller's stream.
 * hmat_interface_t.finalize gives the kept buffers back.
 * Blocks whose ACA needs more columns than its first room (32) run again: at
   eps 1e-13 the ranks are above it and the matrix is within 1,000 eps of the
@@ -75,3 +76,33 @@ def test_aca_rooms():
     K = np.exp(-np.sqrt(((P[:, None] - P[None]) ** 2).sum(axis=2)) / 0.5)
     assert np.linalg.norm(h.to_dense() - K) <= 1e-10 * np.linalg.norm(K)
     h.close()
+
+
+def test_closed_with_work_queued():
+    """A matrix closed while products on the caller's stream are queued: the next
+    matrix of the same size takes its buffers, the products stay those of the
+    first."""
+    import torch
+    n = 1500
+    rng = np.random.default_rng(3)
+    for k in range(3):
+        t = hmat_amd.ClusterTree(_points(n, 20 + k), 64)
+        h = hmat_amd.HMatrix(t)
+        h.assemble(length=0.5, nugget=1e-1, eps=1e-6)
+        A = h.to_dense()
+        x = rng.standard_normal((4, n))
+        xd = torch.tensor(x, device="cuda")
+        yd = [torch.zeros_like(xd) for _ in range(40)]
+        s = torch.cuda.Stream()
+        torch.cuda.synchronize()
+        h.set_stream(s.cuda_stream)
+        for y in yd:
+            h.gemv_device(xd.data_ptr(), y.data_ptr(), 4)
+        h.close()
+        g = hmat_amd.HMatrix(t)
+        g.assemble(length=0.1, nugget=3.0, eps=1e-6)
+        s.synchronize()
+        bound = 4 * n * 2.0 ** -53 * (np.abs(A) @ np.abs(x.T))
+        for y in yd:
+            assert (np.abs(y.cpu().numpy().T - A @ x.T) <= bound).all()
+        g.close()
