@@ -167,11 +167,12 @@ __device__ inline bool wg_xty_any(PX X, int ldx, int kx, PX Y, int ldy, int ky, 
   return true;
 }
 
-// G = X^T X (k x k, ld ldg, both triangles) for X (p x k, ld ldx, k <= 16 kNb <= 48):
+// G = X^T X (k x k, ld ldg, both triangles) for X (p x k, ld ldx, k <= 16 kNb <= 32):
 // wg_xty for one panel, each entry loaded once and the tiles on and above the
 // diagonal only; kU slabs' loads in flight per wavefront.
 template <int kNb, int kU, typename PX>
 __device__ void wg_gram(PX X, int ldx, int k, int p, lptr<double> G, int ldg, lptr<double> part) {
+  static_assert(kNb <= 2, "the tiles' numbering below");
   constexpr int kTiles = kNb * (kNb + 1) / 2;
   const int lane = threadIdx.x & (kWave - 1), w = threadIdx.x / kWave;
   const int kk = lane >> 4, ii = lane & 15;
@@ -216,7 +217,7 @@ __device__ void wg_gram(PX X, int ldx, int k, int p, lptr<double> G, int ldg, lp
 #pragma unroll
   for (int t = 0; t < kTiles; ++t) {
     // tile t is (a, b), a <= b, row by row
-    const int a = t < kNb ? 0 : (t < 2 * kNb - 1 ? 1 : 2), b = a == 0 ? t : (a == 1 ? t - kNb + 1 : 2);
+    const int a = t < kNb ? 0 : 1, b = t < kNb ? t : 1;
     const int q = threadIdx.x;
     double s = 0.0;
 #pragma unroll

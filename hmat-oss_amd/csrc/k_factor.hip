@@ -1425,7 +1425,7 @@ __device__ void concat_side(PD dst, int ld, int rows, bool bside, const FTask& t
 // Both sides at once for K <= kColsMax: a lane builds each column's descriptor,
 // then every wavefront copies four columns at a time, their loads in flight
 // together and no index divided.
-constexpr int kColsMax = 40;
+constexpr int kColsMax = 32;
 constexpr int kColDoubles = 6 * kColsMax;  // LDS for the descriptors (2 K of three doubles)
 
 template <typename T, typename PD>
@@ -1733,8 +1733,11 @@ __device__ void qr_global(gptr<double> Va, int m, gptr<double> Vb, int n, int K,
 // A' = A P1 R11^-1 U sqrt(S), B' = B P1 R11^-1 V sqrt(S).  Q is orthonormal to
 // about 1e-16 / 1e-13 = 1e-3, so the truncated product stays within eps.
 // ---------------------------------------------------------------------------
-// Widest sum in this form: its small matrices fit in LDS (K = 40: 130 KB).  33 to
-// 38 columns took 1.0 to 1.4 ms as Householder QR with a workgroup's Jacobi.
+// Widest sum in this form.  Squaring the panels' condition costs accuracy that
+// wider sums, which come with tight cuts, do not have: with 33 to 40 columns and
+// eps = 1e-7 the result was 3.5e-7 off instead of 1e-7, two ranks short (at 1e-8
+// 28 to 36 times the best error, against 5 to 7 times through Householder QR,
+// which takes 1,100 us there instead of 550).
 constexpr int kGramMaxK = kColsMax;
 constexpr double kGramTol = 1e-13;
 constexpr double kGramJacobiTol2 = 1e-16;
@@ -1843,12 +1846,9 @@ __device__ void gram_recompress(PV Va, int lda, PV Vb, int ldb, const FTask& t, 
   if (K <= 16) {
     wg_gram<1, kU>(Va, lda, K, m, Ga, K, part);
     wg_gram<1, kU>(Vb, ldb, K, n, Gb, K, part);
-  } else if (K <= 32) {
+  } else {
     wg_gram<2, kU / 2>(Va, lda, K, m, Ga, K, part);
     wg_gram<2, kU / 2>(Vb, ldb, K, n, Gb, K, part);
-  } else {
-    wg_gram<3, 2>(Va, lda, K, m, Ga, K, part);
-    wg_gram<3, 2>(Vb, ldb, K, n, Gb, K, part);
   }
   const int wid = threadIdx.x / kWave, lane = threadIdx.x & (kWave - 1);
   if (wid < 2) {
@@ -1874,18 +1874,12 @@ __device__ void gram_recompress(PV Va, int lda, PV Vb, int ldb, const FTask& t, 
   __syncthreads();
   // columns orthogonal to 1e-8 of their norms: far below the FP32 data's
   // rounding once scaled by the eps cut
-  if (ra <= kCoreMax && rb <= kCoreMax) {
-    if (wid == 0) {
-      const int c = wave_core_svd(Cm, ra, ra, rb, kGramJacobiTol2, fmax(1e-30, 1e-16 * eps * eps));
-      const int k = wave_sorted_cut(Cm, ra, ra, c, sig, order, eps);
-      if (lane < c) scale[lane] = 1.0 / sqrt(sig[lane]);
-      if (lane == 0) ranks[2] = k;
-    }
-  } else {
-    jacobi_svd(Cm, ra, ra, rb, lptr<double>(nullptr), rb, nullptr, 40, kGramJacobiTol2);
-    sorted_norms(Cm, ra, ra, rb, sig, order);
-    if (threadIdx.x < rb) scale[threadIdx.x] = 1.0 / sqrt(sig[threadIdx.x]);
-    if (threadIdx.x == 0) ranks[2] = find_k(sig, order, rb, eps);
+  static_assert(kGramMaxK <= kCoreMax, "the core SVD of one wavefront");
+  if (wid == 0) {
+    const int c = wave_core_svd(Cm, ra, ra, rb, kGramJacobiTol2, fmax(1e-30, 1e-16 * eps * eps));
+    const int k = wave_sorted_cut(Cm, ra, ra, c, sig, order, eps);
+    if (lane < c) scale[lane] = 1.0 / sqrt(sig[lane]);
+    if (lane == 0) ranks[2] = k;
   }
   __syncthreads();
   int nk = ranks[2];

@@ -1,6 +1,5 @@
 """Core SVD of the recompressions on one wavefront (FADD and RKRK) at the edges
-of its register forms (16, 24 and 32 columns) and above (FADD of 40 and 41
-columns, where the FP32 Gram form ends), with cores that
+of its register forms (16, 24 and 32 columns) and above, with cores that
 are rectangular, rank deficient, zero or of one column, against numpy's
 truncated SVD.  The singular values fall by 0.6 a step, so the cut at eps has a
 relative gap of 0.4 and the truncated matrix moves by a few K u / 0.4 of its
@@ -110,3 +109,43 @@ def test_rkrk_core_sizes(fp32):
         # one rank more or less at the cut is eps s[0]
         tol = (1e-5 if k == kw else EPS) if fp32 else 1e-11
         assert np.linalg.norm(got - want) <= tol * s[0], what
+
+
+@pytest.mark.parametrize("eps", [1e-6, 1e-7])
+def test_fadd_fp32_tight_eps(eps):
+    """FP32 sums of more than 32 columns at cuts near the panels' rounding.  The
+    recompression works in FP64, so the distance to the exact sum is that of the
+    cut, at most sqrt(K) eps s[0], and the rounding of the new panels A, B
+    (2^-24 each of entries whose products sum to |A| |B^T|, whose norm is at
+    most the sum of the singular values)."""
+    rng = np.random.default_rng(13)
+    tasks, keep = [], []
+    for m, n, kt, kp in [(130, 140, 16, 17), (130, 140, 18, 18), (70, 90, 20, 20), (700, 900, 20, 20),
+                         (130, 140, 20, 21)]:
+        K = kt + kp
+
+        def panels(k):
+            a = np.linalg.qr(rng.standard_normal((m, k)))[0] * 10.0 ** (-8.0 * np.arange(k) / k)
+            b = np.linalg.qr(rng.standard_normal((n, k)))[0]
+            return a.astype(np.float32).astype(np.float64), b.astype(np.float32).astype(np.float64)
+        (ta, tb), (pa, pb) = panels(kt), panels(kp)
+        TA, TB = np.zeros((m, K)), np.zeros((n, K))
+        TA[:, :kt], TB[:, :kt] = ta, tb
+        h = [tr.dev(TA, True), tr.dev(TB, True), tr.ints([kt]), tr.dev(pa, True), tr.dev(pb, True), tr.ints([kp])]
+        t = tr.FTask()
+        t.type, t.eps, t.nparts = tr.T_FADD, eps, 1
+        t.tgt = tr.rkref(h[0], h[1], m, n, K, h[2])
+        t.parts[0].rk = tr.rkref(h[3], h[4], m, n, kp, h[5])
+        t.parts[0].alpha = 0.5
+        tasks.append(t)
+        keep.append((ta @ tb.T + 0.5 * pa @ pb.T, h, (m, n, kt, kp)))
+    assert tr.run(tasks, tr.T_FADD, True) == [0, 0]
+    for S, h, what in keep:
+        k = int(h[2].cpu().numpy()[0])
+        R = tr.host(h[0])[:, :k] @ tr.host(h[1])[:, :k].T
+        s = np.linalg.svd(S, compute_uv=False)
+        kw = tr.find_k(s, eps)
+        err, cut = np.linalg.norm(S - R), np.linalg.norm(s[kw:])
+        print(f"fp32 eps={eps} {what}: rank {k} of {kw}, error {err / s[0]:.2e}, cut {cut / s[0]:.2e}", flush=True)
+        assert abs(k - kw) <= 1, (what, k, kw)
+        assert err <= 1.01 * max(cut, eps * s[0]) + 2 * 2.0 ** -24 * s.sum(), what
