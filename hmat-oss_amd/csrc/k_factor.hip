@@ -368,6 +368,9 @@ __device__ inline double chain_rcp(double d) {
   y = fma(fma(-s, y, 1.0), y, y);
   return fabs(d) <= 1.79e308 ? __builtin_amdgcn_ldexp(y, -e) : 1.0 / d;
 }
+// A power of two that brings a divisor whose reciprocal is above the largest
+// finite number (below 5.6e-309) into range: a / d = (a up) / (d up).
+__device__ inline double chain_up(double d) { return fabs(d) < 0x1p-1000 ? 0x1p+500 : 1.0; }
 // a / d with y = 1 / d: the product corrected by its remainder (a == d gives 1)
 __device__ inline double chain_div(double a, double d, double y) {
   const double q = a * y;
@@ -494,7 +497,8 @@ __device__ void potrf_lds(double* L, int ld, int n, int* info) {
         const double d = lane_read(a[j], j);
         bad |= !(d > 0.0);
         diag = i == j ? a[j] : diag;
-        const double m = a[j] * chain_rcp(d);
+        const double up = chain_up(d);
+        const double m = (a[j] * up) * chain_rcp(d * up);
         if (lane < kNb) mult[i + kNb * j] = m;
 #pragma unroll
         for (int c = j + 1; c < kNb; ++c) a[c] -= m * lane_read(a[j], c);
@@ -776,13 +780,13 @@ __device__ void getrf_lds(double* P, int ld, int n, int* piv, int* info) {
         }
         // a quotient and not a product with 1 / d: the multiplier of a row equal to
         // the pivot's is then exactly 1, and a singular leaf ends on an exact zero
-        const double y = chain_rcp(d);
+        const double up = chain_up(d), du = d * up, y = chain_rcp(du);
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
           // interchange of the positions j and pp
           pos[h] = pos[h] == pp ? j : (pos[h] == j ? pp : pos[h]);
           if (pos[h] > j) {
-            const double l = chain_div(a[h][j], d, y);
+            const double l = chain_div(a[h][j] * up, du, y);
             a[h][j] = l;
 #pragma unroll
             for (int c = j + 1; c < kNb; ++c) a[h][c] -= l * u[c];

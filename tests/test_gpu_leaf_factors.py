@@ -78,3 +78,46 @@ def test_getrf_sizes(fp32):
     sing = keep[9].copy()
     sing[:, 20] = 0.0
     assert _run(tr.T_GETRF, [keep[3], sing], fp32, [tr.ints(np.zeros(128)), tr.ints(np.zeros(128))])[1][1] != 0
+
+
+def test_pivots_below_the_reciprocals_range():
+    """Pivots whose reciprocal overflows (FP64): zeros below them stay zeros, and
+    the quotients of entries of their size are those of the same leaf scaled up.
+    The other columns do not see them (their rows of L or U are zero or of
+    1e-310), so the bounds are those of the sizes test."""
+    rng = np.random.default_rng(8)
+    tiny = 3.0 * 2.0 ** -1030
+    for n in (17, 40, 100):
+        g = rng.standard_normal((n, n))
+        spd = g @ g.T / n + 0.1 * np.eye(n)
+        j = n // 2
+        spd[j, :], spd[:, j] = 0.0, 0.0
+        spd[j, j] = tiny
+        dev, flags = _run(tr.T_POTRF, [spd], False)
+        L = tr.host(dev[0])
+        assert flags == [0, 0] and np.isfinite(L).all() and abs(L[j, j] - tiny ** 0.5) <= 1e-15 * tiny ** 0.5
+        assert (np.abs(L @ L.T - spd) <= 8 * n * 2.0 ** -53 * (np.abs(L) @ np.abs(L.T)) + 2.0 ** -1074).all(), n
+        lu = rng.standard_normal((n, n))
+        lu[:, j] = 0.0
+        lu[j, :] = 0.0
+        lu[j, j] = tiny
+        piv = [tr.ints(np.full(n, -1))]
+        dev, flags = _run(tr.T_GETRF, [lu], False, piv)
+        F = tr.host(dev[0])
+        want, pv, info = sl.lapack.dgetrf(lu)
+        assert flags == [0, 0] and info == 0 and np.isfinite(F).all()
+        assert np.array_equal(piv[0].cpu().numpy(), pv)
+        L, U = np.tril(F, -1) + np.eye(n), np.triu(F)
+        B = lu.copy()
+        for i, q in enumerate(pv):
+            B[[i, q]] = B[[q, i]]
+        assert (np.abs(L @ U - B) <= 8 * n * 2.0 ** -53 * (np.abs(L) @ np.abs(U)) + 2.0 ** -1074).all(), n
+    # a leaf that is tiny throughout: powers of two (no entry is rounded on the
+    # way), LU of the scaled leaf
+    n = 24
+    a = np.tril(2.0 ** rng.integers(-3, 0, (n, n)), -1) * np.where(rng.random((n, n)) < 0.5, -1.0, 1.0)
+    a = np.where(rng.random((n, n)) < 0.8, 0.0, a) + np.eye(n)
+    piv = [tr.ints(np.full(n, -1))]
+    dev, flags = _run(tr.T_GETRF, [a * 2.0 ** -1040], False, piv)
+    want = sl.lapack.dgetrf(a)[0]
+    assert flags == [0, 0] and np.array_equal(np.tril(tr.host(dev[0]), -1), np.tril(want, -1))
