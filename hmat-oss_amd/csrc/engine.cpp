@@ -869,17 +869,25 @@ void Matrix::build_gemv_plan() {
 
 size_t Matrix::gemv_scratch_elems(int nrhs) const { return (size_t)plan_.counted1 * (size_t)nrhs; }
 
+// (the kernels put right-hand sides in their grid's y, which ends at 65,535:
+// wider products go kGemvRhs at a time, through the same scratch)
+constexpr int kGemvRhs = 32768;
+
 template <typename T>
 void Matrix::gemv_launch(double alpha, const T* x, double beta, T* y, int nrhs, int ldx, int ldy,
-                         const Store<T>& st, double* zpart, double* z, double* slots) {
+                         const Store<T>& st, double* zpart, double* z, double* slots, int per) {
   const GemvPlan& P = plan_;
   const int* ranks = st.ranks.template as<int>();
-  launch_gemv_zpass<T>(ranks, st.data(), P.zitems.as<ZItem>(), P.nzlong, P.nz, x, ldx, nrhs, zpart, z, stream);
-  launch_gemv_zreduce(P.zred.as<ZReduce>(), P.nzred, ranks, zpart, nrhs, z, stream);
-  launch_gemv_ypass<T>(ranks, st.data(), P.yitems.as<YItem>(), P.ny, P.contrib.as<YContrib>(), z, slots, x,
-                       ldx, nrhs, stream);
-  launch_gemv_yfinal<T>(P.yfinal.as<YFinal>(), P.nfinal, P.slotlist.as<int64_t>(), slots, y, ldy, nrhs,
-                        alpha, beta, stream);
+  for (int r = 0; r < nrhs; r += per) {
+    const int nr = std::min(per, nrhs - r);
+    const T* xr = x + (size_t)r * ldx;
+    launch_gemv_zpass<T>(ranks, st.data(), P.zitems.as<ZItem>(), P.nzlong, P.nz, xr, ldx, nr, zpart, z, stream);
+    launch_gemv_zreduce(P.zred.as<ZReduce>(), P.nzred, ranks, zpart, nr, z, stream);
+    launch_gemv_ypass<T>(ranks, st.data(), P.yitems.as<YItem>(), P.ny, P.contrib.as<YContrib>(), z, slots, xr,
+                         ldx, nr, stream);
+    launch_gemv_yfinal<T>(P.yfinal.as<YFinal>(), P.nfinal, P.slotlist.as<int64_t>(), slots, y + (size_t)r * ldy,
+                          ldy, nr, alpha, beta, stream);
+  }
 }
 
 template <typename T>
@@ -890,15 +898,16 @@ void Matrix::gemv_device(double alpha, const T* x, double beta, T* y, int nrhs, 
   if (!plan_.built) build_gemv_plan();
   if (!plan_.built) throw std::runtime_error("gemv: leaf clusters above 512 rows are not provided");
   GemvPlan& P = plan_;
-  if (P.nrhs < nrhs) {
+  const int per = std::min(nrhs, kGemvRhs);
+  if (P.nrhs < per) {
     HMX_CHECK(hipStreamSynchronize(stream));
-    P.zpart.ensure(std::max<int64_t>(P.zpart1 * nrhs, 1) * sizeof(double));
-    P.z.ensure(std::max<int64_t>(P.z1 * nrhs, 1) * sizeof(double));
-    P.slots.ensure(std::max<int64_t>(P.slot1 * nrhs, 1) * sizeof(double));
-    P.nrhs = nrhs;
+    P.zpart.ensure(std::max<int64_t>(P.zpart1 * per, 1) * sizeof(double));
+    P.z.ensure(std::max<int64_t>(P.z1 * per, 1) * sizeof(double));
+    P.slots.ensure(std::max<int64_t>(P.slot1 * per, 1) * sizeof(double));
+    P.nrhs = per;
   }
   gemv_launch<T>(alpha, x, beta, y, nrhs, ldx, ldy, st, P.zpart.as<double>(), P.z.as<double>(),
-                 P.slots.as<double>());
+                 P.slots.as<double>(), per);
 }
 
 template <typename T>
@@ -918,7 +927,7 @@ void Matrix::gemv_device_scratch(double alpha, const T* x, double beta, T* y, in
   double* zpart = scratch;
   double* z = zpart + P.zpart1 * nrhs;
   double* slots = z + P.z1 * nrhs;
-  gemv_launch<T>(alpha, x, beta, y, nrhs, n_cols(), n_rows(), st, zpart, z, slots);
+  gemv_launch<T>(alpha, x, beta, y, nrhs, n_cols(), n_rows(), st, zpart, z, slots, nrhs);
 }
 template void Matrix::gemv_device_scratch<double>(double, const double*, double, double*, int,
                                                   const Store<double>&, double*, size_t);

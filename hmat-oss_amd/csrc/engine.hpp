@@ -298,7 +298,7 @@ class Matrix {
   void build_gemv_plan();
   template <typename T>
   void gemv_launch(double alpha, const T* x, double beta, T* y, int nrhs, int ldx, int ldy,
-                   const Store<T>& st, double* zpart, double* z, double* slots);
+                   const Store<T>& st, double* zpart, double* z, double* slots, int per);
   GemvPlan plan_;
   DevBuf overflow_;
   std::shared_ptr<struct FactorState> fstate_;

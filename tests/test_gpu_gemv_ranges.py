@@ -101,3 +101,20 @@ def test_gemv_two_trees(rows, cols):
                             C.cast(C.byref(be), C.c_void_p), y.ctypes.data, nrhs) == 0
         assert (np.abs(y[tr.indices] - want) <= bound).all()
     h.close()
+
+
+def test_gemv_more_right_hand_sides_than_a_grid_has_rows():
+    import torch
+    n, nrhs = 60, 70001
+    h = hmat_amd.HMatrix(hmat_amd.ClusterTree(np.random.default_rng(1).random((n, 3)), 16))
+    h.assemble()
+    A = h.to_dense()
+    x = torch.randn(nrhs, n, dtype=torch.float64, device="cuda")
+    y0 = torch.randn(nrhs, n, dtype=torch.float64, device="cuda")
+    y = y0.clone()
+    torch.cuda.synchronize()
+    h.gemv_device(x.data_ptr(), y.data_ptr(), nrhs, alpha=2.0, beta=1.0)
+    X, Y = x.cpu().numpy(), y0.cpu().numpy()
+    bound = 4 * n * 2.0 ** -53 * (np.abs(X) @ (2.0 * np.abs(A)) + np.abs(Y))
+    assert (np.abs(y.cpu().numpy() - (2.0 * (X @ A) + Y)) <= bound).all()
+    h.close()
