@@ -815,7 +815,7 @@ void Matrix::build_gemv_plan() {
   std::vector<YContrib> contrib;
   std::vector<YFinal> yf;
   std::vector<int64_t> slist;
-  const int64_t array = (int64_t)(kNoAllocArrayBytes / sizeof(double)), admit = (int64_t)(kNoAllocScratchBytes / sizeof(double));
+  const int64_t array = (int64_t)(kNoAllocScratchBytes / sizeof(double));
   int64_t slots_used = 0;
   for (int64_t grain = std::min<int64_t>(32768, std::max<int64_t>(4096, total / 2048));; grain *= 2) {
     yi.clear();
@@ -843,10 +843,10 @@ void Matrix::build_gemv_plan() {
       fin.end = (int)slist.size();
       yf.push_back(fin);
     }
-    // the allocation-free entry point admits nrhs by counted1 and must hold
-    // this plan's scratch then: fewer, longer runs where it would not
-    const int64_t most = std::max<int64_t>(admit / std::max<int64_t>(P.counted1, 1), 1);
-    if ((zpart + zbuf + slots_used) * most <= array || P.counted1 > admit || (int64_t)yi.size() <= (int64_t)ranges.size())
+    // the allocation-free entry point admits products by counted1 and lays them
+    // out in its array, one right-hand side at a time if need be: fewer, longer
+    // runs where not even that would fit
+    if (zpart + zbuf + slots_used <= array || P.counted1 > array || (int64_t)yi.size() <= (int64_t)ranges.size())
       break;
   }
   upload(P.zitems, zi.data(), zi.size() * sizeof(ZItem), stream);
@@ -862,6 +862,10 @@ void Matrix::build_gemv_plan() {
   P.nzred = (int)zr.size();
   P.ny = (int)yi.size();
   P.nfinal = (int)yf.size();
+  // (leaf clusters above 128 rows have up to four slots per mirrored leaf where
+  // the count has one: scratch of the matrix's own if they exceed the array)
+  if (zpart + zbuf + slots_used > array && P.counted1 <= array)
+    P.noalloc.ensure((size_t)(zpart + zbuf + slots_used) * sizeof(double));
   P.built = true;
   P.nrhs = 0;
   HMX_CHECK(hipStreamSynchronize(stream));
@@ -919,15 +923,28 @@ void Matrix::gemv_device_scratch(double alpha, const T* x, double beta, T* y, in
   if (nrhs < 1) throw std::runtime_error("gemv: nrhs must be positive");
   const GemvPlan& P = plan_;
   const size_t need = gemv_scratch_elems(nrhs);
-  if (need * sizeof(double) > kNoAllocScratchBytes ||
-      (size_t)(P.zpart1 + P.z1 + P.slot1) * (size_t)nrhs > scratch_elems)
+  if (need > scratch_elems)
     throw std::runtime_error("gemv: needs " + std::to_string(need * sizeof(double)) +
                              " bytes of scratch, the allocation-free entry point has " +
-                             std::to_string(kNoAllocScratchBytes));
+                             std::to_string(scratch_elems * sizeof(double)));
+  // as many right-hand sides at a time as the layout has room for: whole
+  // matrix-core tiles of 32, or parts of equal size below that
+  const size_t one = std::max<size_t>(P.zpart1 + P.z1 + P.slot1, 1);
+  if (one > scratch_elems) {
+    scratch = P.noalloc.as<double>();
+    scratch_elems = one;
+  }
+  int per = (int)std::min<size_t>(std::min(nrhs, kGemvRhs), scratch_elems / one);
+  if (per < nrhs) {
+    if (per >= 32)
+      per -= per % 32;
+    else
+      per = (nrhs + (nrhs + per - 1) / per - 1) / ((nrhs + per - 1) / per);
+  }
   double* zpart = scratch;
-  double* z = zpart + P.zpart1 * nrhs;
-  double* slots = z + P.z1 * nrhs;
-  gemv_launch<T>(alpha, x, beta, y, nrhs, n_cols(), n_rows(), st, zpart, z, slots, nrhs);
+  double* z = zpart + P.zpart1 * per;
+  double* slots = z + P.z1 * per;
+  gemv_launch<T>(alpha, x, beta, y, nrhs, n_cols(), n_rows(), st, zpart, z, slots, per);
 }
 template void Matrix::gemv_device_scratch<double>(double, const double*, double, double*, int,
                                                   const Store<double>&, double*, size_t);

@@ -89,6 +89,7 @@ struct GemvPlan {
   int64_t zpart1 = 0, z1 = 0, slot1 = 0;  // scratch doubles per right-hand side
   int64_t counted1 = 0;  // the count by which the allocation-free entry point admits products
   DevBuf zpart, z, slots;
+  DevBuf noalloc;  // scratch of the allocation-free entry point where its array is too small
 };
 
 struct Stats {

@@ -753,7 +753,7 @@ HMX_INST(float)
 // they read, so nothing needs clearing between calls.  Host code must not use
 // the array's name as a device address: noalloc_gemv_scratch() returns the
 // device address looked up with hipGetSymbolAddress, once per device.
-static __device__ __align__(256) double scratch[kNoAllocArrayBytes / sizeof(double)];
+static __device__ __align__(256) double scratch[kNoAllocScratchBytes / sizeof(double)];
 
 double* noalloc_gemv_scratch(size_t* elems) {
   static std::mutex mu;
@@ -770,7 +770,7 @@ double* noalloc_gemv_scratch(size_t* elems) {
                                hipGetErrorString(e));
     ptr[dev] = static_cast<double*>(p);
   }
-  *elems = kNoAllocArrayBytes / sizeof(double);
+  *elems = kNoAllocScratchBytes / sizeof(double);
   return ptr[dev];
 }
 

@@ -149,11 +149,9 @@ void launch_pick_scale(const double* V, int ldv, int rows, int first, int count,
                        const double* lam, double e, double* out, hipStream_t s);
 
 // Fixed device scratch of the allocation-free H-gemv: products of up to
-// kNoAllocScratchBytes of temporaries by gemv_scratch_elems' count are taken;
-// the array holds the most that the present plan lays out for such a product.
+// kNoAllocScratchBytes of temporaries by gemv_scratch_elems' count are taken.
 // Returns its device address on the current device (looked up once per device).
 constexpr size_t kNoAllocScratchBytes = size_t(64) << 20;
-constexpr size_t kNoAllocArrayBytes = 4 * kNoAllocScratchBytes;
 double* noalloc_gemv_scratch(size_t* elems);
 
 template <typename T>

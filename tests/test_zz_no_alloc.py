@@ -74,3 +74,32 @@ def test_noalloc_gemv_rejects_oversized_product():
     with pytest.raises(hmat_amd.EngineError, match="scratch"):
         h.gemv_device_noalloc(x.data_ptr(), y.data_ptr(), nrhs)
     h.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,leaf,height", [(2500, 128, 1.0), (2500, 128, 30.0), (9000, 500, 40.0), (20000, 100, 1.6)])
+def test_noalloc_gemv_up_to_its_bound(n, leaf, height):
+    """Every product up to the bound of 64 MiB is taken, also where the plan lays out
+    more than the count behind the bound (then a part of the right-hand sides at
+    a time), and loading the library holds no more than that array."""
+    import torch
+    t, h = _matrix(n, height, 9, leaf)
+    x = torch.zeros((1, n), dtype=torch.float64, device="cuda")
+
+    def refused(nrhs):
+        try:
+            h.gemv_device_noalloc(x.data_ptr(), x.data_ptr(), nrhs)   # refused before it reads x
+        except hmat_amd.EngineError as e:
+            return int(str(e).split("needs ")[1].split()[0])
+        raise AssertionError("taken")
+    one = refused(1 << 20) >> 20                       # bytes of a right-hand side
+    nrhs = (64 << 20) // one
+    say(f"noalloc n={n} leaf={leaf}: {one} bytes a right-hand side, {nrhs} of them")
+    assert refused(nrhs + 1) == (nrhs + 1) * one
+    A = np.abs(h.to_dense()) if n < 20000 else None
+    for k in (nrhs, nrhs // 3):
+        ya, yb, x0, y0 = _both(h, k, 4)
+        # sums in another order where a part of one right-hand side remains
+        bound = 8 * n * 2.0 ** -53 * (A @ np.abs(x0) + np.abs(y0)) if A is not None else 1e-12 * np.abs(ya).max()
+        assert (np.abs(ya - yb) <= bound).all()
+    h.close()
