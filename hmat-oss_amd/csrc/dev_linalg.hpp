@@ -564,12 +564,11 @@ __device__ inline double group_sum_c(double v) {
 // (r < R) of G (and of V when kV); the loads use clamped rows and a select,
 // the columns are read once per round and written back after the rotation.
 // Requires rows (and cols when kV) <= R kG, kG == group_lanes(pairs, kLanes)
-// and tracked norms; floor_rel as 1e-30 in team_jacobi.  Without V (kV false) the caller recovers the right
+// and tracked norms.  Without V (kV false) the caller recovers the right
 // singular vectors from the input, as G_in^T U.
 template <int kLanes, int R, int kG, bool kV, typename PG>
 __device__ inline int team_jacobi_rows(PG G, int ldg, int rows, int cols, PG V, int ldv,
-                                       lptr<double> sh2, lptr<double> nrm, int max_sweeps, double tol2 = 1e-26,
-                                       double floor_rel = 1e-30) {
+                                       lptr<double> sh2, lptr<double> nrm, int max_sweeps, double tol2 = 1e-26) {
   const int tid = team_tid<kLanes>();
   if constexpr (kV) {
     for (int e = tid; e < cols * cols; e += kLanes) {
@@ -607,7 +606,7 @@ __device__ inline int team_jacobi_rows(PG G, int ldg, int rows, int cols, PG V, 
     team_sync<kLanes>();
     double f = 0.0;
     for (int c = 0; c < cols; ++c) f += nrm[c];
-    const double floor2 = floor_rel * f;
+    const double floor2 = 1e-30 * f;
     int rotated = 0;
     for (int rd = 0; rd < rounds; ++rd) {
       for (int pk = grp; pk < half; pk += ngrp) {
@@ -771,7 +770,7 @@ __device__ inline lptr<double> core_buffer() {
 // kG lanes per pair, kR rows per lane (rows <= kG kR), cols <= 128 / kG; W has
 // cols rounded up to even columns, ld rows >= kG kR, zero outside the matrix.
 template <int kG, int kR>
-__device__ inline void slot_jacobi(lptr<double> W, int ld, int cols, double tol2, double floor_rel) {
+__device__ inline void slot_jacobi(lptr<double> W, int ld, int cols, double tol2) {
   const int lane = threadIdx.x & (kWave - 1);
   const int h = (cols + 1) / 2, rounds = 2 * h - 1;
   const int i = lane / kG, sub = lane % kG;
@@ -803,7 +802,7 @@ __device__ inline void slot_jacobi(lptr<double> W, int ld, int cols, double tol2
       a = group_sum_c<kG>(a);
       b = group_sum_c<kG>(b);
       c2 = group_sum_c<kG>(c2);
-      if (sweep == 0 && rd == 0) floor2 = floor_rel * wave_sum(act && sub == 0 ? a + b : 0.0);
+      if (sweep == 0 && rd == 0) floor2 = 1e-30 * wave_sum(act && sub == 0 ? a + b : 0.0);
       const bool turn = c2 * c2 > tol2 * a * b && fabs(c2) > floor2;
       double t, c, s;
       jacobi_rot(a, b, c2, t, c, s);
@@ -868,7 +867,7 @@ __device__ inline int core_rows(lptr<double> G, int ldg, int rows, int cols, lpt
 }
 
 // (one wavefront; rows, cols <= kCoreMax)
-__device__ inline int wave_core_svd(lptr<double> G, int ldg, int rows, int cols, double tol2, double floor_rel) {
+__device__ inline int wave_core_svd(lptr<double> G, int ldg, int rows, int cols, double tol2) {
   const lptr<double> W = core_buffer();
   const int lane = threadIdx.x & (kWave - 1);
   int r;
@@ -876,12 +875,12 @@ __device__ inline int wave_core_svd(lptr<double> G, int ldg, int rows, int cols,
   if (rows <= 16) {
     r = cols <= 16 ? core_rows<16>(G, ldg, rows, cols, W, ld) : core_rows<32>(G, ldg, rows, cols, W, ld);
     __builtin_amdgcn_wave_barrier();
-    if (r > 1) slot_jacobi<8, 2>(W, ld, r, tol2, floor_rel);
+    if (r > 1) slot_jacobi<8, 2>(W, ld, r, tol2);
   } else {
     ld = 33;
     r = cols <= 24 ? core_rows<24>(G, ldg, rows, cols, W, ld) : core_rows<32>(G, ldg, rows, cols, W, ld);
     __builtin_amdgcn_wave_barrier();
-    if (r > 1) slot_jacobi<4, 8>(W, ld, r, tol2, floor_rel);
+    if (r > 1) slot_jacobi<4, 8>(W, ld, r, tol2);
   }
   __builtin_amdgcn_wave_barrier();
   for (int e = lane; e < rows * r; e += kWave) G[e % rows + e / rows * ldg] = W[e % rows + e / rows * ld];

@@ -167,16 +167,13 @@ __global__ void __launch_bounds__(kBlock, 2) k_svd_compress(const LeafDesc* desc
   for (int e = threadIdx.x; e < gr * gc; e += kBlock) W[e] = get(e % gr, e / gr);
   __syncthreads();
   const int r = gr <= 52 ? pivoted_rows<26>(gr, gc, tol, W, ldw) : pivoted_rows<50>(gr, gc, tol, W, ldw);
-  // pairs whose inner product is below 1e-16 eps^2 ||G||^2 turn a kept column by
-  // less than 1e-16
   const lptr<double> w3 = (lptr<double>)W;
-  const double floor_rel = fmax(1e-30, 1e-16 * eps * eps);
   if (r <= 32)
-    team_jacobi_rows<kBlock, 7, 16, false>(w3, ldw, gc, r, lptr<double>(nullptr), 0, (lptr<double>)sh2, (lptr<double>)sig, 40, 1e-26, floor_rel);
+    team_jacobi_rows<kBlock, 7, 16, false>(w3, ldw, gc, r, lptr<double>(nullptr), 0, (lptr<double>)sh2, (lptr<double>)sig, 40);
   else if (r <= 64)
-    team_jacobi_rows<kBlock, 13, 8, false>(w3, ldw, gc, r, lptr<double>(nullptr), 0, (lptr<double>)sh2, (lptr<double>)sig, 40, 1e-26, floor_rel);
+    team_jacobi_rows<kBlock, 13, 8, false>(w3, ldw, gc, r, lptr<double>(nullptr), 0, (lptr<double>)sh2, (lptr<double>)sig, 40);
   else
-    team_jacobi_rows<kBlock, 25, 4, false>(w3, ldw, gc, r, lptr<double>(nullptr), 0, (lptr<double>)sh2, (lptr<double>)sig, 40, 1e-26, floor_rel);
+    team_jacobi_rows<kBlock, 25, 4, false>(w3, ldw, gc, r, lptr<double>(nullptr), 0, (lptr<double>)sh2, (lptr<double>)sig, 40);
   sorted_norms(W, ldw, gc, r, sig, order);
   int k = find_k(sig, order, r, eps);
   if (k > d.cap) {

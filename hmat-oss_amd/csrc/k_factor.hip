@@ -1634,7 +1634,7 @@ __device__ void qr_finish(PV Va, int lda, int m, PV Vb, int ldb, int n, int K, c
       __syncthreads();
     }
     if (threadIdx.x < kWave) {
-      const int c = wave_core_svd(g, K, K, K, 1e-26, fmax(1e-30, 1e-16 * eps * eps));
+      const int c = wave_core_svd(g, K, K, K, 1e-26);
       if constexpr (kInLds) {
         const int k = wave_sorted_cut(g, K, K, c, w.sig, w.order, eps);
         if (threadIdx.x == 0) core_cut = k;
@@ -1880,7 +1880,7 @@ __device__ void gram_recompress(PV Va, int lda, PV Vb, int ldb, const FTask& t, 
   // rounding once scaled by the eps cut
   static_assert(kGramMaxK <= kCoreMax, "the core SVD of one wavefront");
   if (wid == 0) {
-    const int c = wave_core_svd(Cm, ra, ra, rb, kGramJacobiTol2, fmax(1e-30, 1e-16 * eps * eps));
+    const int c = wave_core_svd(Cm, ra, ra, rb, kGramJacobiTol2);
     const int k = wave_sorted_cut(Cm, ra, ra, c, sig, order, eps);
     if (lane < c) scale[lane] = 1.0 / sqrt(sig[lane]);
     if (lane == 0) ranks[2] = k;
@@ -2179,7 +2179,7 @@ __device__ void rkrk_body(const FTask& t, int k1, int k2, P ws, lptr<double> par
       for (int e = threadIdx.x; e < gr * gc; e += kBlock) Gin[e] = G[e];
       __syncthreads();
       if (threadIdx.x < kWave) {
-        const int c = wave_core_svd(G, gr, gr, gc, 1e-26, fmax(1e-30, 1e-16 * t.eps * t.eps));
+        const int c = wave_core_svd(G, gr, gr, gc, 1e-26);
         const int k = wave_sorted_cut(G, gr, gr, c, sig, order, t.eps);
         if (threadIdx.x == 0) {
           flag[0] = c;
