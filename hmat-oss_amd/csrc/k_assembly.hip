@@ -132,12 +132,13 @@ __device__ int pivoted_rows(int gr, int gc, double tol, double* W, int ldw) {
 
 // Truncated SVD of a small admissible leaf (compression.cpp:224-251).  The
 // block's numerical rank is well below its size, so it is first reduced to W
-// (pivoted_rows, cut at 1e-14 of its norm), and the one-sided Jacobi runs on
+// (pivoted_rows, cut at 1e-15 of its norm,
+// the level below which the Jacobi rotates nothing), and the one-sided Jacobi runs on
 // W's columns, already graded from the largest to the smallest, without
 // accumulating rotations: its columns become sigma_j v_j, and u_j = G v_j /
 // sigma_j from the block's entries evaluated once more (A B^T is then G's exact
 // projection on the kept v_j).  Bound: the serial steps of the reduction and
-// of the Jacobi rounds.  2,407 blocks of 98 x 98 (N = 50,000): 2.3 ms; 107 ms
+// of the Jacobi rounds.  2,407 blocks of 98 x 98 (N = 50,000): 2.8 ms; 107 ms
 // with the Jacobi on the whole blocks and its rotations accumulated.
 template <typename T>
 __global__ void __launch_bounds__(kBlock, 2) k_svd_compress(const LeafDesc* desc, const int* list,
@@ -163,7 +164,7 @@ __global__ void __launch_bounds__(kBlock, 2) k_svd_compress(const LeafDesc* desc
     return tab ? tab[i + (size_t)j * d.m] : entry(rp, cp, kp, d.r0 + i, d.c0 + j);
   };
   const int ldw = gc | 1;  // odd: the rounds' strided accesses spread over the banks
-  const double tol = fmin(1e-14, 1e-2 * eps);
+  const double tol = fmin(1e-15, 1e-2 * eps);
   for (int e = threadIdx.x; e < gr * gc; e += kBlock) W[e] = get(e % gr, e / gr);
   __syncthreads();
   const int r = gr <= 52 ? pivoted_rows<26>(gr, gc, tol, W, ldw) : pivoted_rows<50>(gr, gc, tol, W, ldw);
