@@ -983,6 +983,10 @@ int hmx_solve_refined_device(hmat_matrix_t* h, double* b, int nrhs, double tol, 
   return rc ? -1 : it;
 }
 
+int hmx_release_memory(void) {
+  return guard([] { hmx::release_kept_memory(); });
+}
+
 int hmx_run_batch(hmat_matrix_t** ms, hmat_assemble_context_t** ctx, int count, int algo,
                   int mixed, double tol, double** b, const int* nrhs, int threads,
                   double* seconds, int* status) {

@@ -122,6 +122,8 @@ int orth(rocblas_handle h, const double* Y, int rows, int p, Work& w, hipStream_
 void Matrix::compress_giants(const std::vector<int>& list, PointSet rp, PointSet cp,
                              KernelParams kp, double eps) {
   if (list.empty()) return;
+  // rocBLAS and rocSOLVER take their workspaces from the driver
+  release_kept_memory();
   BlasHandle H(stream);
   DevBuf A, Y, Z, sd, sl;
   Work w;

@@ -181,6 +181,7 @@ _EXPORTS = {
     "hmat_mi355x_kernel_compute": (None, [_vp, C.c_int, C.c_int, _vp]),
     "hmx_last_error": (C.c_char_p, []),
     "hmx_gemv_device": (C.c_int, [_vp, C.c_int, C.c_double, _vp, C.c_double, _vp, C.c_int]),
+    "hmx_release_memory": (C.c_int, []),
     "hmx_gemv_device_noalloc": (C.c_int, [_vp, C.c_int, C.c_double, _vp, C.c_double, _vp,
                                           C.c_int]),
     "hmx_run_batch": (C.c_int, [_vp, _vp, C.c_int, C.c_int, C.c_int, C.c_double, _vp, _vp,
@@ -234,6 +235,12 @@ def interface(value_type=HMAT_DOUBLE_PRECISION):
     it = hmat_interface_t()
     lib.hmat_init_mi355x_interface(C.byref(it), value_type)
     return it
+
+
+def release_memory():
+    """Gives the device buffers kept from closed matrices back to the driver
+    (up to an eighth of the device's memory, for torch or another allocator)."""
+    _check(load().hmx_release_memory(), "hmx_release_memory")
 
 
 class ClusterTree:

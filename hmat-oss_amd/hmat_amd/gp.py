@@ -26,7 +26,7 @@ import math
 import numpy as np
 
 from . import (FACT_LLT, HMatrix, KERNEL_EXPONENTIAL, KERNEL_EXPONENTIAL_DLENGTH, KERNEL_GAUSSIAN,
-               KERNEL_GAUSSIAN_DLENGTH)
+               KERNEL_GAUSSIAN_DLENGTH, release_memory)
 
 _DERIVATIVE = {KERNEL_EXPONENTIAL: KERNEL_EXPONENTIAL_DLENGTH,
                KERNEL_GAUSSIAN: KERNEL_GAUSSIAN_DLENGTH}
@@ -36,6 +36,18 @@ def rademacher(n, count, seed):
     """count seeded Rademacher vectors (n x count, entries +-1, float64)."""
     rng = np.random.default_rng(seed)
     return np.where(rng.integers(0, 2, size=(n, count)) == 0, -1.0, 1.0)
+
+
+def _with_memory(step):
+    """step(), and once more after giving back the buffers kept from closed
+    matrices if torch has run out of device memory."""
+    import torch
+    try:
+        return step()
+    except torch.OutOfMemoryError:
+        pass
+    release_memory()
+    return step()
 
 
 class _State:
@@ -51,6 +63,9 @@ class _State:
 
     def solve(self, b_user, tol=None):
         """K^{-1} b (user numbering, N x nrhs float64 torch tensor on the device)."""
+        return _with_memory(lambda: self._solve(b_user, tol))
+
+    def _solve(self, b_user, tol):
         import torch
         bh = b_user[torch.as_tensor(self.idx, device=b_user.device)]
         bd = bh.T.contiguous()
@@ -103,14 +118,18 @@ class GPNegLogLikelihood:
                     D = HMatrix(st.tree, lowrank_eps=st.eps)
                     D.assemble(kind=_DERIVATIVE[st.kind], length=st.length, nugget=0.0, eps=st.eps)
                     # dK/dl applied to [alpha, Z] in one H-gemv (hmat numbering)
-                    X = torch.cat([alpha, Z], dim=1)
                     ih = torch.as_tensor(st.idx, device=dev)
-                    xd = X[ih].T.contiguous()
-                    yd = torch.zeros_like(xd)
-                    D.gemv_device(xd.data_ptr(), yd.data_ptr(), xd.shape[0])
-                    torch.cuda.synchronize()
-                    DX = torch.empty_like(X)
-                    DX[ih] = yd.T
+
+                    def product():
+                        X = torch.cat([alpha, Z], dim=1)
+                        xd = X[ih].T.contiguous()
+                        yd = torch.zeros_like(xd)
+                        D.gemv_device(xd.data_ptr(), yd.data_ptr(), xd.shape[0])
+                        torch.cuda.synchronize()
+                        DX = torch.empty_like(X)
+                        DX[ih] = yd.T
+                        return DX
+                    DX = _with_memory(product)
                     D.close()
                     d_alpha = float((alpha[:, 0] * DX[:, 0]).sum())
                     tr_l = float((S * DX[:, 1:]).sum()) / ctx.probes

@@ -141,6 +141,13 @@ HMAT_API int hmx_stats(hmat_matrix_t *m, double *out);
  * set, the *_device entry points are stream-ordered and do not synchronise. */
 HMAT_API int hmx_set_stream(hmat_matrix_t *m, void *stream);
 
+/* No counterpart in hmat-oss.  Device buffers of destroyed matrices are kept
+ * for the next ones, up to an eighth of the device's memory (it is given back
+ * by itself when an allocation of this library fails, and by the interface's
+ * finalize).  This call gives them back at once, for another allocator of the
+ * process that runs out of memory. */
+HMAT_API int hmx_release_memory(void);
+
 /* Upper bound on Rk panel capacity used for new matrices (default 160). */
 HMAT_API void hmx_set_rank_capacity(int cap);
 

@@ -5,7 +5,7 @@
   product equals that of the matrix's own leaves (4 N u |A| |x|), every solve
   leaves the compression's residual.
 * A matrix closed with products queued on the caller's stream.
-* hmat_interface_t.finalize gives the kept buffers back.
+* hmat_interface_t.finalize and hmx_release_memory give the kept buffers back.
 * Blocks whose ACA needs more columns than its first room (32) run again: at
   eps 1e-13 the ranks are above it and the matrix is within 1,000 eps of the
   exact kernel's."""
@@ -62,6 +62,9 @@ def test_buffers_reused_and_given_back():
     assert hmat_amd.interface().finalize() == 0
     assert torch.cuda.mem_get_info()[0] > before
     _one(1000, 8, 64, factor=True)
+    before = torch.cuda.mem_get_info()[0]
+    hmat_amd.release_memory()
+    assert torch.cuda.mem_get_info()[0] > before
 
 
 def test_aca_rooms():
