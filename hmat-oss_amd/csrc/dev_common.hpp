@@ -91,9 +91,10 @@ __host__ __device__ inline double kernel_value(const KernelParams& k, double dx,
 
 // ---- address spaces ----------------------------------------------------------
 // Pointers read from memory (task records) or passed between functions are
-// generic, and their accesses flat: slower, and counted with the LDS accesses,
-// so that every wait for LDS also waits for the loads in flight.  Operands
-// known to be in global memory or in LDS are cast to these types first.
+// generic, and their accesses flat: counted with the LDS accesses, so that
+// every wait for LDS also waits for the loads in flight.  Operands known to be
+// in global memory or in LDS are cast to these types first.  An LDS pointer is
+// never tested against null: 0 is the address of an array there.
 template <typename T>
 struct InGlobal {
   typedef T __attribute__((address_space(1))) type;

@@ -395,7 +395,7 @@ constexpr int kJacobiMaxCols = 256;  // columns whose norms the Jacobi keeps in 
 // |g| > 1e-30 ||G||_F^2 (columns
 // at rounding level of ||G|| carry nothing for the truncation thresholds used
 // here).  Returns the number of sweeps.  'sh2' is 2 + kWaves shared doubles of
-// scratch (workgroup team only); 'nrm' holds cols doubles or is null.
+// scratch (workgroup team only); 'nrm' holds kJacobiMaxCols doubles.
 // Rotation of one-sided Jacobi zeroing the inner product c2 of two columns
 // with squared norms a and b: t = tan = sign(d) 2 c2 / (|d| + sqrt(d^2 + 4 c2^2))
 // with d = b - a, c = 1 / sqrt(1 + t^2), s = c t.  d and 2 c2 are first
@@ -421,11 +421,15 @@ __device__ inline void jacobi_rot(double a, double b, double c2, double& t, doub
   s = y * t;
 }
 
-template <int kLanes, typename PG>
+// (kV and 'track' and not null pointers: the address of an LDS array can be 0,
+// which is what a null LDS pointer is.  The norms' array sits there in FADD, and
+// while it was tested against null the untracked loop ran: 98 x 98 sums of 64
+// columns took 4.0 ms instead of 2.9)
+template <int kLanes, bool kV, typename PG>
 __device__ inline int team_jacobi(PG G, int ldg, int rows, int cols, PG V, int ldv,
                                   lptr<double> sh2, lptr<double> nrm, int max_sweeps, double tol2 = 1e-26) {
   const int tid = team_tid<kLanes>();
-  if (V != nullptr)
+  if constexpr (kV)
     for (int e = tid; e < cols * cols; e += kLanes) {
       const int i = e % cols, j = e / cols;
       V[i + (size_t)j * ldv] = (i == j) ? 1.0 : 0.0;
@@ -442,7 +446,7 @@ __device__ inline int team_jacobi(PG G, int ldg, int rows, int cols, PG V, int l
   if (kLanes >= kWave && rows >= 128 && g0 < 16) g0 = 16;
   const int g = g0, ngrp = kLanes / g, grp = tid / g, sub = tid % g;
   // without scratch for every column the norms are recomputed pair by pair
-  const bool track = nrm != nullptr && cols <= kJacobiMaxCols;
+  const bool track = cols <= kJacobiMaxCols;
   int sweep = 0;
   for (; sweep < max_sweeps; ++sweep) {
     // column norms (and the Frobenius floor) afresh each sweep
@@ -462,7 +466,7 @@ __device__ inline int team_jacobi(PG G, int ldg, int rows, int cols, PG V, int l
         const double x = G[e % rows + (size_t)(e / rows) * ldg];
         f += x * x;
       }
-      f = team_sum<kLanes>(f, sh2 ? sh2 + 2 : lptr<double>(nullptr));
+      f = team_sum<kLanes>(f, sh2 + 2);
     }
     const double floor2 = 1e-30 * f;
     int rotated = 0;
@@ -512,7 +516,7 @@ __device__ inline int team_jacobi(PG G, int ldg, int rows, int cols, PG V, int l
           gp[i] = c * x - s * y;
           gq[i] = s * x + c * y;
         }
-        if (V != nullptr) {
+        if constexpr (kV) {
           const PG vp = V + (size_t)p * ldv;
           const PG vq = V + (size_t)q * ldv;
           for (int i = sub; i < cols; i += g) {
@@ -698,33 +702,24 @@ __device__ inline int team_jacobi_rows(PG G, int ldg, int rows, int cols, PG V, 
   return sweep;
 }
 
-// Dispatch on the group size and rows per lane; V == nullptr skips the
-// accumulation of V.  Shapes outside the instantiated ones use team_jacobi.
+// Dispatch on the group size and rows per lane; without kV the accumulation of
+// V is left out.  Shapes outside the instantiated ones use team_jacobi.
 template <int kLanes, bool kV, typename PG>
-__device__ inline int team_jacobi_sel(PG G, int ldg, int rows, int cols, PG V, int ldv,
+__device__ inline int team_jacobi_any(PG G, int ldg, int rows, int cols, PG V, int ldv,
                                       lptr<double> sh2, lptr<double> nrm, int max_sweeps, double tol2 = 1e-26) {
-  const int half = ((cols + 1) & ~1) / 2;
-  const int g = group_lanes(half, kLanes);
-  const int span = kV ? (rows > cols ? rows : cols) : rows;
-  const int need = (span + g - 1) / g;
+  if (cols <= kJacobiMaxCols && cols >= 2 && rows >= 1) {
+    const int half = ((cols + 1) & ~1) / 2;
+    const int g = group_lanes(half, kLanes);
+    const int span = kV ? (rows > cols ? rows : cols) : rows;
+    const int need = (span + g - 1) / g;
 #define HMX_JR(G_, R_)                                                                             \
   if (g == G_ && need <= R_)                                                                       \
     return team_jacobi_rows<kLanes, R_, G_, kV>(G, ldg, rows, cols, V, ldv, sh2, nrm, max_sweeps, tol2);
-  HMX_JR(16, 2)
-  HMX_JR(8, 8)
+    HMX_JR(16, 2)
+    HMX_JR(8, 8)
 #undef HMX_JR
-  return team_jacobi<kLanes>(G, ldg, rows, cols, V, ldv, sh2, nrm, max_sweeps, tol2);
-}
-
-template <int kLanes, typename PG>
-__device__ inline int team_jacobi_any(PG G, int ldg, int rows, int cols, PG V, int ldv,
-                                      lptr<double> sh2, lptr<double> nrm, int max_sweeps, double tol2 = 1e-26) {
-  if (nrm != nullptr && cols <= kJacobiMaxCols && cols >= 2 && rows >= 1) {
-    if (V != nullptr)
-      return team_jacobi_sel<kLanes, true>(G, ldg, rows, cols, V, ldv, sh2, nrm, max_sweeps, tol2);
-    return team_jacobi_sel<kLanes, false>(G, ldg, rows, cols, V, ldv, sh2, nrm, max_sweeps, tol2);
   }
-  return team_jacobi<kLanes>(G, ldg, rows, cols, V, ldv, sh2, nrm, max_sweeps, tol2);
+  return team_jacobi<kLanes, kV>(G, ldg, rows, cols, V, ldv, sh2, nrm, max_sweeps, tol2);
 }
 
 // The norms of the workgroup's Jacobi: one array for every instantiation.
@@ -733,13 +728,12 @@ __device__ inline lptr<double> jacobi_norms() {
   return (lptr<double>)nrm;
 }
 
-// Workgroup version used by the existing call sites (cols <= kJacobiMaxCols);
-// V == nullptr leaves V out.
-template <typename PG>
+// Workgroup version (cols <= kJacobiMaxCols); without kV, V is not touched.
+template <bool kV, typename PG>
 __device__ inline void jacobi_svd(PG G, int ldg, int rows, int cols, PG V, int ldv,
                                   int* /*flag*/, int max_sweeps = 40, double tol2 = 1e-26) {
   __shared__ double sh2[2 + kWaves];
-  team_jacobi_any<kBlock>(G, ldg, rows, cols, V, ldv, (lptr<double>)sh2, jacobi_norms(), max_sweeps, tol2);
+  team_jacobi_any<kBlock, kV>(G, ldg, rows, cols, V, ldv, (lptr<double>)sh2, jacobi_norms(), max_sweeps, tol2);
 }
 
 // ---------------------------------------------------------------------------

@@ -170,11 +170,11 @@ __global__ void __launch_bounds__(kBlock, 2) k_svd_compress(const LeafDesc* desc
   const int r = gr <= 52 ? pivoted_rows<26>(gr, gc, tol, W, ldw) : pivoted_rows<50>(gr, gc, tol, W, ldw);
   const lptr<double> w3 = (lptr<double>)W;
   if (r <= 32)
-    team_jacobi_rows<kBlock, 7, 16, false>(w3, ldw, gc, r, lptr<double>(nullptr), 0, (lptr<double>)sh2, (lptr<double>)sig, 40);
+    team_jacobi_rows<kBlock, 7, 16, false>(w3, ldw, gc, r, w3, 0, (lptr<double>)sh2, (lptr<double>)sig, 40);
   else if (r <= 64)
-    team_jacobi_rows<kBlock, 13, 8, false>(w3, ldw, gc, r, lptr<double>(nullptr), 0, (lptr<double>)sh2, (lptr<double>)sig, 40);
+    team_jacobi_rows<kBlock, 13, 8, false>(w3, ldw, gc, r, w3, 0, (lptr<double>)sh2, (lptr<double>)sig, 40);
   else
-    team_jacobi_rows<kBlock, 25, 4, false>(w3, ldw, gc, r, lptr<double>(nullptr), 0, (lptr<double>)sh2, (lptr<double>)sig, 40);
+    team_jacobi_rows<kBlock, 25, 4, false>(w3, ldw, gc, r, w3, 0, (lptr<double>)sh2, (lptr<double>)sig, 40);
   sorted_norms(W, ldw, gc, r, sig, order);
   int k = find_k(sig, order, r, eps);
   if (k > d.cap) {
@@ -541,7 +541,7 @@ __device__ int truncate_panels(double* A, int m, double* B, int n, int k, const 
     w.g[i + (size_t)j * k] = s;
   }
   __syncthreads();
-  jacobi_svd((gptr<double>)w.g, k, k, k, (gptr<double>)w.v, k, flag);
+  jacobi_svd<true>((gptr<double>)w.g, k, k, k, (gptr<double>)w.v, k, flag);
   sorted_norms(w.g, k, k, k, w.sig, w.order);
   int nk = find_k(w.sig, w.order, k, eps);
   if (nk > cap) {

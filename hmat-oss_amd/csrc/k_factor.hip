@@ -1325,9 +1325,9 @@ template <typename T>
 __device__ int dense_to_rk(double* G, bool in_lds, int gr, int gc, bool tr, double* V, double* sig, int* order,
                            double eps, RkRef out, int* overflow, int* flag) {
   if (in_lds)
-    jacobi_svd((lptr<double>)G, gr, gr, gc, (lptr<double>)V, gc, flag);
+    jacobi_svd<true>((lptr<double>)G, gr, gr, gc, (lptr<double>)V, gc, flag);
   else
-    jacobi_svd((gptr<double>)G, gr, gr, gc, (gptr<double>)V, gc, flag);
+    jacobi_svd<true>((gptr<double>)G, gr, gr, gc, (gptr<double>)V, gc, flag);
   sorted_norms(G, gr, gr, gc, sig, order);
   int k = find_k(sig, order, gc, eps);
   if (k > out.cap) {
@@ -1648,16 +1648,16 @@ __device__ void qr_finish(PV Va, int lda, int m, PV Vb, int ldb, int n, int K, c
       __syncthreads();
     }
   } else if constexpr (kInLds) {
-    jacobi_svd(w.g, K, K, K, P(nullptr), K, flag);
+    jacobi_svd<false>(w.g, K, K, K, w.g, K, flag);
   } else if (K * K <= kShDoubles) {
     // the rounds' loads and stores hit LDS instead of the L2
     for (int e = threadIdx.x; e < K * K; e += kBlock) stage[e] = w.g[e];
     __syncthreads();
-    jacobi_svd(stage, K, K, K, lptr<double>(nullptr), K, flag);
+    jacobi_svd<false>(stage, K, K, K, stage, K, flag);
     for (int e = threadIdx.x; e < K * K; e += kBlock) w.g[e] = stage[e];
     __syncthreads();
   } else {
-    jacobi_svd(w.g, K, K, K, P(nullptr), K, flag);
+    jacobi_svd<false>(w.g, K, K, K, w.g, K, flag);
     __syncthreads();
   }
   int nk;
@@ -2198,7 +2198,7 @@ __device__ void rkrk_body(const FTask& t, int k1, int k2, P ws, lptr<double> par
       done = true;
     }
   if (!done) {
-    jacobi_svd(G, gr, gr, gc, V, gc, flag);
+    jacobi_svd<true>(G, gr, gr, gc, V, gc, flag);
     sorted_norms(G, gr, gr, gc, sig, order);
   }
   int nk = done ? flag[1] : find_k(sig, order, r, t.eps);
