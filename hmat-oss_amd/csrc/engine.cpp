@@ -431,16 +431,20 @@ void Matrix::assemble_pass(const KernelSpec& k, const CompressionSpec& comp) {
   // ACA blocks, the largest first, in launches bounded by a workspace budget.
   // Most blocks stop far below the room their leaf's capacity would give
   // (ranks of 5 to 25 in panels of 320 columns, 16 GB of workspace at
-  // N = 50,000): a first round with panels of kAcaRoom columns, and the blocks
+  // N = 50,000): a first round with panels of 'room' columns, and the blocks
   // that fill them run again, from their start, with four times the room up to
-  // their full one.  The real form of complex blocks has ranks above a hundred and
-  // starts with its full room: rooms of 128 took the assembly of 20,000 Helmholtz
-  // points from 411 to 644 ms.
-  constexpr int kAcaRoom = 32;
+  // their full one.  32 columns hold what eps = 1e-4 needs (2-D and 3-D clouds of
+  // up to 50,000 points); below it a second run costs more than the memory of
+  // 128 columns: 50,000 points at 1e-8 28.3 ms of ACA with 32, 18.2 with 128 as
+  // with the full room, at 1e-12 92 against 77 ms, a cloud of 30,000 at 1e-5
+  // 19.0 against 12.7.  The real form of complex blocks has ranks above a hundred
+  // and starts with its full room: rooms of 128 took the assembly of 20,000
+  // Helmholtz points from 411 to 644 ms.
+  const int first_room = comp.eps >= 0.99e-4 ? 32 : 128;
   std::vector<AcaTask> acat;
   for (int l : aca) {
     const int full_room = aca_kmax(s64.hdesc[l]);
-    const int room = embedded ? full_room : std::min(full_room, kAcaRoom);
+    const int room = embedded ? full_room : std::min(full_room, first_room);
     acat.push_back(AcaTask{l, room, 0, -1, room == full_room});
   }
   const int64_t budget = acat.empty() ? 0 : aca_budget_doubles();

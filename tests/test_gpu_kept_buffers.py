@@ -6,9 +6,8 @@
   leaves the compression's residual.
 * A matrix closed with products queued on the caller's stream.
 * hmat_interface_t.finalize and hmx_release_memory give the kept buffers back.
-* Blocks whose ACA needs more columns than its first room (32) run again: at
-  eps 1e-13 the ranks are above it and the matrix is within 1,000 eps of the
-  exact kernel's."""
+* Blocks whose ACA needs more columns than its first room (32 at eps 1e-4, 128
+  below) run again: the matrix is within 1,000 eps of the exact kernel's."""
 import threading
 
 import numpy as np
@@ -78,6 +77,22 @@ def test_aca_rooms():
     P = pts[t.indices]
     K = np.exp(-np.sqrt(((P[:, None] - P[None]) ** 2).sum(axis=2)) / 0.5)
     assert np.linalg.norm(h.to_dense() - K) <= 1e-10 * np.linalg.norm(K)
+    h.close()
+
+
+@pytest.mark.parametrize("eps,length,above", [(1e-4, 0.05, 32), (1e-9, 0.1, 128)])
+def test_aca_rooms_filled(eps, length, above):
+    n = 3000
+    pts = np.random.default_rng(6).random((n, 3)) * [1.0, 1.0, 2.0]
+    t = hmat_amd.ClusterTree(pts, 100)
+    h = hmat_amd.HMatrix(t, eta=100.0, lowrank_eps=eps)
+    h.assemble(length=length, nugget=0.0, eps=eps)
+    tab = h.leaf_table()
+    print("largest rank", tab[:, 5].max(), flush=True)
+    assert tab[(tab[:, 4] == 1) & (np.maximum(tab[:, 0], tab[:, 1]) >= 100)][:, 5].max() > above
+    P = pts[t.indices]
+    K = np.exp(-np.sqrt(((P[:, None] - P[None]) ** 2).sum(axis=2)) / length)
+    assert np.linalg.norm(h.to_dense() - K) <= 1e3 * eps * np.linalg.norm(K)
     h.close()
 
 
