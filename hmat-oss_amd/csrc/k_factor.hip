@@ -1617,38 +1617,24 @@ template <typename T, typename PV, typename P, typename PI>
 __device__ void qr_finish(PV Va, int lda, int m, PV Vb, int ldb, int n, int K, const QrScratch<P, PI>& w,
                           double eps, RkRef out, int* overflow, int* flag, lptr<double> stage) {
   constexpr bool kInLds = std::is_same_v<P, lptr<double>>;
-  __shared__ int core_rank, core_cut;
-  int r = K;  // columns of the rotated core
+  __shared__ int core_cut;
   // one-sided Jacobi on G without V: G_in (kept in w.v) gives the right side
   // afterwards as G_in^T U, so the rounds only rotate G
   for (int e = threadIdx.x; e < K * K; e += kBlock) w.v[e] = w.g[e];
   __syncthreads();
-  if (K <= kCoreMax) {
-    // in LDS, a global core through its free part
-    lptr<double> g;
-    if constexpr (kInLds) {
-      g = w.g;
-    } else {
-      g = stage;
-      for (int e = threadIdx.x; e < K * K; e += kBlock) g[e] = w.g[e];
-      __syncthreads();
-    }
-    if (threadIdx.x < kWave) {
-      const int c = wave_core_svd(g, K, K, K, 1e-26);
-      if constexpr (kInLds) {
-        const int k = wave_sorted_cut(g, K, K, c, w.sig, w.order, eps);
+  bool cut = false;
+  if constexpr (kInLds) {
+    if (K <= kCoreMax) {
+      if (threadIdx.x < kWave) {
+        const int c = wave_core_svd(w.g, K, K, K, 1e-26);
+        const int k = wave_sorted_cut(w.g, K, K, c, w.sig, w.order, eps);
         if (threadIdx.x == 0) core_cut = k;
       }
-      if (threadIdx.x == 0) core_rank = c;
-    }
-    __syncthreads();
-    r = core_rank;
-    if constexpr (!kInLds) {
-      for (int e = threadIdx.x; e < K * r; e += kBlock) w.g[e] = g[e];
       __syncthreads();
+      cut = true;
+    } else {
+      jacobi_svd<false>(w.g, K, K, K, w.g, K, flag);
     }
-  } else if constexpr (kInLds) {
-    jacobi_svd<false>(w.g, K, K, K, w.g, K, flag);
   } else if (K * K <= kShDoubles) {
     // the rounds' loads and stores hit LDS instead of the L2
     for (int e = threadIdx.x; e < K * K; e += kBlock) stage[e] = w.g[e];
@@ -1661,11 +1647,11 @@ __device__ void qr_finish(PV Va, int lda, int m, PV Vb, int ldb, int n, int K, c
     __syncthreads();
   }
   int nk;
-  if (kInLds && K <= kCoreMax) {
+  if (cut) {
     nk = core_cut;
   } else {
-    sorted_norms(w.g, K, K, r, w.sig, w.order);
-    nk = find_k(w.sig, w.order, r, eps);
+    sorted_norms(w.g, K, K, K, w.sig, w.order);
+    nk = find_k(w.sig, w.order, K, eps);
   }
   if (nk > out.cap) {
     if (threadIdx.x == 0) atomicOr(overflow, 1);
