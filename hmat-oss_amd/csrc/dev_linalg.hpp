@@ -756,9 +756,12 @@ __device__ inline void jacobi_svd(PG G, int ldg, int rows, int cols, PG V, int l
 // ---------------------------------------------------------------------------
 constexpr int kCoreMax = 32;
 
-__device__ inline lptr<double> core_buffer() {
-  __shared__ double w[kCoreMax * (kCoreMax + 1)];
-  return (lptr<double>)w;
+// doubles of W for a core of rows x cols: odd leading dimensions spread the
+// columns' rows over the banks; an even number of columns
+__host__ __device__ constexpr int core_ld(int rows) { return rows <= 16 ? 17 : 33; }
+__host__ __device__ constexpr int core_work(int rows, int cols) {
+  const int c = rows < cols ? rows : cols;
+  return core_ld(rows) * (c + (c & 1));
 }
 
 // kG lanes per pair, kR rows per lane (rows <= kG kR), cols <= 128 / kG; W has
@@ -860,18 +863,15 @@ __device__ inline int core_rows(lptr<double> G, int ldg, int rows, int cols, lpt
   return s;
 }
 
-// (one wavefront; rows, cols <= kCoreMax)
-__device__ inline int wave_core_svd(lptr<double> G, int ldg, int rows, int cols, double tol2) {
-  const lptr<double> W = core_buffer();
-  const int lane = threadIdx.x & (kWave - 1);
+// (one wavefront; rows, cols <= kCoreMax; W: core_work(rows, cols) doubles)
+__device__ inline int wave_core_svd(lptr<double> G, int ldg, int rows, int cols, lptr<double> W, double tol2) {
+  const int lane = threadIdx.x & (kWave - 1), ld = core_ld(rows);
   int r;
-  int ld = 17;  // odd: the columns' rows spread over the banks
   if (rows <= 16) {
     r = cols <= 16 ? core_rows<16>(G, ldg, rows, cols, W, ld) : core_rows<32>(G, ldg, rows, cols, W, ld);
     __builtin_amdgcn_wave_barrier();
     if (r > 1) slot_jacobi<8, 2>(W, ld, r, tol2);
   } else {
-    ld = 33;
     r = cols <= 24 ? core_rows<24>(G, ldg, rows, cols, W, ld) : core_rows<32>(G, ldg, rows, cols, W, ld);
     __builtin_amdgcn_wave_barrier();
     if (r > 1) slot_jacobi<4, 8>(W, ld, r, tol2);

@@ -1015,7 +1015,7 @@ __global__ void __launch_bounds__(kBlock) k_hodlr(const FTask* tasks, double* ws
 // Rows (mode 0) / columns (modes 1, 2) of X are independent: a task is cut
 // into tiles of kTrsmCols of them, one workgroup each.
 // ---------------------------------------------------------------------------
-constexpr int kShDoubles = 18432;  // 144 KiB of LDS per workgroup, beside the core SVD's buffer
+constexpr int kShDoubles = 19456;  // 152 KiB of LDS per workgroup
 
 // A wavefront solves 16 independent rows / columns of X on its own: X^T (mode
 // 0) or X is cut into 16 x 16 blocks that stay in registers in the layout in
@@ -1371,8 +1371,14 @@ struct QrScratch {
 using LdsScratch = QrScratch<lptr<double>, lptr<int>>;
 using GlobalScratch = QrScratch<gptr<double>, gptr<int>>;
 
-// doubles of the scratch above
-__device__ inline int64_t qr_core(int K) { return 6 * (int64_t)K * K + 5 * (int64_t)K; }
+// doubles of the scratch above.  The core SVD of up to kCoreMax columns works in
+// x and w, which are free then; where they are too small (K below 10, and 17) it
+// goes past their end.
+__device__ inline int64_t qr_core(int K) {
+  const int64_t K2 = (int64_t)K * K;
+  const int64_t past = K <= kCoreMax ? core_work(K, K) - 2 * K2 : 0;
+  return 6 * K2 + 5 * (int64_t)K + (past > 0 ? past : 0);
+}
 
 template <typename W, typename P>
 __device__ inline W carve_qr(P core, int K) {
@@ -1626,7 +1632,7 @@ __device__ void qr_finish(PV Va, int lda, int m, PV Vb, int ldb, int n, int K, c
   if constexpr (kInLds) {
     if (K <= kCoreMax) {
       if (threadIdx.x < kWave) {
-        const int c = wave_core_svd(w.g, K, K, K, 1e-26);
+        const int c = wave_core_svd(w.g, K, K, K, w.x, 1e-26);
         const int k = wave_sorted_cut(w.g, K, K, c, w.sig, w.order, eps);
         if (threadIdx.x == 0) core_cut = k;
       }
@@ -1726,8 +1732,8 @@ __device__ void qr_global(gptr<double> Va, int m, gptr<double> Vb, int n, int K,
 // Widest sum in this form.  Squaring the panels' condition costs accuracy that
 // wider sums, which come with tight cuts, do not have: with 33 to 40 columns and
 // eps = 1e-7 the result was 3.5e-7 off instead of 1e-7, two ranks short (at 1e-8
-// 28 to 36 times the best error, against 5 to 7 times through Householder QR,
-// which takes 1,100 us there instead of 550).
+// 19 to 36 times the best error, against 5 to 7 times through Householder QR;
+// 256 sums of 33 columns and 100 rows take 620 us that way, 570 in this form).
 constexpr int kGramMaxK = kColsMax;
 constexpr double kGramTol = 1e-13;
 constexpr double kGramJacobiTol2 = 1e-16;
@@ -1864,9 +1870,10 @@ __device__ void gram_recompress(PV Va, int lda, PV Vb, int ldb, const FTask& t, 
   __syncthreads();
   // columns orthogonal to 1e-8 of their norms: far below the FP32 data's
   // rounding once scaled by the eps cut
+  // (core_work(32, 32) is less than the Gram tiles' part, core_work(16, 16) too)
   static_assert(kGramMaxK <= kCoreMax, "the core SVD of one wavefront");
   if (wid == 0) {
-    const int c = wave_core_svd(Cm, ra, ra, rb, kGramJacobiTol2);
+    const int c = wave_core_svd(Cm, ra, ra, rb, part, kGramJacobiTol2);
     const int k = wave_sorted_cut(Cm, ra, ra, c, sig, order, eps);
     if (lane < c) scale[lane] = 1.0 / sqrt(sig[lane]);
     if (lane == 0) ranks[2] = k;
@@ -2160,12 +2167,13 @@ __device__ void rkrk_body(const FTask& t, int k1, int k2, P ws, lptr<double> par
   bool done = false;
   if constexpr (std::is_same_v<P, lptr<double>>)
     if (gr <= kCoreMax) {
-      // V (gc x r) = G_in^T U with the copy of G kept behind the output factors
-      const P Gin = sig + gc + gc + (gc & 1) + (size_t)(gr + gc) * gc;
+      // V (gc x r) = G_in^T U with the copy of G kept behind the output factors,
+      // and behind it the core SVD's work
+      const P Gin = sig + gc + gc + (gc & 1) + (size_t)(gr + gc) * gc, W = Gin + gr * gc;
       for (int e = threadIdx.x; e < gr * gc; e += kBlock) Gin[e] = G[e];
       __syncthreads();
       if (threadIdx.x < kWave) {
-        const int c = wave_core_svd(G, gr, gr, gc, 1e-26);
+        const int c = wave_core_svd(G, gr, gr, gc, W, 1e-26);
         const int k = wave_sorted_cut(G, gr, gr, c, sig, order, t.eps);
         if (threadIdx.x == 0) {
           flag[0] = c;
@@ -2229,7 +2237,8 @@ __global__ void __launch_bounds__(kBlock) k_rkrk(const FTask* tasks, double* wsb
   const int64_t need = (int64_t)gr * gc + (int64_t)gc * gc + 2 * gc + 1;
   // SVD scratch, then the output factors (at most (gr + gc) x gc)
   const auto s3 = (lptr<double>)sh;
-  if (need + (int64_t)(gr + gc) * gc + (int64_t)gr * gc <= kShDoubles)
+  const int64_t core = gr <= kCoreMax ? (int64_t)gr * gc + core_work(gr, gc) : 0;
+  if (need + (int64_t)(gr + gc) * gc + core <= kShDoubles)
     rkrk_body<T, lptr<double>, lptr<int>>(t, k1, k2, s3, s3 + need, kShDoubles - need, overflow, flag);
   else
     rkrk_body<T, gptr<double>, gptr<int>>(t, k1, k2, (gptr<double>)(wsbase + t.ws), s3, kShDoubles, overflow, flag);
