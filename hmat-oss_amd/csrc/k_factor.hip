@@ -1,7 +1,8 @@
 // Batched task kernels of the H-LLt factorisation and the H-triangular solves.
 // Each launch processes the tasks of one type in one dependency wave; the
-// tasks of a launch are independent.  Dense arithmetic runs in the storage
-// type T (FP64 or FP32); QR/SVD of the recompressions run in FP64.
+// tasks of a launch are independent.  GEMM, LDLt, acaFull and the elementwise
+// tasks run in the storage type T (FP64 or FP32); POTRF and GETRF of leaves of up
+// to 128 rows, TRSM and the QR / SVD of the recompressions in FP64.
 #include "dev_linalg.hpp"
 #include "dev_panel.hpp"
 #include "factor_kernels.hpp"
@@ -294,9 +295,9 @@ __global__ void __launch_bounds__(256) k_gemm(const FTask* tasks, const GemmTile
 }
 
 // ---------------------------------------------------------------------------
-// POTRF (lower, left-looking): column j is updated by one thread per row with
-// the already factorised columns (row of L read from LDS, L[j,:] broadcast),
-// then scaled.  Two barriers per column.  LDS holds the block when n <= 128.
+// POTRF (lower).  Leaves of up to kLdsDense rows are factorised in LDS in FP64
+// (potrf_lds), larger ones and the HODLR node blocks in global memory in the
+// type they have (potrf_body).
 // ---------------------------------------------------------------------------
 constexpr int kLdsDense = 128;
 
@@ -307,9 +308,10 @@ constexpr int kTrsmCols = 64;  // independent rows / columns of a TRSM tile: 16 
 // 2,048 x 65 at 535 us, with 255 CUs idle
 constexpr int kElemsPerTile = 2048;
 
-// Right-looking blocked Cholesky: each 16-column panel is factorised
-// left-looking (short dots over the panel only), then the trailing lower
-// triangle gets the panel's rank-16 update with all threads.
+// Right-looking blocked Cholesky in global memory: each 16-column panel is
+// factorised left-looking (one thread per row, short dots over the panel only, two
+// barriers per column), then the trailing lower triangle gets the panel's rank-16
+// update with all threads.
 template <typename T>
 __device__ void potrf_body(T* L, int ld, int n, int* info) {
   for (int jb = 0; jb < n; jb += kNb) {
@@ -1732,7 +1734,7 @@ __device__ void qr_global(gptr<double> Va, int m, gptr<double> Vb, int n, int K,
 // Widest sum in this form.  Squaring the panels' condition costs accuracy that
 // wider sums, which come with tight cuts, do not have: with 33 to 40 columns and
 // eps = 1e-7 the result was 3.5e-7 off instead of 1e-7, two ranks short (at 1e-8
-// 19 to 36 times the best error, against 5 to 7 times through Householder QR;
+// 18 to 36 times the best error, against 5 to 7 times through Householder QR;
 // 256 sums of 33 columns and 100 rows take 620 us that way, 570 in this form).
 constexpr int kGramMaxK = kColsMax;
 constexpr double kGramTol = 1e-13;
@@ -2246,8 +2248,10 @@ __global__ void __launch_bounds__(kBlock) k_rkrk(const FTask* tasks, double* wsb
 
 // ---------------------------------------------------------------------------
 // ACAFULL: acaFull (compression.cpp:270-355) on a dense temp (modified)
-constexpr int kAcaLds = 16384;  // entries of the LDS copy (a 128 x 128 leaf product)
 // ---------------------------------------------------------------------------
+// entries of the LDS copy: blocks of more than 128 rows or columns (up to that
+// they are kept in registers) with at most this many entries
+constexpr int kAcaLds = 16384;
 // acaFull's stopping estimate after term nu (the reference sums l < nu - 1):
 // est += 2 sum_l (a_nu . a_l)(b_nu . b_l) + |a_nu|^2 |b_nu|^2; true when the new
 // term is below eps of it.  Each wavefront takes the terms l = w, w + 4, ...

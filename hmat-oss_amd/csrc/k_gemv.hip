@@ -684,6 +684,15 @@ void launch_cg_p(double* p, const double* z, const double* rz_new, const double*
 }
 template void launch_convert<float, double>(const float*, double*, size_t, hipStream_t);
 
+// One right-hand side takes the vector kernels, two and more the matrix cores,
+// whose tiles are 16 wide: a whole product of 1 / 2 / 4 / 8 / 16 right-hand sides
+// measured 97 / 258 / 262 / 273 / 288 us (N = 50,021, FP64), 27 / 93 / 94 / 96 / 98
+// (N = 10,007, leaves of 100 rows), 54 / 190 / 192 / 197 / 204 (N = 30,011, FP32,
+// non-symmetric) and 92 / 244 / 248 / 255 / 244 us (N = 8,000, complex).  Below
+// the line a tile is mostly zeros: two right-hand sides cost more than two
+// products of one each, three about as much as three; with a vector form for
+// several right-hand sides at once (eight at a time, leaves in LDS) two took 326,
+// 158, 275 and 811 us.
 template <typename T>
 void launch_gemv_zpass(const int* ranks, const T* arena, const ZItem* items, int nlong, int count,
                        const T* x, int ldx, int nrhs, double* zpart, double* z, hipStream_t s) {
