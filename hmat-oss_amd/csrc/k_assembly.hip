@@ -71,6 +71,12 @@ __device__ int pivoted_rows(int gr, int gc, double tol, double* W, int ldw) {
   }
   __syncthreads();
   n2 += dpp_swap<0xB1>(n2);
+  if (!(n2 <= 1.79e308)) {
+    // a column with infinities or NaN carries nothing, the others stay
+    n2 = 0.0;
+#pragma unroll
+    for (int r = 0; r < kR; ++r) g[r] = 0.0;
+  }
   double stop = 0.0;
   int s = 0;
   for (; s < gc; ++s) {
@@ -201,7 +207,8 @@ __global__ void __launch_bounds__(kBlock, 2) k_svd_compress(const LeafDesc* desc
     }
     if (row < gr)
       for (int c = h * half; c < (h ? gc : half); ++c) {
-        const double v = get(row, c);
+        double v = get(row, c);
+        v = fabs(v) <= 1.79e308 ? v : 0.0;  // (the column was left out)
 #pragma unroll
         for (int b = 0; b < kC; ++b) acc[b] += v * wj[b][c];
       }

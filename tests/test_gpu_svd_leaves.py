@@ -43,3 +43,46 @@ def test_svd_leaves(n, leaf, eps, kind, length):
     print(f"svd leaves n={n}: {seen} blocks", flush=True)
     assert seen > 0
     h.close()
+
+
+@pytest.mark.parametrize("bad", [np.nan, np.inf])
+def test_svd_leaves_non_finite(bad):
+    """One entry of one block is infinite or NaN (host functions): its column (its row
+    in a block with more columns than rows) is left out, the rest of the block and
+    every other block stay."""
+    import ctypes as C
+    n, eps = 197, 1e-6
+    rng = np.random.default_rng(3)
+    pts = np.column_stack([rng.random(n), rng.random(n), 12.0 * rng.random(n)])
+    tree = hmat_amd.ClusterTree(pts, 50)
+    P = pts[tree.indices]
+    K = np.exp(-np.linalg.norm(P[:, None] - P[None], axis=2) / 2.0)
+    h = hmat_amd.HMatrix(tree, lower_symmetric=False, lowrank_eps=eps)
+    where = [(r0 + 5, c0 + 7) for m, k, r0, c0, kd in h.leaf_shapes() if kd == 1][:2]
+    for at in where:
+        K[at] = bad
+    pos = np.argsort(tree.indices)
+
+    @hmat_amd.INTERACTION_FUNC
+    def entry(ctx, i, j, out):
+        C.cast(out, C.POINTER(C.c_double))[0] = K[pos[i], pos[j]]
+    h.assemble_functions(simple=entry, eps=eps)
+    hit = 0
+    for m, k, r0, c0, kd, rank, a, b in h.leaves():
+        if kd == 0:
+            continue
+        G = K[r0:r0 + m, c0:c0 + k].copy()
+        if not np.isfinite(G).all():
+            hit += 1
+            if m >= k:
+                G[:, ~np.isfinite(G).all(axis=0)] = 0.0
+            else:
+                G[~np.isfinite(G).all(axis=1), :] = 0.0
+        U, s, Vt = np.linalg.svd(G)
+        want = int((s > eps * s[0]).sum())
+        T = (U[:, :want] * s[:want]) @ Vt[:want]
+        gap = 1.0 + s[want - 1] / (s[want - 1] - s[want])
+        assert rank == want
+        assert np.linalg.norm(a @ b.T - T) <= 1e3 * 2.0 ** -53 * s[0] * gap
+    assert hit == 2
+    h.close()
