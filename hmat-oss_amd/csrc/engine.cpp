@@ -451,13 +451,15 @@ void Matrix::assemble_pass(const KernelSpec& k, const CompressionSpec& comp) {
   const int partial = comp.method == 2;
   DevBuf ws, dt;
   const int nleaf = (int)bt->leaves.size();
+  int shown = 0;  // (blocks that run again are counted back: the reports only rise)
   while (!acat.empty()) {
     sort_aca_by_size(acat, s64.hdesc);
     bool again = false;
     size_t i = 0;
     while (i < acat.size()) {
       HMX_CHECK(hipStreamSynchronize(stream));
-      report_assembly(nleaf - (int)(acat.size() - i), nleaf);
+      shown = std::max(shown, nleaf - (int)(acat.size() - i));
+      report_assembly(shown, nleaf);
       std::vector<AcaTask> batch;
       int64_t used = 0;
       while (i < acat.size()) {
